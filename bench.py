@@ -67,7 +67,7 @@ def parse():
 
 
 # kernels whose launch time the bench reads back from the library's event timing
-TIMED_KERNELS = ["k_pix2tri", "k_pix2tri_tier2", "k_pix2tri_tier3", "k_pack_tree",
+TIMED_KERNELS = ["k_pix2tri", "k_pack_tree",
                  "k_build_init", "k_centroid_aabb", "k_morton_hist", "k_hist_all", "k_onesweep",
                  "k_sort_finish", "k_sort_groups", "k_topology",
                  "k_refit_treelet", "k_refit_top", "k_fill_u32"]
@@ -1142,14 +1142,9 @@ def main():
         # child boxes (48 B); per tested leaf the triangle's indices (12 B) and
         # vertices (36 B)
         cast_bytes = num_pix * (24 + 8) + 60 * cast_counts[0] + 48 * cast_counts[1]
-        complete = cast_counts[2] <= stack  # every ray finished in k_pix2tri
         k_ms = k1["avg_ms"]
         name = "k_pix2tri"
-        if not complete:
-            k_ms = sum(kernels[k]["avg_ms"] * kernels[k]["launches_per_step"]
-                       for k in ("k_pix2tri", "k_pix2tri_tier2", "k_pix2tri_tier3") if k in kernels)
-            name = "k_pix2tri + restart tiers"
-        cc = read_counters("cast:k_pix2tri") if complete else None
+        cc = read_counters("cast:k_pix2tri")
         roof = {
             "bound": "hbm",
             "kernel": name,

@@ -23,7 +23,6 @@ namespace dmsh {
 namespace bat {
 
 constexpr uint32_t kMeshKeyShift = 30;
-constexpr uint32_t kXcds = 8;
 
 // The segment holding element x (x < off[M]): the last m with off[m] <= x,
 // which skips empty segments (repeated offsets).
@@ -659,7 +658,8 @@ static __global__ __launch_bounds__(256) void k_batch_pack_leaf(BatchTrees b, ui
                 err);
 }
 
-struct BatchCast {
+// The images of a batch: mesh m's is its pixels, widths[m] wide.
+struct BatchSrc {
   uint32_t M;
   const uint32_t* mesh2tri;
   const uint32_t* node_off;
@@ -671,135 +671,31 @@ struct BatchCast {
   const rc::LeafTri* leaf;
   const float* aabb;
   const float* transforms;  // [M][16] ndc2world, column-major
-  uint32_t* pix2tri;
-  float* pix2t;
-  uint32_t* counts;  // [0] tier-2 queue, [1] tier-3 queue, [2] non-finite box flag,
-                     // [3] offsets rejected, [16 + 16 x] tile counter of XCD x
-  uint32_t* list2;
-  uint32_t* list3;
-  uint2* deep_stack;
-  uint32_t* err;
+  const uint32_t* counts;
+  __device__ __forceinline__ uint32_t num_tiles() const { return counts[3] ? 0u : tile_off[M]; }
+  __device__ __forceinline__ bool load(uint32_t tile, uint32_t lane, rc::PixelJob& j) const {
+    const uint32_t m = rc::wave_segment(tile_off, M, tile);
+    const uint32_t p0 = pix_off[m], tb = mesh2tri[m];
+    j.pk = rc::Packed{inner + inner_off[m], leaf + tb, aabb + (size_t)node_off[m] * 6,
+                      mesh2tri[m + 1] - tb};
+    j.T = transforms + (size_t)m * 16;
+    j.w = widths[m];
+    j.h = (pix_off[m + 1] - p0) / j.w;
+    const uint32_t tiles_x = ceil_div_u32(j.w, 8u), lt = tile - tile_off[m];
+    j.iw = (lt % tiles_x) * 8u + (lane & 7u);
+    j.ih = (lt / tiles_x) * 8u + (lane >> 3);
+    j.out = p0 + j.ih * j.w + j.iw;
+    j.regular = counts[2] == 0u;
+    return j.iw < j.w && j.ih < j.h;
+  }
 };
 
-__device__ __forceinline__ rc::Packed packed_of(const BatchCast& a, uint32_t m) {
-  const uint32_t tb = a.mesh2tri[m];
-  return rc::Packed{a.inner + a.inner_off[m], a.leaf + tb, a.aabb + (size_t)a.node_off[m] * 6,
-                    a.mesh2tri[m + 1] - tb};
-}
-
-__device__ __forceinline__ void batch_write(const BatchCast& a, uint32_t gp, const rc::Hit& h) {
-  a.pix2tri[gp] = h.has ? h.tri : DMSH_U32MAX;
-  if (a.pix2t) a.pix2t[gp] = h.has ? h.t : 0.f;
-}
-
-// Next tile for the calling wave (the same value in every lane), or
-// num_tiles when none is left.
-__device__ __forceinline__ uint32_t next_tile(const BatchCast& a, uint32_t num_tiles,
-                                              uint32_t& xcd) {
-  const uint32_t per = (num_tiles + kXcds - 1) / kXcds;
-  for (uint32_t tries = 0; tries < kXcds; ++tries) {
-    const uint32_t lo = xcd * per;
-    const uint32_t hi = (lo + per < num_tiles) ? lo + per : num_tiles;
-    uint32_t t = 0;
-    if ((threadIdx.x & 63u) == 0) t = atomicAdd(a.counts + 16 + 16 * xcd, 1u);
-    t = __builtin_amdgcn_readfirstlane(t) + lo;
-    if (t < hi) return t;
-    xcd = (xcd + 1) % kXcds;
-  }
-  return num_tiles;
-}
-
-// Tier 1 over all meshes: persistent workgroups of W waves, each wave taking
-// its own tiles (no barrier between them; W is the workgroup size the
-// autotuner picks).
 template <int S, int W>
-__global__ __launch_bounds__(64 * W) void k_batch_pix2tri(BatchCast a) {
-  __shared__ uint2 s_stack_all[W][S][64];
-  uint2 (*s_stack)[64] = s_stack_all[threadIdx.x >> 6];
-  const uint32_t lane = threadIdx.x & 63u;
-  if (a.counts[3]) return;  // offsets rejected
-  const uint32_t num_tiles = a.tile_off[a.M];
-  const bool boxes_finite = a.counts[2] == 0u;
-  uint32_t xcd = blockIdx.x % kXcds;
-  for (;;) {
-    const uint32_t tile = next_tile(a, num_tiles, xcd);
-    if (tile >= num_tiles) break;
-    const uint32_t m = find_segment(a.tile_off, a.M, tile);
-    const uint32_t w = a.widths[m], p0 = a.pix_off[m], h = (a.pix_off[m + 1] - p0) / w;
-    const uint32_t tiles_x = ceil_div_u32(w, 8u), lt = tile - a.tile_off[m];
-    const uint32_t iw = (lt % tiles_x) * 8u + (lane & 7u), ih = (lt / tiles_x) * 8u + (lane >> 3);
-    if (iw < w && ih < h) {
-      float T[16];
-      rc::load_transform(a.transforms + (size_t)m * 16, T);
-      float org[3], dir[3];
-      ray_for_pixel(iw, ih, w, h, T, org, dir);
-      rc::LdsStack<S> stk{&s_stack[0][lane], 64};
-      rc::Hit hit;
-      const int st = rc::trace(packed_of(a, m), org, dir, stk, hit, boxes_finite);
-      const uint32_t gp = p0 + ih * w + iw;
-      if (st == rc::kTraceOverflow) a.list2[atomicAdd(a.counts + 0, 1u)] = gp;
-      else batch_write(a, gp, hit);
-    }
-  }
-}
-
-__device__ __forceinline__ void batch_pixel(const BatchCast& a, uint32_t gp, uint32_t& m,
-                                            uint32_t& iw, uint32_t& ih, uint32_t& w,
-                                            uint32_t& h) {
-  m = find_segment(a.pix_off, a.M, gp);
-  w = a.widths[m];
-  const uint32_t p0 = a.pix_off[m];
-  h = (a.pix_off[m + 1] - p0) / w;
-  ih = (gp - p0) / w;
-  iw = gp - p0 - ih * w;
-}
-
-static __global__ __launch_bounds__(64) void k_batch_pix2tri_tier2(BatchCast a,
-                                                                   uint32_t total_pix) {
-  __shared__ uint2 s_stack[rc::kTier2Frames][64];
-  if (a.counts[3]) return;
-  uint32_t count = a.counts[0];
-  if (count > total_pix) count = total_pix;
-  const bool boxes_finite = a.counts[2] == 0u;
-  rc::LdsStack<rc::kTier2Frames> stk{&s_stack[0][threadIdx.x], 64};
-  for (uint32_t e = blockIdx.x * 64u + threadIdx.x; e < count; e += gridDim.x * 64u) {
-    const uint32_t gp = a.list2[e];
-    uint32_t m, iw, ih, w, h;
-    batch_pixel(a, gp, m, iw, ih, w, h);
-    float T[16], org[3], dir[3];
-    rc::load_transform(a.transforms + (size_t)m * 16, T);
-    ray_for_pixel(iw, ih, w, h, T, org, dir);
-    rc::Hit hit;
-    const int st = rc::trace(packed_of(a, m), org, dir, stk, hit, boxes_finite);
-    if (st == rc::kTraceOverflow) a.list3[atomicAdd(a.counts + 1, 1u)] = gp;
-    else batch_write(a, gp, hit);
-  }
-}
-
-static __global__ __launch_bounds__(64) void k_batch_pix2tri_tier3(BatchCast a,
-                                                                   uint32_t total_pix) {
-  const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t nthr = gridDim.x * blockDim.x;
-  if (a.counts[3]) return;
-  uint32_t count = a.counts[1];
-  if (count > total_pix) count = total_pix;
-  const bool boxes_finite = a.counts[2] == 0u;
-  rc::GlobalStack stk{a.deep_stack + (size_t)gid * rc::kDeepFrames};
-  for (uint32_t e = gid; e < count; e += nthr) {
-    const uint32_t gp = a.list3[e];
-    uint32_t m, iw, ih, w, h;
-    batch_pixel(a, gp, m, iw, ih, w, h);
-    float T[16], org[3], dir[3];
-    rc::load_transform(a.transforms + (size_t)m * 16, T);
-    ray_for_pixel(iw, ih, w, h, T, org, dir);
-    rc::Hit hit;
-    const int st = rc::trace(packed_of(a, m), org, dir, stk, hit, boxes_finite);
-    if (st != rc::kTraceOk) {
-      raise_error(a.err, DMSH_DEVERR_STACK);
-      hit.has = false;
-    }
-    batch_write(a, gp, hit);
-  }
+__global__ __launch_bounds__(64 * W) void k_batch_pix2tri(BatchSrc src, rc::CastState st,
+                                                          uint32_t* __restrict__ pix2tri,
+                                                          float* __restrict__ pix2t) {
+  __shared__ uint64_t s_stack[W][S][64];
+  rc::cast_wave<S, W>(src, st, (rc::LdsFrame*)&s_stack[threadIdx.x >> 6][0][0], pix2tri, pix2t);
 }
 
 }  // namespace bat

@@ -10,10 +10,8 @@ using namespace dmsh;
 
 namespace {
 
-constexpr uint32_t kCastCounts = 256;  // see bat::BatchCast::counts
-
-std::atomic<int> g_batch_stack{20};      // LDS frames per lane of the batched tier 1
-std::atomic<int> g_batch_wgs_per_cu{16};  // persistent ray-cast waves per CU
+std::atomic<int> g_batch_stack{12};       // LDS frames per lane of the ray-cast
+std::atomic<int> g_batch_wgs_per_cu{32};  // persistent ray-cast waves per CU
 std::atomic<int> g_batch_sort_items{16};  // elements per thread of the digit passes
 std::atomic<int> g_batch_sort_seg{1};     // segmented passes + finish (up to kSegMaxMeshes)
 std::atomic<int> g_batch_cast_waves{1};   // waves per ray-cast workgroup
@@ -102,45 +100,70 @@ inline bool carve_batch_build(Arena& a, uint32_t M, uint32_t n, BatchBuildLayout
 }
 
 struct BatchCastLayout {
-  uint32_t* counts;  // [kCastCounts]
+  uint32_t* counts;  // [rc::kCastCounts]
   uint32_t* inner_off;
   uint32_t* tile_off;
-  uint32_t* list2;
-  uint32_t* list3;
-  uint2* deep;
+  uint64_t* spill;
   rc::InnerNode* inner;
   rc::LeafTri* leaf;
 };
 
+// Spill area of a launch over `images` images with num_pix pixels in all
+// (whole workgroups of up to 4 waves).
+inline uint64_t* take_spill(Arena& a, uint64_t num_pix, uint64_t images) {
+  return a.take<uint64_t>(((size_t)rc::cast_waves(rc::max_tiles(num_pix, images)) + 3) *
+                       rc::kSpillPerWave);
+}
+
 inline bool carve_batch_cast(Arena& a, uint32_t M, uint32_t n, uint32_t num_pix,
                              BatchCastLayout& L) {
-  L.counts = a.take<uint32_t>(kCastCounts);
+  L.counts = a.take<uint32_t>(rc::kCastCounts);
   L.inner_off = a.take<uint32_t>((size_t)M + 1);
   L.tile_off = a.take<uint32_t>((size_t)M + 1);
-  L.list2 = a.take<uint32_t>(num_pix ? num_pix : 1);
-  L.list3 = a.take<uint32_t>(num_pix ? num_pix : 1);
-  L.deep = a.take<uint2>((size_t)rc::kDeepSlots * rc::kDeepFrames);
+  L.spill = take_spill(a, num_pix, M);
   L.inner = a.take<rc::InnerNode>(n ? n : 1);
   L.leaf = a.take<rc::LeafTri>(n ? n : 1);
   return a.ok();
 }
 
-template <int S>
-void launch_batch_tier1(hipStream_t s, uint32_t waves, const bat::BatchCast& a) {
-  switch (g_batch_cast_waves.load()) {
-    case 2:
-      launch("k_batch_pix2tri", bat::k_batch_pix2tri<S, 2>, dim3(ceil_div(waves, 2)), dim3(128), 0,
-             s, a);
-      break;
-    case 4:
-      launch("k_batch_pix2tri", bat::k_batch_pix2tri<S, 4>, dim3(ceil_div(waves, 4)), dim3(256), 0,
-             s, a);
-      break;
-    default:
-      launch("k_batch_pix2tri", bat::k_batch_pix2tri<S, 1>, dim3(waves), dim3(64), 0, s, a);
-      break;
+// Launches Cast<S, W> for the tuned number of LDS frames S and waves per
+// workgroup W.
+template <template <int, int> class Cast, class Src>
+void launch_cast(hipStream_t s, uint32_t max_tiles, const Src& src, const rc::CastState& st,
+                 uint32_t* pix2tri, float* pix2t) {
+  auto go = [&](auto kernel, const char* label, int frames, uint32_t w) {
+    const uint32_t per_cu =
+        std::min((uint32_t)g_batch_wgs_per_cu.load(), rc::resident_waves(frames));
+    const uint32_t waves = std::min(rc::cast_waves(max_tiles), (uint32_t)device_cu_count() * per_cu);
+    launch(label, kernel, dim3(ceil_div(waves, w)), dim3(64 * w), 0, s, src, st, pix2tri, pix2t);
+  };
+  auto with_waves = [&](auto frames) {
+    constexpr int S = decltype(frames)::value;
+    switch (g_batch_cast_waves.load()) {
+      case 2: go(Cast<S, 2>::kernel(), Cast<S, 2>::label(), S, 2u); break;
+      case 4: go(Cast<S, 4>::kernel(), Cast<S, 4>::label(), S, 4u); break;
+      default: go(Cast<S, 1>::kernel(), Cast<S, 1>::label(), S, 1u); break;
+    }
+  };
+  switch (g_batch_stack.load()) {
+    case 16: with_waves(std::integral_constant<int, 16>()); break;
+    case 20: with_waves(std::integral_constant<int, 20>()); break;
+    case 24: with_waves(std::integral_constant<int, 24>()); break;
+    case 32: with_waves(std::integral_constant<int, 32>()); break;
+        default: with_waves(std::integral_constant<int, 12>()); break;
   }
 }
+
+template <int S, int W>
+struct BatchCastKernel {
+  static auto kernel() { return &bat::k_batch_pix2tri<S, W>; }
+  static const char* label() { return "k_batch_pix2tri"; }
+};
+template <int S, int W>
+struct ReqCastKernel {
+  static auto kernel() { return &srv::k_req_pix2tri<S, W>; }
+  static const char* label() { return "k_req_pix2tri"; }
+};
 
 // Offsets of a batch of built trees (as for the batched cast, without images).
 __global__ __launch_bounds__(1024) void k_pack_offsets(uint32_t M, uint32_t total_tri,
@@ -170,24 +193,15 @@ struct ReqLayout {
   uint32_t* counts;
   uint32_t* tile_off;
   uint32_t* pix_off;
-  uint32_t* list2;
-  uint32_t* list3;
-  uint2* deep;
+  uint64_t* spill;
 };
 
 inline bool carve_req(Arena& a, uint32_t R, uint32_t num_pix, ReqLayout& L) {
-  L.counts = a.take<uint32_t>(kCastCounts);
+  L.counts = a.take<uint32_t>(rc::kCastCounts);
   L.tile_off = a.take<uint32_t>((size_t)R + 1);
   L.pix_off = a.take<uint32_t>((size_t)R + 1);
-  L.list2 = a.take<uint32_t>(num_pix ? num_pix : 1);
-  L.list3 = a.take<uint32_t>(num_pix ? num_pix : 1);
-  L.deep = a.take<uint2>((size_t)rc::kDeepSlots * rc::kDeepFrames);
+  L.spill = take_spill(a, num_pix, R);
   return a.ok();
-}
-
-template <int S>
-void launch_req_tier1(hipStream_t s, uint32_t grid, const srv::ReqCast& a) {
-  launch("k_req_pix2tri", srv::k_req_pix2tri<S>, dim3(grid), dim3(64), 0, s, a);
 }
 
 int device_cus() {
@@ -205,7 +219,8 @@ extern "C" {
 int dmsh_batch_set_tuning(const char* key, int value) {
   if (!key) return DMSH_ERR_INVALID;
   if (std::strcmp(key, "batch.stack") == 0) {
-    if (value != 16 && value != 20 && value != 24 && value != 32) return DMSH_ERR_INVALID;
+    if (value != 12 && value != 16 && value != 20 && value != 24 && value != 32)
+      return DMSH_ERR_INVALID;
     g_batch_stack.store(value);
     return DMSH_OK;
   }
@@ -431,7 +446,7 @@ int dmsh_batch_pix2tri(void* stream, uint32_t num_mesh, uint32_t total_tri, uint
   if (!err) return DMSH_ERR_HIP;
   hipStream_t s = as_stream(stream);
   const uint32_t M = num_mesh, n = total_tri;
-  int rc = sortk::launch_fill(s, L.counts, kCastCounts, 0u);
+  int rc = sortk::launch_fill(s, L.counts, rc::kCastCounts, 0u);
   if (rc != DMSH_OK) return rc;
   launch("k_batch_cast_offsets", bat::k_batch_cast_offsets, dim3(1), dim3(1024), 0, s, M, n,
          total_vtx, total_pix, mesh2tri, mesh2vtx, mesh2node, mesh2pix, mesh2width, L.inner_off,
@@ -447,38 +462,11 @@ int dmsh_batch_pix2tri(void* stream, uint32_t num_mesh, uint32_t total_tri, uint
            L.leaf, err);
     if ((rc = launch_status()) != DMSH_OK) return rc;
   }
-  bat::BatchCast a;
-  a.M = M;
-  a.mesh2tri = mesh2tri;
-  a.node_off = mesh2node;
-  a.inner_off = L.inner_off;
-  a.tile_off = L.tile_off;
-  a.pix_off = mesh2pix;
-  a.widths = mesh2width;
-  a.inner = L.inner;
-  a.leaf = L.leaf;
-  a.aabb = bvhnode2aabb;
-  a.transforms = transforms_ndc2world;
-  a.pix2tri = pix2tri;
-  a.pix2t = pix2t;
-  a.counts = L.counts;
-  a.list2 = L.list2;
-  a.list3 = L.list3;
-  a.deep_stack = L.deep;
-  a.err = err;
-  const uint32_t grid = (uint32_t)device_cus() * (uint32_t)g_batch_wgs_per_cu.load();
-  switch (g_batch_stack.load()) {
-    case 16: launch_batch_tier1<16>(s, grid, a); break;
-    case 20: launch_batch_tier1<20>(s, grid, a); break;
-    case 32: launch_batch_tier1<32>(s, grid, a); break;
-    default: launch_batch_tier1<24>(s, grid, a); break;
-  }
-  if ((rc = launch_status()) != DMSH_OK) return rc;
-  launch("k_batch_pix2tri_tier2", bat::k_batch_pix2tri_tier2, dim3(rc::kTier2Blocks), dim3(64), 0,
-         s, a, total_pix);
-  if ((rc = launch_status()) != DMSH_OK) return rc;
-  launch("k_batch_pix2tri_tier3", bat::k_batch_pix2tri_tier3, dim3(rc::kDeepSlots / 64), dim3(64),
-         0, s, a, total_pix);
+  const bat::BatchSrc src{M,         mesh2tri,   mesh2node, L.inner_off, L.tile_off,
+                          mesh2pix,  mesh2width, L.inner,   L.leaf,      bvhnode2aabb,
+                          transforms_ndc2world,  L.counts};
+  launch_cast<BatchCastKernel>(s, rc::max_tiles(total_pix, M), src,
+                               rc::CastState{L.counts, L.spill, err}, pix2tri, pix2t);
   return launch_status();
 }
 
@@ -546,27 +534,15 @@ int dmsh_cast_requests(void* stream, uint32_t num_req, const dmsh_cast_request* 
   uint32_t* err = device_error_word();
   if (!err) return DMSH_ERR_HIP;
   hipStream_t s = as_stream(stream);
-  int rc = sortk::launch_fill(s, L.counts, kCastCounts, 0u);
+  int rc = sortk::launch_fill(s, L.counts, rc::kCastCounts, 0u);
   if (rc != DMSH_OK) return rc;
   const srv::Request* req = reinterpret_cast<const srv::Request*>(requests);
   launch("k_req_offsets", srv::k_req_offsets, dim3(1), dim3(1024), 0, s, num_req, total_pix, req,
          L.tile_off, L.pix_off, L.counts + 3, err);
   if ((rc = launch_status()) != DMSH_OK) return rc;
-  srv::ReqCast a{num_req, req, L.tile_off, L.pix_off, pix2tri, pix2t, L.counts,
-                 L.list2, L.list3, L.deep, err};
-  const uint32_t grid = (uint32_t)device_cus() * (uint32_t)g_batch_wgs_per_cu.load();
-  switch (g_batch_stack.load()) {
-    case 16: launch_req_tier1<16>(s, grid, a); break;
-    case 20: launch_req_tier1<20>(s, grid, a); break;
-    case 32: launch_req_tier1<32>(s, grid, a); break;
-    default: launch_req_tier1<24>(s, grid, a); break;
-  }
-  if ((rc = launch_status()) != DMSH_OK) return rc;
-  launch("k_req_pix2tri_tier2", srv::k_req_pix2tri_tier2, dim3(rc::kTier2Blocks), dim3(64), 0, s,
-         a, total_pix);
-  if ((rc = launch_status()) != DMSH_OK) return rc;
-  launch("k_req_pix2tri_tier3", srv::k_req_pix2tri_tier3, dim3(rc::kDeepSlots / 64), dim3(64), 0,
-         s, a, total_pix);
+  const srv::ReqSrc src{num_req, req, L.tile_off, L.counts};
+  launch_cast<ReqCastKernel>(s, rc::max_tiles(total_pix, num_req), src,
+                             rc::CastState{L.counts, L.spill, err}, pix2tri, pix2t);
   return launch_status();
 }
 

@@ -12,58 +12,60 @@ using namespace dmsh;
 
 namespace {
 
-// Defaults from a sweep on the 2^21-triangle / 2048^2-ray workload (MI355X),
-// whose deepest ray needs 24 frames: 16 frames x 1 wave 3.36 ms (some rays
-// restart in tier 2), 24 x 1 3.37 ms (none do), 24 x 2 3.53 ms, 32 x 1
-// 3.98 ms, 32 x 4 5.12 ms.
-std::atomic<int> g_cast_stack{20};  // LDS frames per lane (tier 1)
-std::atomic<int> g_cast_waves{1};   // waves per workgroup (tier 1)
+// LDS frames a lane: 12 keep 26 waves on a CU.  2^21 triangles at 2048^2 take
+// 2.07 ms with 12, 2.17 with 8 (more frames in the spill area), 2.26 with 16,
+// 2.52 with 20 (16 waves).
+std::atomic<int> g_cast_stack{12};
+std::atomic<int> g_cast_waves{1};   // waves per workgroup
 
 struct CastLayout {
   uint32_t* counts;
-  uint32_t* list2;
-  uint32_t* list3;
-  uint2* deep;
+  uint64_t* spill;
   rc::InnerNode* inner;
   rc::LeafTri* leaf;
 };
 
-inline bool carve_cast(Arena& a, uint32_t num_tri, uint32_t num_pix, CastLayout& L) {
-  L.counts = a.take<uint32_t>(64);
-  L.list2 = a.take<uint32_t>(num_pix ? num_pix : 1);
-  L.list3 = a.take<uint32_t>(num_pix ? num_pix : 1);
-  L.deep = a.take<uint2>((size_t)rc::kDeepSlots * rc::kDeepFrames);
+inline uint32_t image_tiles(uint32_t img_w, uint32_t img_h) {
+  return ceil_div(img_w, 8) * ceil_div(img_h, 8);
+}
+
+inline bool carve_cast(Arena& a, uint32_t num_tri, uint32_t img_w, uint32_t img_h, CastLayout& L) {
+  L.counts = a.take<uint32_t>(rc::kCastCounts);
+  // whole workgroups of up to 4 waves
+  L.spill = a.take<uint64_t>(((size_t)rc::cast_waves(image_tiles(img_w, img_h)) + 3) *
+                          rc::kSpillPerWave);
   L.inner = a.take<rc::InnerNode>(num_tri > 1 ? num_tri - 1 : 1);
   L.leaf = a.take<rc::LeafTri>(num_tri ? num_tri : 1);
   return a.ok();
 }
 
-template <int S, int WAVES>
-void launch_tier1(hipStream_t s, const rc::Packed& pk, const float* T, const rc::CastArgs& a) {
-  launch("k_pix2tri", (rc::k_pix2tri<S, WAVES>), dim3(ceil_div(a.num_tiles, WAVES)),
-                     dim3(64 * WAVES), 0, s, pk, T, a);
+template <int S, int W>
+void launch_pix2tri(hipStream_t s, const rc::ImageSrc& src, const rc::CastState& st,
+                    uint32_t* pix2tri, float* pix2t) {
+  const uint32_t waves = std::min(rc::cast_waves(src.tiles),
+                                  (uint32_t)device_cu_count() * rc::resident_waves(S));
+  launch("k_pix2tri", (rc::k_pix2tri<S, W>), dim3(ceil_div(waves, W)), dim3(64 * W), 0, s, src, st, pix2tri, pix2t);
 }
 
 template <int S>
-bool launch_tier1_waves(int waves, hipStream_t s, const rc::Packed& pk, const float* T,
-                        const rc::CastArgs& a) {
+void launch_pix2tri_waves(int waves, hipStream_t s, const rc::ImageSrc& src,
+                          const rc::CastState& st, uint32_t* pix2tri, float* pix2t) {
   switch (waves) {
-    case 1: launch_tier1<S, 1>(s, pk, T, a); return true;
-    case 2: launch_tier1<S, 2>(s, pk, T, a); return true;
-    case 4: launch_tier1<S, 4>(s, pk, T, a); return true;
-    default: return false;
+    case 2: launch_pix2tri<S, 2>(s, src, st, pix2tri, pix2t); break;
+    case 4: launch_pix2tri<S, 4>(s, src, st, pix2tri, pix2t); break;
+    default: launch_pix2tri<S, 1>(s, src, st, pix2tri, pix2t); break;
   }
 }
 
-bool launch_tier1_any(int stack, int waves, hipStream_t s, const rc::Packed& pk, const float* T,
-                      const rc::CastArgs& a) {
+void launch_pix2tri_any(int stack, int waves, hipStream_t s, const rc::ImageSrc& src,
+                        const rc::CastState& st, uint32_t* pix2tri, float* pix2t) {
   switch (stack) {
-    case 12: return launch_tier1_waves<12>(waves, s, pk, T, a);
-    case 16: return launch_tier1_waves<16>(waves, s, pk, T, a);
-    case 20: return launch_tier1_waves<20>(waves, s, pk, T, a);
-    case 24: return launch_tier1_waves<24>(waves, s, pk, T, a);
-    case 32: return launch_tier1_waves<32>(waves, s, pk, T, a);
-    default: return false;
+    case 8: launch_pix2tri_waves<8>(waves, s, src, st, pix2tri, pix2t); break;
+    case 16: launch_pix2tri_waves<16>(waves, s, src, st, pix2tri, pix2t); break;
+    case 20: launch_pix2tri_waves<20>(waves, s, src, st, pix2tri, pix2t); break;
+    case 24: launch_pix2tri_waves<24>(waves, s, src, st, pix2tri, pix2t); break;
+    case 32: launch_pix2tri_waves<32>(waves, s, src, st, pix2tri, pix2t); break;
+    default: launch_pix2tri_waves<12>(waves, s, src, st, pix2tri, pix2t); break;
   }
 }
 
@@ -74,7 +76,7 @@ extern "C" {
 int dmsh_set_tuning(const char* key, int value) {
   if (!key) return DMSH_ERR_INVALID;
   if (std::strcmp(key, "pix2tri.stack") == 0) {
-    if (value != 12 && value != 16 && value != 20 && value != 24 && value != 32)
+    if (value != 8 && value != 12 && value != 16 && value != 20 && value != 24 && value != 32)
       return DMSH_ERR_INVALID;
     g_cast_stack.store(value);
     return DMSH_OK;
@@ -97,7 +99,7 @@ int dmsh_get_tuning(const char* key) {
 size_t dmsh_pix2tri_workspace_bytes(uint32_t num_tri, uint32_t img_w, uint32_t img_h) {
   Arena a{nullptr, 0, 0};
   CastLayout L;
-  carve_cast(a, num_tri, img_w * img_h, L);
+  carve_cast(a, num_tri, img_w, img_h, L);
   return a.off + 256;
 }
 
@@ -114,11 +116,11 @@ int dmsh_pix2tri(void* stream, uint32_t* pix2tri, float* pix2t, uint32_t num_tri
     return DMSH_ERR_WORKSPACE;
   Arena ar{static_cast<char*>(ws), ws_bytes, 0};
   CastLayout L;
-  if (!carve_cast(ar, num_tri, (uint32_t)num_pix, L)) return DMSH_ERR_WORKSPACE;
+  if (!carve_cast(ar, num_tri, img_w, img_h, L)) return DMSH_ERR_WORKSPACE;
   uint32_t* err = device_error_word();
   if (!err) return DMSH_ERR_HIP;
   hipStream_t s = as_stream(stream);
-  int st = sortk::launch_fill(s, L.counts, 3, 0u);
+  int st = sortk::launch_fill(s, L.counts, rc::kCastCounts, 0u);
   if (st != DMSH_OK) return st;
   if (num_tri > 0) {
     launch("k_pack_tree", rc::k_pack_tree, dim3(ceil_div(2 * (uint64_t)num_tri - 1, 256)),
@@ -126,27 +128,15 @@ int dmsh_pix2tri(void* stream, uint32_t* pix2tri, float* pix2t, uint32_t num_tri
            num_vtx, L.counts + 2, err);
     if ((st = launch_status()) != DMSH_OK) return st;
   }
-  rc::Packed pk{L.inner, L.leaf, bvhnode2aabb, num_tri};
-  rc::CastArgs a;
-  a.pix2tri = pix2tri;
-  a.pix2t = pix2t;
-  a.img_w = img_w;
-  a.img_h = img_h;
-  a.tiles_x = ceil_div(img_w, 8);
-  a.num_tiles = a.tiles_x * ceil_div(img_h, 8);
-  a.counts = L.counts;
-  a.list2 = L.list2;
-  a.list3 = L.list3;
-  a.deep_stack = L.deep;
-  a.err = err;
-  if (!launch_tier1_any(g_cast_stack.load(), g_cast_waves.load(), s, pk, transform_ndc2world, a))
-    return DMSH_ERR_INVALID;
-  if ((st = launch_status()) != DMSH_OK) return st;
-  launch("k_pix2tri_tier2", rc::k_pix2tri_tier2, dim3(rc::kTier2Blocks), dim3(64), 0, s, pk,
-                     transform_ndc2world, a);
-  if ((st = launch_status()) != DMSH_OK) return st;
-  launch("k_pix2tri_tier3", rc::k_pix2tri_tier3, dim3(rc::kDeepSlots / 64), dim3(64), 0, s, pk,
-                     transform_ndc2world, a);
+  const rc::ImageSrc src{{L.inner, L.leaf, bvhnode2aabb, num_tri},
+                         transform_ndc2world,
+                         img_w,
+                         img_h,
+                         ceil_div(img_w, 8),
+                         image_tiles(img_w, img_h),
+                         L.counts};
+  launch_pix2tri_any(g_cast_stack.load(), g_cast_waves.load(), s, src,
+                     rc::CastState{L.counts, L.spill, err}, pix2tri, pix2t);
   return launch_status();
 }
 

@@ -27,12 +27,13 @@
 // (the reference layout needs a row load, then dependent box / index / vertex
 // gathers).  The values are copies, so the arithmetic is unchanged.
 //
-// Stack tiers: the main kernel keeps S frames per lane in LDS
-// ([depth][thread], conflict-free for 64-bit accesses); a ray that needs more
-// is queued and restarted by a kernel with 64 LDS frames, and a ray that needs
-// more than that by one with a 4096-frame stack in global memory.  Pixels go
-// to waves in 8x8 tiles and tiles to XCDs in contiguous runs, so neighbouring
-// rays share BVH nodes in one L2.
+// Stack: a lane's first S frames sit in LDS ([frame][lane], conflict-free for
+// 64-bit accesses), the next kSpillFrames in its wave's spill area in the
+// workspace.  A lane that needs more is searched again alone, with the whole
+// spill area of its wave (kDeepFrames frames) as its stack; beyond that it
+// raises DMSH_DEVERR_STACK.  So one launch serves every ray, and S can be small
+// enough for 26 waves on a CU.  Pixels go to waves in 8x8 tiles; a fixed grid of
+// waves takes tiles until none is left (TileDeal).
 #pragma once
 
 #include "dmsh_common.hpp"
@@ -44,10 +45,11 @@ namespace rc {
 constexpr uint32_t kLeafBit = 0x40000000u;   // child ref: leaf slot
 constexpr uint32_t kIndexMask = 0x3FFFFFFFu;
 constexpr uint32_t kMaxTri = 0x3FFFFFFFu;    // child refs hold 30-bit indices
-constexpr int kTier2Frames = 64;
-constexpr uint32_t kDeepFrames = 4096;
-constexpr uint32_t kDeepSlots = 256;
-constexpr uint32_t kTier2Blocks = 512;
+constexpr int kSpillFrames = 64;                // spilled frames per lane
+constexpr uint32_t kDeepFrames = 64u * kSpillFrames;  // a lone lane's frames
+constexpr uint32_t kMaxCastWaves = 8192;        // 32 waves on each of 256 CUs
+constexpr uint32_t kXcds = 8;
+constexpr uint32_t kCastCounts = 32 + 32 * kXcds;  // words of CastState::counts
 
 enum : int { kTraceOk = 0, kTraceOverflow = 1, kTraceBadIndex = 2 };
 
@@ -101,7 +103,9 @@ __device__ __forceinline__ void store_inner(InnerNode* __restrict__ inner, uint3
   InnerNode nd;
   if (bad) {
     raise_error(err, DMSH_DEVERR_INDEX);
-    // an empty box on both sides: every ray misses this node
+    // an inverted box on both sides: every ray misses this node (in the
+    // general slab test, which the flag selects)
+    atomicOr(nonfinite, 1u);
     nd.a = make_float4(1.f, 1.f, 1.f, 0.f);
     nd.b = make_float4(0.f, 0.f, 1.f, 1.f);
     nd.c = make_float4(1.f, 0.f, 0.f, 0.f);
@@ -115,6 +119,8 @@ __device__ __forceinline__ void store_inner(InnerNode* __restrict__ inner, uint3
 #pragma unroll
     for (int k = 0; k < 6; ++k)
       fin = fin && fabsf(b0[k]) < __builtin_inff() && fabsf(b1[k]) < __builtin_inff();
+#pragma unroll
+    for (int k = 0; k < 3; ++k) fin = fin && b0[k] <= b0[k + 3] && b1[k] <= b1[k + 3];
     if (!fin) atomicOr(nonfinite, 1u);
   }
   inner[i] = nd;
@@ -123,9 +129,10 @@ __device__ __forceinline__ void store_inner(InnerNode* __restrict__ inner, uint3
 // 16-byte part `part` of the record store_inner writes for children (c0,
 // c1): parts 0..2 hold the children's bounds x0..x3 (box 0 bounds 0-3;
 // bounds 4, 5 of box 0 and 0, 1 of box 1; box 1 bounds 2-5), part 3 the
-// refs.  A record whose children do not fit the layout raises (part 0) and
-// is the one every ray misses; a part with a bound that is not finite sets
-// *nonfinite.  Writing the four parts from consecutive threads makes a
+// refs.  A record whose children do not fit the layout raises (part 0), is
+// the one every ray misses and sets *nonfinite, as a part with a bound that is
+// not finite does (the boxes here are the refit's own: with finite bounds
+// lo <= hi).  Writing the four parts from consecutive threads makes a
 // wave's store one contiguous kilobyte.
 __device__ __forceinline__ uint4 inner_part_bits(uint32_t part, uint32_t c0, uint32_t c1,
                                                  float x0, float x1, float x2, float x3,
@@ -136,7 +143,10 @@ __device__ __forceinline__ uint4 inner_part_bits(uint32_t part, uint32_t c0, uin
   const uint32_t r0 = child_ref(c0, num_leaf, bad);
   const uint32_t r1 = child_ref(c1, num_leaf, bad);
   if (bad) {
-    if (part == 0u) raise_error(err, DMSH_DEVERR_INDEX);
+    if (part == 0u) {
+      raise_error(err, DMSH_DEVERR_INDEX);
+      atomicOr(nonfinite, 1u);
+    }
     if (part == 3u) return make_uint4(kLeafBit, kLeafBit, 0u, 0u);
     const float4 e = part == 0u   ? make_float4(1.f, 1.f, 1.f, 0.f)
                      : part == 1u ? make_float4(0.f, 0.f, 1.f, 1.f)
@@ -228,20 +238,62 @@ struct Hit {
   uint32_t tri;
 };
 
+// A frame: the child ref in the low half, its entry t's bits in the high one.
+__device__ __forceinline__ uint64_t make_frame(uint32_t ref, float t) {
+  return (uint64_t)__float_as_uint(t) << 32 | ref;
+}
+__device__ __forceinline__ float frame_t(uint64_t f) { return __uint_as_float((uint32_t)(f >> 32)); }
+
+// LDS words by an LDS pointer: through a generic one the stack's accesses
+// become flat memory instructions, which also wait for the vector memory
+// (the serving cast took 2.8 instead of 1.5 ms).
+using LdsFrame = __attribute__((address_space(3))) uint64_t;
+
+// A lane's first S frames in LDS, the next kSpillFrames in its wave's spill
+// area (see the header).  lds and spill point at the lane's column of 64.
 template <int S>
-struct LdsStack {
-  uint2* base;
-  int stride;
-  static constexpr int kCap = S;
-  __device__ __forceinline__ void store(int i, uint2 f) { base[i * stride] = f; }
-  __device__ __forceinline__ uint2 load(int i) const { return base[i * stride]; }
+struct SplitStack {
+  LdsFrame* lds;
+  uint64_t* spill;
+  int sp = 0;
+  __device__ __forceinline__ bool push(uint64_t f) {
+    if (sp < S) {
+      lds[sp * 64] = f;
+    } else {
+      if (sp == S + kSpillFrames) return false;
+      spill[(sp - S) * 64] = f;
+    }
+    ++sp;
+    return true;
+  }
+  // Pops to the next frame whose entry t does not exceed `best`; false when
+  // none is left.
+  __device__ __forceinline__ bool pop(float best, uint64_t& f) {
+    while (sp > 0) {
+      --sp;
+      f = sp < S ? lds[sp * 64] : spill[(sp - S) * 64];
+      if (!(frame_t(f) > best)) return true;
+    }
+    return false;
+  }
 };
 
-struct GlobalStack {
-  uint2* base;
-  static constexpr int kCap = (int)kDeepFrames;
-  __device__ __forceinline__ void store(int i, uint2 f) { base[i] = f; }
-  __device__ __forceinline__ uint2 load(int i) const { return base[i]; }
+// One lane's frames in a run of kDeepFrames words of global memory.
+struct DeepStack {
+  uint64_t* base;
+  uint32_t sp = 0;
+  __device__ __forceinline__ bool push(uint64_t f) {
+    if (sp == kDeepFrames) return false;
+    base[sp++] = f;
+    return true;
+  }
+  __device__ __forceinline__ bool pop(float best, uint64_t& f) {
+    while (sp > 0) {
+      f = base[--sp];
+      if (!(frame_t(f) > best)) return true;
+    }
+    return false;
+  }
 };
 
 // Rust's tuple `<` on (tmin, tmax).
@@ -262,21 +314,51 @@ __device__ __forceinline__ void leaf_test(const Packed& pk, uint32_t slot, const
   tri_out = has ? __float_as_uint(lt.c.y) : DMSH_U32MAX;
 }
 
-// Slab test for rays with finite origin and finite reciprocal direction on
-// every axis, against a finite box.  No t below can be NaN then, so min / max
-// instructions pick the same values as the compare-and-select of slab_hit up
-// to the sign of a zero, which no later comparison can see.
-__device__ __forceinline__ bool slab_hit_finite(const RaySlab& r, const float lo[3],
-                                                const float hi[3], float& tmin_out,
-                                                float& tmax_out) {
-  const float a0 = (lo[0] - r.o[0]) * r.inv[0], b0 = (hi[0] - r.o[0]) * r.inv[0];
-  const float a1 = (lo[1] - r.o[1]) * r.inv[1], b1 = (hi[1] - r.o[1]) * r.inv[1];
-  const float a2 = (lo[2] - r.o[2]) * r.inv[2], b2 = (hi[2] - r.o[2]) * r.inv[2];
-  const float tmin = fmaxf(fmaxf(fminf(a0, b0), fminf(a1, b1)), fminf(a2, b2));
-  const float tmax = fminf(fminf(fmaxf(a0, b0), fmaxf(a1, b1)), fmaxf(a2, b2));
+// Slab test for a regular ray (see regular_ray) against a finite box with
+// lo <= hi.  The plane a ray enters through is lo for a positive reciprocal and
+// hi for a negative one: with lo <= hi and correctly rounded (so monotone)
+// subtraction and product that t is the smaller of the two, so selecting the
+// plane gives what the general test's compare-and-select gives, up to the sign
+// of a zero, which no later comparison can see.  A parallel axis carries the
+// reciprocal +inf: lo < o gives -inf, lo > o gives +inf, and lo == o gives NaN,
+// which fmaxf ignores as it would -inf (for hi: fminf, +inf); so an origin
+// outside the slab leaves tmin = +inf or tmax = -inf and misses (the ray has an
+// axis that is not parallel, whose t is finite or of the missing sign), and one
+// inside leaves the axis out, as the general test does.
+__device__ __forceinline__ bool slab_hit_regular(const RaySlab& r, const bool neg[3],
+                                                 const float lo[3], const float hi[3],
+                                                 float& tmin_out, float& tmax_out) {
+  float tn[3], tf[3];
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    tn[i] = ((neg[i] ? hi[i] : lo[i]) - r.o[i]) * r.inv[i];
+    tf[i] = ((neg[i] ? lo[i] : hi[i]) - r.o[i]) * r.inv[i];
+  }
+  const float tmin = fmaxf(fmaxf(tn[0], tn[1]), tn[2]);
+  const float tmax = fminf(fminf(tf[0], tf[1]), tf[2]);
   tmin_out = tmin;
   tmax_out = tmax;
   return !(tmin > tmax) && !(tmax < 0.f);
+}
+
+// Whether slab_hit_regular serves this ray: a finite origin, and per axis a
+// finite nonzero reciprocal or a direction of exactly 0, not 0 on all three.
+// Makes the reciprocals of parallel axes +inf.
+__device__ __forceinline__ bool regular_ray(RaySlab& r, bool neg[3]) {
+  bool ok = true, some = false;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const float a = fabsf(r.inv[i]);
+    ok = ok && a > 0.f && fabsf(r.o[i]) < __builtin_inff();  // false for a NaN
+    some = some || a < __builtin_inff();
+  }
+  ok = ok && some;
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    if (ok && r.par[i]) r.inv[i] = __builtin_inff();
+    neg[i] = r.inv[i] < 0.f;
+  }
+  return ok;
 }
 
 constexpr uint32_t kNoTest = DMSH_U32MAX;
@@ -286,35 +368,23 @@ constexpr uint32_t kNoTest = DMSH_U32MAX;
 // search when the stack runs out); then expands the lane's node, if any; then
 // runs the (single) leaf-test site if the pop or the expansion produced a
 // leaf, so a wave whose lanes diverge between these steps pays for the
-// triangle test once.
-template <bool kFinite, class Stack>
-__device__ __forceinline__ int trace_loop(const Packed& pk, const RaySlab& r, const float org[3],
-                                          const float dir[3], Stack& stk, Hit& out) {
-  bool res_has = false;
-  float res_t = 0.f;
-  uint32_t res_tri = DMSH_U32MAX;
+// triangle test once.  best is +inf until a triangle is hit.
+template <bool kRegular, class Stack>
+__device__ __forceinline__ int trace_loop(const Packed& pk, const RaySlab& r, const bool neg[3],
+                                          const float org[3], const float dir[3], Stack& stk,
+                                          Hit& out) {
+  float best = __builtin_inff();
+  uint32_t best_tri = DMSH_U32MAX;
   uint32_t node = 0;
-  int sp = 0;
   bool expand = true;
   for (;;) {
     uint32_t test = kNoTest;
     if (!expand) {
-      uint2 f = make_uint2(0u, 0u);
-      bool found = false;
-      while (sp > 0) {
-        f = stk.load(--sp);
-        if (!(res_has && __uint_as_float(f.y) > res_t)) {
-          found = true;
-          break;
-        }
-      }
-      if (!found) break;
-      if (f.x & kLeafBit) {
-        test = f.x & kIndexMask;
-      } else {
-        node = f.x;
-        expand = true;
-      }
+      uint64_t f;
+      if (!stk.pop(best, f)) break;
+      node = (uint32_t)f;
+      expand = !(node & kLeafBit);
+      if (!expand) test = node & kIndexMask;
     }
     if (expand) {
       const InnerNode nd = pk.inner[node];
@@ -322,9 +392,9 @@ __device__ __forceinline__ int trace_loop(const Packed& pk, const RaySlab& r, co
       const float l1[3] = {nd.b.z, nd.b.w, nd.c.x}, h1[3] = {nd.c.y, nd.c.z, nd.c.w};
       float tl0, tl1, tr0, tr1;
       bool hl, hr;
-      if (kFinite) {
-        hl = slab_hit_finite(r, l0, h0, tl0, tl1);
-        hr = slab_hit_finite(r, l1, h1, tr0, tr1);
+      if (kRegular) {
+        hl = slab_hit_regular(r, neg, l0, h0, tl0, tl1);
+        hr = slab_hit_regular(r, neg, l1, h1, tr0, tr1);
       } else {
         hl = slab_hit(r, l0, h0, tl0, tl1);
         hr = slab_hit(r, l1, h1, tr0, tr1);
@@ -332,8 +402,10 @@ __device__ __forceinline__ int trace_loop(const Packed& pk, const RaySlab& r, co
       uint32_t next = kNoTest;
       if (hl && hr) {
         const bool nl = tuple_lt(tl0, tl1, tr0, tr1);
-        if (sp == Stack::kCap) return kTraceOverflow;
-        stk.store(sp++, make_uint2(nl ? nd.d.y : nd.d.x, __float_as_uint(nl ? tr0 : tl0)));
+        const float tfar = nl ? tr0 : tl0;
+        // a far child beyond the best hit would only be skipped later
+        if (!(tfar > best) && !stk.push(make_frame(nl ? nd.d.y : nd.d.x, tfar)))
+          return kTraceOverflow;
         next = nl ? nd.d.x : nd.d.y;
       } else if (hl || hr) {
         next = hl ? nd.d.x : nd.d.y;
@@ -352,34 +424,29 @@ __device__ __forceinline__ int trace_loop(const Packed& pk, const RaySlab& r, co
       float t;
       uint32_t tri;
       leaf_test(pk, test, org, dir, has, t, tri);
-      if (has && (!res_has || t <= res_t)) {
-        res_has = true;
-        res_t = t;
-        res_tri = tri;
+      if (has && t <= best) {
+        best = t;
+        best_tri = tri;
       }
     }
   }
-  out.has = res_has;
-  out.t = res_t;
-  out.tri = res_tri;
+  out.has = best < __builtin_inff();
+  out.t = best;
+  out.tri = best_tri;
   return kTraceOk;
 }
 
-// boxes_finite: every packed child box is finite (checked while packing).
+// regular: every packed child box is finite with lo <= hi (checked while
+// packing).
 template <class Stack>
 __device__ __forceinline__ int trace(const Packed& pk, const float org[3], const float dir[3],
-                                     Stack& stk, Hit& out, bool boxes_finite) {
+                                     Stack& stk, Hit& out, bool regular) {
   out.has = false;
   out.t = 0.f;
   out.tri = DMSH_U32MAX;
   if (pk.num_leaf == 0) return kTraceOk;
   RaySlab r;
   make_slab(org, dir, r);
-  const bool lane_finite = !r.par[0] && !r.par[1] && !r.par[2] &&
-                           fabsf(org[0]) < __builtin_inff() && fabsf(org[1]) < __builtin_inff() &&
-                           fabsf(org[2]) < __builtin_inff();
-  // one path for the whole wave, so the vote must come before any return
-  const bool all_finite = __all(boxes_finite && lane_finite);
   {
     const float lo[3] = {pk.root_box[0], pk.root_box[1], pk.root_box[2]};
     const float hi[3] = {pk.root_box[3], pk.root_box[4], pk.root_box[5]};
@@ -387,128 +454,198 @@ __device__ __forceinline__ int trace(const Packed& pk, const float org[3], const
     if (!slab_hit(r, lo, hi, ta, tb)) return kTraceOk;
   }
   if (pk.num_leaf == 1) {
-    bool has;
-    float t;
-    uint32_t tri;
-    leaf_test(pk, 0, org, dir, has, t, tri);
-    out.has = has;
-    out.t = t;
-    out.tri = tri;
+    leaf_test(pk, 0, org, dir, out.has, out.t, out.tri);
     return kTraceOk;
   }
-  if (all_finite) return trace_loop<true>(pk, r, org, dir, stk, out);
-  return trace_loop<false>(pk, r, org, dir, stk, out);
+  // one path for all lanes still here
+  bool neg[3];
+  RaySlab q = r;
+  if (__all(regular && regular_ray(q, neg)))
+    return trace_loop<true>(pk, q, neg, org, dir, stk, out);
+  return trace_loop<false>(pk, r, neg, org, dir, stk, out);
 }
 
-// Workgroups are dealt to the 8 XCDs round-robin; renumber them so that each
-// XCD receives one contiguous run of logical blocks.
-__device__ __forceinline__ uint32_t xcd_contiguous(uint32_t b, uint32_t nblk) {
-  const uint32_t per = nblk / 8u, rem = nblk % 8u, x = b % 8u, local = b / 8u;
-  const uint32_t start = (x < rem) ? x * (per + 1u) : rem * (per + 1u) + (x - rem) * per;
-  return start + local;
+// Tiles of the images of one launch, dealt to a fixed grid of waves.  Chunks
+// of neighbouring tiles go to the XCDs in turn: their rays share BVH nodes in
+// one L2, and every XCD gets a like share of the work, so no wave has to look
+// for tiles elsewhere.  A wave's first tile is that of its own place in its
+// XCD's list, the later ones come from the XCD's ticket counter one at a time.
+// (Device-scope atomics on one word run ~14 ns one after another: when every
+// wave also went past the other XCDs' counters at the end, that alone took 60 us
+// of a launch.  Runs of 2 to 8 tiles a ticket, or a fixed share with tickets
+// only for the rest, were slower: 24 requests of 7.3 M rays in all 1.61 ms with
+// single tiles, 1.78 with runs of 2, 1.86 with 8, 1.79 to 2.0 with a fixed
+// share.)
+struct TileDeal {
+  uint32_t* ticket;        // of this XCD
+  uint32_t shift;          // log2 of the chunk
+  uint32_t groups, group;  // XCDs in use, this wave's
+  uint32_t len;            // tiles (some past the end) of this XCD
+  uint32_t waves;          // waves of this XCD
+  uint32_t own;            // this wave's first, then kTaken
+  static constexpr uint32_t kTaken = DMSH_U32MAX;
+
+  template <int W>
+  static __device__ __forceinline__ TileDeal make(uint32_t* counts, uint32_t num_tiles) {
+    TileDeal d;
+    d.groups = gridDim.x < kXcds ? gridDim.x : kXcds;
+    d.group = blockIdx.x % d.groups;
+    d.ticket = counts + 32u + 32u * d.group;
+    // chunks of up to 256 tiles, at least 16 of them on each XCD
+    const uint32_t want = num_tiles / (d.groups * 16u);
+    d.shift = want == 0u ? 0u : 31u - (uint32_t)__builtin_clz(want);
+    if (d.shift > 8u) d.shift = 8u;
+    const uint32_t round = d.groups << d.shift;
+    d.len = (num_tiles / round + (num_tiles % round != 0u ? 1u : 0u)) << d.shift;
+    d.waves = (gridDim.x + d.groups - 1u - d.group) / d.groups * (uint32_t)W;
+    d.own = blockIdx.x / d.groups * (uint32_t)W + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    return d;
+  }
+  // the next tile, the same in every lane (it may be past the end); false
+  // when none is left
+  __device__ __forceinline__ bool next(uint32_t& tile) {
+    uint32_t q = own;
+    if (q == kTaken) {
+      if (waves >= len) return false;
+      uint32_t t = 0u;
+      if ((threadIdx.x & 63u) == 0u) t = atomicAdd(ticket, 1u);
+      q = waves + __builtin_amdgcn_readfirstlane(t);
+    }
+    own = kTaken;
+    if (q >= len) return false;
+    tile = (((q >> shift) * groups + group) << shift) + (q & ((1u << shift) - 1u));
+    return true;
+  }
+};
+
+// Largest m < M with off[m] <= x (off[0] <= x; off ascending), by the whole
+// wave: 64 entries a round trip.
+__device__ __forceinline__ uint32_t wave_segment(const uint32_t* __restrict__ off, uint32_t M,
+                                                 uint32_t x) {
+  const uint32_t lane = threadIdx.x & 63u;
+  uint32_t lo = 0u, n = M;
+  for (;;) {
+    const uint32_t step = n / 64u + (n % 64u != 0u ? 1u : 0u);
+    const bool mine = lane * step < n;
+    const uint64_t below = __ballot(mine && off[lo + (mine ? lane * step : 0u)] <= x);
+    const uint32_t k = ((uint32_t)__popcll(below) - 1u) * step;
+    lo += k;
+    if (step == 1u) return lo;
+    n = n - k < step ? n - k : step;
+  }
 }
 
-struct CastArgs {
-  uint32_t* pix2tri;
-  float* pix2t;
-  uint32_t img_w, img_h, tiles_x, num_tiles;
-  uint32_t* counts;  // [0]: tier-2 queue length, [1]: tier-3 queue length,
-                     // [2]: nonzero when a packed box is not finite
-  uint32_t* list2;
-  uint32_t* list3;
-  uint2* deep_stack;
+// Upper bound of the 8x8 tiles of `images` images with num_pix pixels in all:
+// a w x h image has at most (w / 8 + 1)(h / 8 + 1) <= wh (1/64 + 1/8) + 9/8.
+inline uint32_t max_tiles(uint64_t num_pix, uint64_t images) {
+  const uint64_t t = num_pix * 9u / 64u + 2u * images + 1u;
+  return t < num_pix ? (uint32_t)t : (uint32_t)num_pix;
+}
+// Waves of a launch over at most `tiles` tiles, and the words of spill area
+// each of them owns.
+inline uint32_t cast_waves(uint32_t tiles) { return tiles < kMaxCastWaves ? tiles : kMaxCastWaves; }
+// Waves per CU that fit its 160 KB of LDS with S frames a lane (of the 32 that
+// their registers allow): a wave of the grid that starts late holds its fixed
+// share of the tiles back.
+constexpr uint32_t resident_waves(int S) {
+  return 160u * 1024u / (uint32_t)(S * 512) < 32u ? 160u * 1024u / (uint32_t)(S * 512) : 32u;
+}
+constexpr size_t kSpillPerWave = (size_t)kSpillFrames * 64;
+
+struct CastState {
+  uint32_t* counts;  // [kCastCounts]: [2] nonzero when a box is not regular (one
+                     // tree, batch), [3] offsets rejected, [32 + 32 x] tickets of XCD x: each on
+                     // a 128-byte line of its own, away from the flags, which
+                     // every tile reads (a load waits behind the line's atomics)
+  uint64_t* spill;   // [waves][kSpillPerWave]
   uint32_t* err;
 };
 
-__device__ __forceinline__ void write_result(const CastArgs& a, uint32_t ip, const Hit& h) {
-  a.pix2tri[ip] = h.has ? h.tri : DMSH_U32MAX;
-  if (a.pix2t) a.pix2t[ip] = h.has ? h.t : 0.f;
+// One wave's share of a launch.  Src: num_tiles(), and load(tile, lane, job)
+// for the pixel of a lane: whether it lies in its image, its ray's transform
+// (16 floats, column-major), tree and output position.
+struct PixelJob {
+  Packed pk;
+  const float* T;
+  uint32_t iw, ih, w, h;
+  uint32_t out;
+  bool regular;
+};
+
+template <int S, int W, class Src>
+__device__ __forceinline__ void cast_wave(const Src& src, const CastState& st, LdsFrame* lds,
+                                          uint32_t* __restrict__ pix2tri,
+                                          float* __restrict__ pix2t) {
+  const uint32_t lane = threadIdx.x & 63u;
+  uint64_t* spill = st.spill + (size_t)(blockIdx.x * (uint32_t)W +
+                                     __builtin_amdgcn_readfirstlane(threadIdx.x >> 6)) *
+                                kSpillPerWave;
+  const uint32_t num_tiles = src.num_tiles();
+  TileDeal deal = TileDeal::make<W>(st.counts, num_tiles);
+  uint32_t tile;
+  while (deal.next(tile)) {
+    if (tile >= num_tiles) continue;
+    PixelJob j;
+    const bool in = src.load(tile, lane, j);
+    bool deep = false;
+    float org[3], dir[3];
+    Hit hit;
+    if (in) {
+      float m[16];
+#pragma unroll
+      for (int k = 0; k < 16; ++k) m[k] = j.T[k];
+      ray_for_pixel(j.iw, j.ih, j.w, j.h, m, org, dir);
+      SplitStack<S> stk{lds + lane, spill + lane};
+      deep = trace(j.pk, org, dir, stk, hit, j.regular) == kTraceOverflow;
+    }
+    // lanes that ran out of frames, one after the other
+    for (uint64_t left = __ballot(deep); left != 0; left &= left - 1) {
+      if (lane == (uint32_t)__builtin_ctzll(left)) {
+        DeepStack stk{spill};
+        if (trace(j.pk, org, dir, stk, hit, false) != kTraceOk) {
+          raise_error(st.err, DMSH_DEVERR_STACK);
+          hit.has = false;
+        }
+      }
+    }
+    if (in) {
+      pix2tri[j.out] = hit.has ? hit.tri : DMSH_U32MAX;
+      if (pix2t) pix2t[j.out] = hit.has ? hit.t : 0.f;
+    }
+  }
+}
+
+// A single image of one tree.
+struct ImageSrc {
+  Packed pk;
+  const float* T;
+  uint32_t img_w, img_h, tiles_x, tiles;
+  const uint32_t* counts;
+  __device__ __forceinline__ uint32_t num_tiles() const { return tiles; }
+  __device__ __forceinline__ bool load(uint32_t tile, uint32_t lane, PixelJob& j) const {
+    j.pk = pk;
+    j.T = T;
+    j.w = img_w;
+    j.h = img_h;
+    j.iw = (tile % tiles_x) * 8u + (lane & 7u);
+    j.ih = (tile / tiles_x) * 8u + (lane >> 3);
+    j.out = j.ih * img_w + j.iw;
+    j.regular = counts[2] == 0u;
+    return j.iw < img_w && j.ih < img_h;
+  }
+};
+
+template <int S, int W>
+__global__ __launch_bounds__(64 * W) void k_pix2tri(ImageSrc src, CastState st,
+                                                    uint32_t* __restrict__ pix2tri,
+                                                    float* __restrict__ pix2t) {
+  __shared__ uint64_t s_stack[W][S][64];
+  cast_wave<S, W>(src, st, (LdsFrame*)&s_stack[threadIdx.x >> 6][0][0], pix2tri, pix2t);
 }
 
 __device__ __forceinline__ void load_transform(const float* __restrict__ T, float m[16]) {
 #pragma unroll
   for (int k = 0; k < 16; ++k) m[k] = T[k];
-}
-
-// Tier 1: one ray per lane, 8x8 pixel tiles per wave.
-template <int S, int WAVES>
-__global__ __launch_bounds__(64 * WAVES) void k_pix2tri(Packed pk, const float* __restrict__ T,
-                                                        CastArgs a) {
-  __shared__ uint2 s_stack[S][64 * WAVES];
-  const uint32_t tid = threadIdx.x, wave = tid >> 6, lane = tid & 63u;
-  const uint32_t tile = xcd_contiguous(blockIdx.x, gridDim.x) * WAVES + wave;
-  if (tile >= a.num_tiles) return;
-  const uint32_t iw = (tile % a.tiles_x) * 8u + (lane & 7u);
-  const uint32_t ih = (tile / a.tiles_x) * 8u + (lane >> 3);
-  if (iw >= a.img_w || ih >= a.img_h) return;
-  float m[16];
-  load_transform(T, m);
-  float org[3], dir[3];
-  ray_for_pixel(iw, ih, a.img_w, a.img_h, m, org, dir);
-  LdsStack<S> stk{&s_stack[0][tid], 64 * WAVES};
-  Hit h;
-  const int st = trace(pk, org, dir, stk, h, a.counts[2] == 0u);
-  const uint32_t ip = ih * a.img_w + iw;
-  if (st == kTraceOverflow) {
-    a.list2[atomicAdd(a.counts + 0, 1u)] = ip;
-    return;
-  }
-  write_result(a, ip, h);
-}
-
-// Tier 2: queued rays, 64 LDS frames per lane, grid-stride over the queue.
-static __global__ __launch_bounds__(64) void k_pix2tri_tier2(Packed pk,
-                                                             const float* __restrict__ T,
-                                                             CastArgs a) {
-  __shared__ uint2 s_stack[kTier2Frames][64];
-  const uint32_t num_pix = a.img_w * a.img_h;
-  uint32_t count = a.counts[0];
-  if (count > num_pix) count = num_pix;
-  float m[16];
-  load_transform(T, m);
-  LdsStack<kTier2Frames> stk{&s_stack[0][threadIdx.x], 64};
-  const bool boxes_finite = a.counts[2] == 0u;
-  for (uint32_t e = blockIdx.x * 64u + threadIdx.x; e < count; e += gridDim.x * 64u) {
-    const uint32_t ip = a.list2[e];
-    const uint32_t ih = ip / a.img_w, iw = ip - ih * a.img_w;
-    float org[3], dir[3];
-    ray_for_pixel(iw, ih, a.img_w, a.img_h, m, org, dir);
-    Hit h;
-    const int st = trace(pk, org, dir, stk, h, boxes_finite);
-    if (st == kTraceOverflow) {
-      a.list3[atomicAdd(a.counts + 1, 1u)] = ip;
-      continue;
-    }
-    write_result(a, ip, h);
-  }
-}
-
-// Tier 3: a fixed grid of kDeepSlots threads, each owning a global stack slot.
-static __global__ __launch_bounds__(64) void k_pix2tri_tier3(Packed pk,
-                                                             const float* __restrict__ T,
-                                                             CastArgs a) {
-  const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t nthr = gridDim.x * blockDim.x;
-  const uint32_t num_pix = a.img_w * a.img_h;
-  uint32_t count = a.counts[1];
-  if (count > num_pix) count = num_pix;
-  float m[16];
-  load_transform(T, m);
-  GlobalStack stk{a.deep_stack + (size_t)gid * kDeepFrames};
-  const bool boxes_finite = a.counts[2] == 0u;
-  for (uint32_t e = gid; e < count; e += nthr) {
-    const uint32_t ip = a.list3[e];
-    const uint32_t ih = ip / a.img_w, iw = ip - ih * a.img_w;
-    float org[3], dir[3];
-    ray_for_pixel(iw, ih, a.img_w, a.img_h, m, org, dir);
-    Hit h;
-    const int st = trace(pk, org, dir, stk, h, boxes_finite);
-    if (st != kTraceOk) {
-      raise_error(a.err, DMSH_DEVERR_STACK);
-      h.has = false;
-    }
-    write_result(a, ip, h);
-  }
 }
 
 // ---------------------------------------------------------------------------

@@ -161,21 +161,6 @@ struct Request {
 };
 static_assert(sizeof(Request) == 96, "request layout");
 
-struct ReqCast {
-  uint32_t R;
-  const Request* req;
-  const uint32_t* tile_off;  // [R + 1]
-  const uint32_t* pix_off;   // [R + 1]
-  uint32_t* pix2tri;
-  float* pix2t;
-  uint32_t* counts;  // [0] tier-2 queue, [1] tier-3 queue, [3] requests rejected,
-                     // [16 + 16 x] tile counter of XCD x
-  uint32_t* list2;
-  uint32_t* list3;
-  uint2* deep_stack;
-  uint32_t* err;
-};
-
 // Tile and pixel offsets of the requests; rejects (counts[3], DMSH_DEVERR_INDEX)
 // images that are empty or do not follow one another in pixel order.
 static __global__ __launch_bounds__(1024) void k_req_offsets(uint32_t R, uint32_t total_pix,
@@ -206,119 +191,37 @@ static __global__ __launch_bounds__(1024) void k_req_offsets(uint32_t R, uint32_
   }
 }
 
-__device__ __forceinline__ rc::Packed packed_of(const Request& q) {
-  const PackedRef p = packed_ref(q.packed, q.num_tri);
-  return rc::Packed{p.inner, p.leaf, p.root_box, q.num_tri};
-}
-
-// The general slab test is taken when the request or the tree says so.
-__device__ __forceinline__ bool boxes_finite(const Request& q) {
-  return q.nonfinite == 0u && (q.num_tri == 0 || *packed_flag(q.packed, q.num_tri) == 0u);
-}
-
-__device__ __forceinline__ void req_write(const ReqCast& a, uint32_t gp, const rc::Hit& h) {
-  a.pix2tri[gp] = h.has ? h.tri : DMSH_U32MAX;
-  if (a.pix2t) a.pix2t[gp] = h.has ? h.t : 0.f;
-}
-
-__device__ __forceinline__ uint32_t req_next_tile(uint32_t* counts, uint32_t num_tiles,
-                                                  uint32_t& xcd) {
-  const uint32_t per = (num_tiles + bat::kXcds - 1) / bat::kXcds;
-  for (uint32_t tries = 0; tries < bat::kXcds; ++tries) {
-    const uint32_t lo = xcd * per;
-    const uint32_t hi = (lo + per < num_tiles) ? lo + per : num_tiles;
-    uint32_t t = 0;
-    if ((threadIdx.x & 63u) == 0) t = atomicAdd(counts + 16 + 16 * xcd, 1u);
-    t = __builtin_amdgcn_readfirstlane(t) + lo;
-    if (t < hi) return t;
-    xcd = (xcd + 1) % bat::kXcds;
+// The images of the requests.  The general slab test is taken when the
+// request or the tree says so.
+struct ReqSrc {
+  uint32_t R;
+  const Request* req;
+  const uint32_t* tile_off;  // [R + 1]
+  const uint32_t* counts;
+  __device__ __forceinline__ uint32_t num_tiles() const { return counts[3] ? 0u : tile_off[R]; }
+  __device__ __forceinline__ bool load(uint32_t tile, uint32_t lane, rc::PixelJob& j) const {
+    const uint32_t r = rc::wave_segment(tile_off, R, tile);
+    const Request& q = req[r];
+    const PackedRef p = packed_ref(q.packed, q.num_tri);
+    j.pk = rc::Packed{p.inner, p.leaf, p.root_box, q.num_tri};
+    j.T = q.ndc2world;
+    j.w = q.img_w;
+    j.h = q.img_h;
+    const uint32_t tiles_x = ceil_div_u32(j.w, 8u), lt = tile - tile_off[r];
+    j.iw = (lt % tiles_x) * 8u + (lane & 7u);
+    j.ih = (lt / tiles_x) * 8u + (lane >> 3);
+    j.out = q.pix_start + j.ih * j.w + j.iw;
+    j.regular = q.nonfinite == 0u && (q.num_tri == 0 || *packed_flag(q.packed, q.num_tri) == 0u);
+    return j.iw < j.w && j.ih < j.h;
   }
-  return num_tiles;
-}
+};
 
-template <int S>
-__global__ __launch_bounds__(64) void k_req_pix2tri(ReqCast a) {
-  __shared__ uint2 s_stack[S][64];
-  const uint32_t lane = threadIdx.x;
-  if (a.counts[3]) return;
-  const uint32_t num_tiles = a.tile_off[a.R];
-  uint32_t xcd = blockIdx.x % bat::kXcds;
-  for (;;) {
-    const uint32_t tile = req_next_tile(a.counts, num_tiles, xcd);
-    if (tile >= num_tiles) break;
-    const uint32_t r = bat::find_segment(a.tile_off, a.R, tile);
-    const Request& q = a.req[r];
-    const uint32_t w = q.img_w, h = q.img_h;
-    const uint32_t tiles_x = ceil_div_u32(w, 8u), lt = tile - a.tile_off[r];
-    const uint32_t iw = (lt % tiles_x) * 8u + (lane & 7u), ih = (lt / tiles_x) * 8u + (lane >> 3);
-    if (iw < w && ih < h) {
-      float T[16];
-      rc::load_transform(q.ndc2world, T);
-      float org[3], dir[3];
-      ray_for_pixel(iw, ih, w, h, T, org, dir);
-      rc::LdsStack<S> stk{&s_stack[0][lane], 64};
-      rc::Hit hit;
-      const int st = rc::trace(packed_of(q), org, dir, stk, hit, boxes_finite(q));
-      const uint32_t gp = q.pix_start + ih * w + iw;
-      if (st == rc::kTraceOverflow) a.list2[atomicAdd(a.counts + 0, 1u)] = gp;
-      else req_write(a, gp, hit);
-    }
-  }
-}
-
-__device__ __forceinline__ uint32_t req_pixel(const ReqCast& a, uint32_t gp, uint32_t& iw,
-                                              uint32_t& ih) {
-  const uint32_t r = bat::find_segment(a.pix_off, a.R, gp);
-  const uint32_t w = a.req[r].img_w;
-  ih = (gp - a.pix_off[r]) / w;
-  iw = gp - a.pix_off[r] - ih * w;
-  return r;
-}
-
-static __global__ __launch_bounds__(64) void k_req_pix2tri_tier2(ReqCast a, uint32_t total_pix) {
-  __shared__ uint2 s_stack[rc::kTier2Frames][64];
-  if (a.counts[3]) return;
-  uint32_t count = a.counts[0];
-  if (count > total_pix) count = total_pix;
-  rc::LdsStack<rc::kTier2Frames> stk{&s_stack[0][threadIdx.x], 64};
-  for (uint32_t e = blockIdx.x * 64u + threadIdx.x; e < count; e += gridDim.x * 64u) {
-    const uint32_t gp = a.list2[e];
-    uint32_t iw, ih;
-    const uint32_t r = req_pixel(a, gp, iw, ih);
-    const Request& q = a.req[r];
-    float T[16], org[3], dir[3];
-    rc::load_transform(q.ndc2world, T);
-    ray_for_pixel(iw, ih, q.img_w, q.img_h, T, org, dir);
-    rc::Hit hit;
-    const int st = rc::trace(packed_of(q), org, dir, stk, hit, boxes_finite(q));
-    if (st == rc::kTraceOverflow) a.list3[atomicAdd(a.counts + 1, 1u)] = gp;
-    else req_write(a, gp, hit);
-  }
-}
-
-static __global__ __launch_bounds__(64) void k_req_pix2tri_tier3(ReqCast a, uint32_t total_pix) {
-  const uint32_t gid = blockIdx.x * blockDim.x + threadIdx.x;
-  const uint32_t nthr = gridDim.x * blockDim.x;
-  if (a.counts[3]) return;
-  uint32_t count = a.counts[1];
-  if (count > total_pix) count = total_pix;
-  rc::GlobalStack stk{a.deep_stack + (size_t)gid * rc::kDeepFrames};
-  for (uint32_t e = gid; e < count; e += nthr) {
-    const uint32_t gp = a.list3[e];
-    uint32_t iw, ih;
-    const uint32_t r = req_pixel(a, gp, iw, ih);
-    const Request& q = a.req[r];
-    float T[16], org[3], dir[3];
-    rc::load_transform(q.ndc2world, T);
-    ray_for_pixel(iw, ih, q.img_w, q.img_h, T, org, dir);
-    rc::Hit hit;
-    const int st = rc::trace(packed_of(q), org, dir, stk, hit, boxes_finite(q));
-    if (st != rc::kTraceOk) {
-      raise_error(a.err, DMSH_DEVERR_STACK);
-      hit.has = false;
-    }
-    req_write(a, gp, hit);
-  }
+template <int S, int W>
+__global__ __launch_bounds__(64 * W) void k_req_pix2tri(ReqSrc src, rc::CastState st,
+                                                        uint32_t* __restrict__ pix2tri,
+                                                        float* __restrict__ pix2t) {
+  __shared__ uint64_t s_stack[W][S][64];
+  rc::cast_wave<S, W>(src, st, (rc::LdsFrame*)&s_stack[threadIdx.x >> 6][0][0], pix2tri, pix2t);
 }
 
 }  // namespace srv

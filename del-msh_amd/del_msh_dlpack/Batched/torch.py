@@ -311,7 +311,7 @@ def _time_ms(fn, reps: int) -> float:
     return start.elapsed_time(stop) / reps
 
 
-def autotune(p: Pipeline, reps: int = 2, stacks=(16, 20, 24, 32), wgs_per_cu=(4, 8, 16, 32),
+def autotune(p: Pipeline, reps: int = 2, stacks=(12, 16, 20, 24, 32), wgs_per_cu=(4, 8, 16, 32),
              cast_waves=(1, 2, 4), treelet_grids=(512, 1024, 2048), sort_items=(8, 12, 16),
              sort_seg=(1, 0)):
     """Times the launch parameters of the batched kernels on this batch and

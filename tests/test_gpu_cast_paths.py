@@ -1,0 +1,75 @@
+"""GPU: the ray-cast where its stack leaves LDS and where its regular slab test
+meets parallel axes on a box's plane, against the oracle bit for bit."""
+
+import numpy as np
+import pytest
+import torch
+
+from del_msh_dlpack import _lib
+import del_msh_dlpack.Pix2Tri.torch as Pix2Tri
+
+pytestmark = pytest.mark.gpu
+
+
+def _cast_equals_oracle(gpu, oracle, tri, vtx, n2w, w, h):
+    bn, aabb = oracle.build_trimesh3(tri, vtx)
+    dev = [torch.from_numpy(a).to(gpu) for a in (tri, vtx, bn, aabb, n2w)]
+    pix, t = Pix2Tri.by_raycasting_with_coeff(*dev, (w, h))
+    want, want_t, _ = oracle.pix2tri(tri, vtx, bn, aabb, n2w.T.reshape(-1), w, h, num_threads=4)
+    assert np.array_equal(pix.cpu().numpy(), want)
+    assert np.array_equal(t.cpu().numpy().view(np.uint32), want_t.view(np.uint32))
+    assert _lib.device_errors() == 0
+    return want
+
+
+# 12 frames in LDS, 64 more in the spill area, then a lone lane's stack
+@pytest.mark.parametrize("sheets", [11, 13, 14, 60, 77, 79, 200])
+@pytest.mark.parametrize("size", [(8, 8), (33, 17)])
+def test_stack_beyond_lds_and_spill(gpu, oracle, sheets, size):
+    """Sheets in one Morton cell, listed far to near, put a frame on the stack
+    for every sheet."""
+    tri, vtx = [], []
+    for k in range(sheets):
+        z = -0.001 + k * (0.0016 / sheets)
+        tri.append([len(vtx), len(vtx) + 1, len(vtx) + 2])
+        vtx += [[-0.5, -0.5, z], [0.6, -0.45, z], [-0.45, 0.6, z]]
+    for s in (-1.0, 1.0):
+        tri.append([len(vtx), len(vtx) + 1, len(vtx) + 2])
+        vtx += [[s * 4, s * 4, 0], [s * 4 + 0.01, s * 4, 0], [s * 4, s * 4 + 0.01, 0]]
+    n2w = np.diag([1.0, 1.0, 1.0, 1.0]).astype(np.float32)
+    want = _cast_equals_oracle(gpu, oracle, np.array(tri, np.uint32), np.array(vtx, np.float32),
+                               n2w, *size)
+    assert (want == sheets - 1).any()
+
+
+@pytest.mark.parametrize("flip", [(1, 1, 1), (-1, 1, 1), (1, 1, -1)])
+@pytest.mark.parametrize("seed", [0, 1])
+def test_rays_in_box_planes(gpu, oracle, flip, seed):
+    """Axis-aligned quads whose edges lie at the pixel centres of an
+    orthographic camera: every ray has two parallel axes and runs in the planes
+    of many boxes (lo == o, hi == o, flat boxes)."""
+    rng = np.random.default_rng(seed)
+    w = 32
+    at = lambda i: 2.0 * (i + 0.5) / w - 1.0
+    tri, vtx = [], []
+    for _ in range(300):
+        x0, y0 = rng.integers(0, w - 1, 2)
+        x1, y1 = x0 + rng.integers(1, 6), y0 + rng.integers(1, 6)
+        z = rng.integers(-8, 8) / 8.0
+        n = len(vtx)
+        vtx += [[at(x0), at(y0), z], [at(x1), at(y0), z], [at(x1), at(y1), z], [at(x0), at(y1), z]]
+        tri += [[n, n + 1, n + 2], [n, n + 2, n + 3]]
+    n2w = np.diag([*flip, 1.0]).astype(np.float32)
+    want = _cast_equals_oracle(gpu, oracle, np.array(tri, np.uint32), np.array(vtx, np.float32),
+                               n2w, w, w)
+    assert (want != 0xFFFFFFFF).sum() > 100
+
+
+def test_rays_without_direction(gpu, oracle):
+    """A camera that maps both NDC planes to one gives rays of length zero,
+    which take the general slab test."""
+    rng = np.random.default_rng(3)
+    vtx = rng.uniform(-1, 1, (60, 3)).astype(np.float32)
+    tri = np.arange(60, dtype=np.uint32).reshape(20, 3)
+    n2w = np.diag([1.0, 1.0, 0.0, 1.0]).astype(np.float32)
+    _cast_equals_oracle(gpu, oracle, tri, vtx, n2w, 16, 16)
