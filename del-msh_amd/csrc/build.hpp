@@ -186,6 +186,40 @@ __device__ __forceinline__ void fit_transform(const uint32_t* __restrict__ keys6
   }
 }
 
+// The reduced box of the copies, in every lane of the wave.
+__device__ __forceinline__ void reduce_box_copies(const uint32_t* __restrict__ keys6,
+                                                  uint32_t k6[6]) {
+#pragma unroll
+  for (int d = 0; d < 6; ++d) k6[d] = keys6[(threadIdx.x & 63u) * kBoxStride + d];
+#pragma unroll
+  for (int off = 32; off >= 1; off >>= 1) {
+#pragma unroll
+    for (int d = 0; d < 6; ++d) {
+      const uint32_t v = __shfl_xor(k6[d], off, 64);
+      k6[d] = d < 3 ? (v < k6[d] ? v : k6[d]) : (v > k6[d] ? v : k6[d]);
+    }
+  }
+}
+
+// The Morton codes of up to sortk::small_capacity elements as the keys of the
+// chunk sort.
+template <typename KeyT>
+struct MortonSrc {
+  const float* pts;
+  const uint32_t* keys6;
+  float T[16];
+  // (wave w reduces all copies for itself: no barrier)
+  __device__ __forceinline__ void prepare() {
+    uint32_t k6[6];
+    reduce_box_copies(keys6, k6);
+    fit_transform(k6, T);
+  }
+  __device__ __forceinline__ KeyT operator()(uint32_t i) const {
+    return morton3_transformed<KeyT>(T, pts[(size_t)i * 3], pts[(size_t)i * 3 + 1],
+                                     pts[(size_t)i * 3 + 2]);
+  }
+};
+
 template <typename KeyT>
 __global__ __launch_bounds__(256) void k_morton_hist(uint32_t n, const float* __restrict__ pts,
                                                      const uint32_t* __restrict__ keys6,
@@ -198,16 +232,7 @@ __global__ __launch_bounds__(256) void k_morton_hist(uint32_t n, const float* __
     (&s_h[0][0])[e] = 0;
   if (threadIdx.x < 64) {  // lane c reads copy c; the wave reduces them
     uint32_t k6[6];
-#pragma unroll
-    for (int d = 0; d < 6; ++d) k6[d] = keys6[threadIdx.x * kBoxStride + d];
-#pragma unroll
-    for (int off = 32; off >= 1; off >>= 1) {
-#pragma unroll
-      for (int d = 0; d < 6; ++d) {
-        const uint32_t v = __shfl_xor(k6[d], off, 64);
-        k6[d] = d < 3 ? (v < k6[d] ? v : k6[d]) : (v > k6[d] ? v : k6[d]);
-      }
-    }
+    reduce_box_copies(keys6, k6);
     if (threadIdx.x == 0) {
 #pragma unroll
       for (int d = 0; d < 6; ++d) s_k6[d] = k6[d];
@@ -334,13 +359,19 @@ inline int build(hipStream_t s, uint32_t n, const uint32_t* tri2vtx, uint32_t nu
                      L.keys6, err);
   if ((rc = launch_status()) != DMSH_OK) return rc;
   KeyT* codes = static_cast<KeyT*>(L.codes);
-  const uint32_t mh_blocks = std::min<uint32_t>(sortk::num_tiles<KeyT>(n), 2048);
-  launch("k_morton_hist", k_morton_hist<KeyT>, dim3(mh_blocks), dim3(256), 0, s, n,
-         TRI ? L.cntr : xyz, L.keys6, codes, sortk::first_hist_pass(P), P, kb, L.sort.hist);
-  if ((rc = launch_status()) != DMSH_OK) return rc;
-  // P is even for 30- and 63-bit codes: the passes end back in `codes`.
-  rc = sortk::run_passes<KeyT>(s, n, kb, L.sort, codes, codes, L.idx, err, true);
-  if (rc != DMSH_OK) return rc;
+  if (n <= sortk::small_capacity<KeyT>()) {
+    rc = sortk::sort_small<KeyT>(s, MortonSrc<KeyT>{TRI ? L.cntr : xyz, L.keys6, {}}, n, kb, codes,
+                                 L.idx, static_cast<KeyT*>(L.sort.alt_keys), L.sort.alt_vals);
+    if (rc != DMSH_OK) return rc;
+  } else {
+    const uint32_t mh_blocks = std::min<uint32_t>(sortk::num_tiles<KeyT>(n), 2048);
+    launch("k_morton_hist", k_morton_hist<KeyT>, dim3(mh_blocks), dim3(256), 0, s, n,
+           TRI ? L.cntr : xyz, L.keys6, codes, sortk::first_hist_pass(P), P, kb, L.sort.hist);
+    if ((rc = launch_status()) != DMSH_OK) return rc;
+    // P is even for 30- and 63-bit codes: the passes end back in `codes`.
+    rc = sortk::run_passes<KeyT>(s, n, kb, L.sort, codes, codes, L.idx, err, true);
+    if (rc != DMSH_OK) return rc;
+  }
   // the topology pass also writes every leaf's box, so the treelet pass
   // loads boxes instead of gathering them
   const bool leaves_in_aabb = refit_option(kRefitLeavesInAabb) == 1;
