@@ -16,8 +16,14 @@
 //     the maximum 64-bit key (edge + 1, step * 4 + pair) per written pixel;
 //     pass 2 repeats the walk and only the write holding the pixel's key
 //     stores its value.
-//   backward: one thread per edge accumulates dL/dp of its two vertices over
-//     its walk and adds them with six float atomics.
+//   backward: dL/dp of an edge's two vertices is accumulated over its walk and
+//     added with six float atomics.
+// A group of kEdgeLanes lanes walks an edge, one step each: the positions are
+// the serial walk's (each lane adds its way to its own), the pixel reads and
+// crossings of the steps run side by side.  With a thread an edge a step cost
+// a chain of up to eight reads and a pass took the longest edge's walk: 46 us
+// for the keys, 50 for the writes and 54 backward on 53 000-triangle meshes at
+// 512^2; with 16 lanes 5.6, 5.8 and 8.6 us.
 // A walk stops once it has left the image in its direction of travel (no
 // pixel after that point can be inside), and edges with a non-finite
 // projection are skipped.
@@ -75,57 +81,63 @@ __device__ __forceinline__ void dldw_intersection_edge2(const float c0[2], const
 // steps a pixel walk may take before it is abandoned (DMSH_DEVERR_WALK)
 constexpr uint32_t kWalkLimit = 1u << 26;
 
+constexpr uint32_t kEdgeLanes = 16;
+static_assert(kWalkLimit % kEdgeLanes == 0, "whole rounds");
+
 struct Pair {
   uint32_t p0, p1;
   float c0[2], c1[2];
 };
 
-// Pair k of the pixel (iw, ih): k = 0 (centre, west|north), 1 (west|north,
-// centre), 2 (centre, east|south), 3 (east|south, centre); west/east when
-// `horizontal`, else the rows ih - 1 / ih + 1.  Index arithmetic is uint32
-// (a west neighbour of column 0 is the previous row's last pixel, the row
-// above row 0 wraps past the image and is dropped by the caller).
-__device__ __forceinline__ Pair make_pair(uint32_t iw, uint32_t ih, uint32_t img_w,
-                                          bool horizontal, int k) {
-  const bool far = (k >> 1) != 0;
-  const uint32_t pc = ih * img_w + iw;
-  const float cx = (float)iw + 0.5f, cy = (float)ih + 0.5f;
-  uint32_t pn;
-  float nx, ny;
-  if (horizontal) {
-    pn = far ? ih * img_w + iw + 1u : ih * img_w + iw - 1u;
-    nx = far ? (float)iw + 1.5f : (float)iw - 0.5f;
-    ny = cy;
-  } else {
-    pn = far ? (ih + 1u) * img_w + iw : (ih - 1u) * img_w + iw;
-    nx = cx;
-    ny = far ? (float)ih + 1.5f : (float)ih - 0.5f;
+// The pairs (0) centre, near; (1) near, centre; (2) centre, far; (3) far,
+// centre of the pixel (iw, ih): near / far are its west / east neighbours when
+// `horizontal`, else those in the rows ih - 1 / ih + 1.  Index arithmetic is
+// uint32 (a west neighbour of column 0 is the previous row's last pixel, the
+// row above row 0 wraps past the image and its pairs are dropped).  Calls
+// fn(pair, rc, seq) for each pair of a foreground and a background pixel that
+// the edge q0 -> q1 crosses, seq = 4 step + pair.
+template <class Fn>
+__device__ __forceinline__ void cross_pixel(const float q0[2], const float q1[2], uint32_t iw,
+                                            uint32_t ih, uint32_t img_w, uint32_t img_h,
+                                            bool horizontal, uint32_t step,
+                                            const uint32_t* __restrict__ pix2tri, Fn& fn) {
+  const uint32_t total = img_w * img_h, pc = ih * img_w + iw;
+  const uint32_t pn[2] = {horizontal ? pc - 1u : (ih - 1u) * img_w + iw,
+                          horizontal ? pc + 1u : (ih + 1u) * img_w + iw};
+  const float c[2] = {(float)iw + 0.5f, (float)ih + 0.5f};
+  // the three reads go out together
+  const bool in[2] = {pn[0] < total, pn[1] < total};
+  const bool bc = pix2tri[pc] == DMSH_U32MAX;
+  const bool bn[2] = {pix2tri[in[0] ? pn[0] : pc] == DMSH_U32MAX,
+                      pix2tri[in[1] ? pn[1] : pc] == DMSH_U32MAX};
+#pragma unroll
+  for (int far = 0; far < 2; ++far) {
+    if (!in[far] || bn[far] == bc) continue;
+    float n[2] = {c[0], c[1]};
+    if (horizontal) n[0] = far ? (float)iw + 1.5f : (float)iw - 0.5f;
+    else n[1] = far ? (float)ih + 1.5f : (float)ih - 0.5f;
+    Pair pr;  // foreground first
+    pr.p0 = bc ? pn[far] : pc;
+    pr.p1 = bc ? pc : pn[far];
+#pragma unroll
+    for (int d = 0; d < 2; ++d) {
+      pr.c0[d] = bc ? n[d] : c[d];
+      pr.c1[d] = bc ? c[d] : n[d];
+    }
+    float rc;
+    if (!intersection_edge2(pr.c0, pr.c1, q1, q0, rc)) continue;
+    fn(pr, rc, step * 4u + 2u * (uint32_t)far + (bc ? 1u : 0u));
   }
-  Pair pr;
-  if (k & 1) {
-    pr.p0 = pn;
-    pr.c0[0] = nx;
-    pr.c0[1] = ny;
-    pr.p1 = pc;
-    pr.c1[0] = cx;
-    pr.c1[1] = cy;
-  } else {
-    pr.p0 = pc;
-    pr.c0[0] = cx;
-    pr.c0[1] = cy;
-    pr.p1 = pn;
-    pr.c1[0] = nx;
-    pr.c1[1] = ny;
-  }
-  return pr;
 }
 
-// Walks the edge q0 -> q1; calls fn(pair, rc, seq) for every crossed
-// foreground/background pair, seq = step * 4 + pair index.  Returns false
-// when the walk hit the step cap.
+// Walks the edge q0 -> q1 with the kEdgeLanes lanes of a group, lane `sub` of
+// which takes the steps sub, sub + kEdgeLanes, ...; every lane of the group
+// calls with the same edge, and lanes of other groups may have left.  Returns
+// false when the walk hit the step cap.
 template <class Fn>
-__device__ __forceinline__ bool walk(const float q0[2], const float q1[2], uint32_t img_w,
-                                     uint32_t img_h, const uint32_t* __restrict__ pix2tri, Fn fn) {
+__device__ __forceinline__ bool walk(const float q0[2], const float q1[2], uint32_t sub,
+                                     uint32_t img_w, uint32_t img_h,
+                                     const uint32_t* __restrict__ pix2tri, Fn fn) {
   const float v01x = q1[0] - q0[0], v01y = q1[1] - q0[1];
   if (v01x == 0.f && v01y == 0.f) return true;
   const bool horizontal = fabsf(v01x) < fabsf(v01y);
@@ -133,30 +145,34 @@ __device__ __forceinline__ bool walk(const float q0[2], const float q1[2], uint3
   const float dx = q1[0] - q0[0], dy = q1[1] - q0[1];
   const float step = fmax_sel(fabsf(dx), fabsf(dy));
   const float slope_x = dx / step, slope_y = dy / step;
-  const uint32_t total = img_w * img_h;
   const float fw = (float)img_w, fh = (float)img_h;
-  for (uint32_t k = 0; k < kWalkLimit; ++k) {
-    const float fx = floorf(x), fy = floorf(y);
-    if (fx >= 0.f && fy >= 0.f && fx < fw && fy < fh) {
+  const uint32_t group = (threadIdx.x & 63u) / kEdgeLanes * kEdgeLanes;
+  for (uint32_t k0 = 0; k0 < kWalkLimit; k0 += kEdgeLanes) {
+    float mx = x, my = y;  // this lane's step, by the serial walk's additions
 #pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        const Pair pr = make_pair((uint32_t)fx, (uint32_t)fy, img_w, horizontal, c);
-        if (pr.p0 >= total || pr.p1 >= total) continue;
-        if (pix2tri[pr.p0] == DMSH_U32MAX || pix2tri[pr.p1] != DMSH_U32MAX) continue;
-        float rc;
-        if (!intersection_edge2(pr.c0, pr.c1, q1, q0, rc)) continue;
-        fn(pr, rc, k * 4u + (uint32_t)c);
+    for (uint32_t i = 1; i <= kEdgeLanes; ++i) {
+      x = x + slope_x;
+      y = y + slope_y;
+      if (i == sub) {
+        mx = x;
+        my = y;
       }
     }
+    // the walk ends after the first step that is past the edge's end, or that
+    // has left the image for good in the direction of travel
     const float eps = 1.0e-3f;
-    if (fabsf(x - q0[0]) > fabsf(q1[0] - q0[0]) + eps) return true;
-    if (fabsf(y - q0[1]) > fabsf(q1[1] - q0[1]) + eps) return true;
-    // left the image for good in the direction of travel: nothing more to do
-    if ((slope_x > 0.f && x >= fw) || (slope_x < 0.f && x < 0.f) || (slope_y > 0.f && y >= fh) ||
-        (slope_y < 0.f && y < 0.f))
-      return true;
-    x = x + slope_x;
-    y = y + slope_y;
+    const bool last = fabsf(mx - q0[0]) > fabsf(q1[0] - q0[0]) + eps ||
+                      fabsf(my - q0[1]) > fabsf(q1[1] - q0[1]) + eps ||
+                      (slope_x > 0.f && mx >= fw) || (slope_x < 0.f && mx < 0.f) ||
+                      (slope_y > 0.f && my >= fh) || (slope_y < 0.f && my < 0.f);
+    const uint32_t ends =
+        (uint32_t)(__ballot(last) >> group) & (uint32_t)((1ull << kEdgeLanes) - 1ull);
+    const bool mine = ends == 0u || sub <= (uint32_t)__builtin_ctz(ends);
+    const float fx = floorf(mx), fy = floorf(my);
+    if (mine && fx >= 0.f && fy >= 0.f && fx < fw && fy < fh)
+      cross_pixel(q0, q1, (uint32_t)fx, (uint32_t)fy, img_w, img_h, horizontal, k0 + sub, pix2tri,
+                  fn);
+    if (ends != 0u) return true;
   }
   return false;
 }
@@ -196,29 +212,31 @@ static __global__ __launch_bounds__(256) void k_zero_u64(unsigned long long* __r
 
 static __global__ __launch_bounds__(64) void k_aa_keys(EdgeArgs a,
                                                        unsigned long long* __restrict__ keys) {
-  const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t e = (blockIdx.x * blockDim.x + threadIdx.x) / kEdgeLanes;
+  const uint32_t sub = threadIdx.x % kEdgeLanes;
   if (e >= a.num_cedge) return;
   float m[16], q0[2], q1[2];
   uint32_t i0, i1;
   if (!edge_setup(a, e, m, i0, i1, q0, q1)) return;
   const unsigned long long hi = (unsigned long long)(e + 1) << 32;
-  const bool done = walk(q0, q1, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t seq) {
+  const bool done = walk(q0, q1, sub, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t seq) {
     atomicMax(keys + (rc < 0.5f ? pr.p0 : pr.p1), hi | seq);
   });
-  if (!done) raise_error(a.err, DMSH_DEVERR_WALK);
+  if (!done && sub == 0u) raise_error(a.err, DMSH_DEVERR_WALK);
 }
 
 static __global__ __launch_bounds__(64) void k_aa_write(EdgeArgs a,
                                                         const unsigned long long* __restrict__ keys,
                                                         const float* __restrict__ vin,
                                                         float* __restrict__ vout) {
-  const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t e = (blockIdx.x * blockDim.x + threadIdx.x) / kEdgeLanes;
+  const uint32_t sub = threadIdx.x % kEdgeLanes;
   if (e >= a.num_cedge) return;
   float m[16], q0[2], q1[2];
   uint32_t i0, i1;
   if (!edge_setup(a, e, m, i0, i1, q0, q1)) return;
   const unsigned long long hi = (unsigned long long)(e + 1) << 32;
-  walk(q0, q1, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t seq) {
+  walk(q0, q1, sub, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t seq) {
     const uint32_t p = rc < 0.5f ? pr.p0 : pr.p1;
     if (keys[p] != (hi | seq)) return;
     const float r0 = rc < 0.5f ? 0.5f + rc : rc - 0.5f;
@@ -241,7 +259,8 @@ __device__ __forceinline__ void proj_jacobian_xy(const float* m, const float* p,
 static __global__ __launch_bounds__(64) void k_aa_bwd(EdgeArgs a, const float* __restrict__ val,
                                                       const float* __restrict__ dldw,
                                                       float* __restrict__ dldw_vtx2xyz) {
-  const uint32_t e = blockIdx.x * blockDim.x + threadIdx.x;
+  const uint32_t e = (blockIdx.x * blockDim.x + threadIdx.x) / kEdgeLanes;
+  const uint32_t sub = threadIdx.x % kEdgeLanes;
   if (e >= a.num_cedge) return;
   float m[16], q0[2], q1[2];
   uint32_t i0, i1;
@@ -250,7 +269,7 @@ static __global__ __launch_bounds__(64) void k_aa_bwd(EdgeArgs a, const float* _
   proj_jacobian_xy(m, a.xyz + (size_t)i0 * 3, J0);
   proj_jacobian_xy(m, a.xyz + (size_t)i1 * 3, J1);
   float g0[3] = {0.f, 0.f, 0.f}, g1[3] = {0.f, 0.f, 0.f};
-  const bool done = walk(q0, q1, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t) {
+  const bool done = walk(q0, q1, sub, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t) {
     const float dv = val[pr.p0] - val[pr.p1];
     const float dldr0 = rc < 0.5f ? dldw[pr.p0] * dv : dldw[pr.p1] * dv;
     float dldq1[2], dldq0[2];
@@ -261,11 +280,18 @@ static __global__ __launch_bounds__(64) void k_aa_bwd(EdgeArgs a, const float* _
       g1[j] += J1[0][j] * dldq1[0] + J1[1][j] * dldq1[1];
     }
   });
-  if (!done) raise_error(a.err, DMSH_DEVERR_WALK);
+  if (!done && sub == 0u) raise_error(a.err, DMSH_DEVERR_WALK);
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
-    unsafeAtomicAdd(dldw_vtx2xyz + (size_t)i0 * 3 + j, g0[j]);
-    unsafeAtomicAdd(dldw_vtx2xyz + (size_t)i1 * 3 + j, g1[j]);
+#pragma unroll
+    for (uint32_t d = kEdgeLanes / 2u; d != 0u; d >>= 1) {
+      g0[j] += __shfl_xor(g0[j], (int)d, (int)kEdgeLanes);
+      g1[j] += __shfl_xor(g1[j], (int)d, (int)kEdgeLanes);
+    }
+    if (sub == 0u) {
+      unsafeAtomicAdd(dldw_vtx2xyz + (size_t)i0 * 3 + j, g0[j]);
+      unsafeAtomicAdd(dldw_vtx2xyz + (size_t)i1 * 3 + j, g1[j]);
+    }
   }
 }
 

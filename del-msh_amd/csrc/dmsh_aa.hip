@@ -13,6 +13,11 @@ struct ContourLayout {
   uint32_t* block_count;
 };
 
+// blocks of 64 threads, kEdgeLanes an edge
+inline uint32_t edge_blocks(uint32_t num_cedge) {
+  return ceil_div(num_cedge, 64u / aa::kEdgeLanes);
+}
+
 inline uint32_t contour_blocks(uint32_t num_edge) { return ceil_div(num_edge, 256); }
 
 inline bool carve_contour(Arena& a, uint32_t num_edge, ContourLayout& L) {
@@ -95,9 +100,9 @@ int dmsh_antialias_fwd(void* stream, uint32_t num_cedge, const uint32_t* cedge2v
   if (st != DMSH_OK) return st;
   aa::EdgeArgs ea{cedge2vtx, num_cedge, vtx2xyz, num_vtx, transform_world2pix,
                   img_w, img_h, pix2tri, err};
-  launch("k_aa_keys", aa::k_aa_keys, dim3(ceil_div(num_cedge, 64)), dim3(64), 0, s, ea, keys);
+  launch("k_aa_keys", aa::k_aa_keys, dim3(edge_blocks(num_cedge)), dim3(64), 0, s, ea, keys);
   if ((st = launch_status()) != DMSH_OK) return st;
-  launch("k_aa_write", aa::k_aa_write, dim3(ceil_div(num_cedge, 64)), dim3(64), 0, s, ea, keys,
+  launch("k_aa_write", aa::k_aa_write, dim3(edge_blocks(num_cedge)), dim3(64), 0, s, ea, keys,
                      pix2vin, pix2vout);
   return launch_status();
 }
@@ -116,7 +121,7 @@ int dmsh_antialias_bwd(void* stream, uint32_t num_cedge, const uint32_t* cedge2v
   if (!err) return DMSH_ERR_HIP;
   aa::EdgeArgs ea{cedge2vtx, num_cedge, vtx2xyz, num_vtx, transform_world2pix,
                   img_w, img_h, pix2tri, err};
-  launch("k_aa_bwd", aa::k_aa_bwd, dim3(ceil_div(num_cedge, 64)), dim3(64), 0, as_stream(stream),
+  launch("k_aa_bwd", aa::k_aa_bwd, dim3(edge_blocks(num_cedge)), dim3(64), 0, as_stream(stream),
                      ea, pix2val, dldw_pix2val, dldw_vtx2xyz);
   return launch_status();
 }
