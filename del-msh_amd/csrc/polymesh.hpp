@@ -5,10 +5,11 @@
 // Point location follows del-msh-cpu/src/polyhedron_mesh.rs:470-575: a
 // depth-first walk of the BVH, left child first, into boxes that contain the
 // point (min <= q <= max on every axis), stopping at the first element that
-// contains it.  The walk needs no stack: it climbs through the parent links
-// of the reference layout (after a left child comes the right one, after a
-// right child the parent's sibling), so it visits the nodes of the
-// recursion in the recursion's order at any tree depth.
+// contains it.  The right children still to visit wait on a stack of
+// kSearchFrames LDS words a lane; a walk that needs more starts again without a
+// stack (search_climb), by climbing the parent links of the reference layout
+// (after a left child comes the right one, after a right child the parent's
+// sibling).  Both visit the nodes of the recursion in the recursion's order.
 //
 // Parametric coordinates of the point in an element (del-geo's
 // tet/pyramid/prism/hex parametric_coord_for_origin is not vendored; this is
@@ -278,79 +279,71 @@ static __global__ __launch_bounds__(256) void k_query_codes(uint32_t num_wtx,
   idx[w] = w;
 }
 
-// one thread per query point; with `order`, thread i takes query order[i]
-static __global__ __launch_bounds__(256) void k_search_elem_contain_points(
-    MeshView m, const uint32_t* __restrict__ bvhnodes, const float* __restrict__ aabb,
-    uint32_t num_wtx, const float* __restrict__ wtx2xyz, uint32_t* __restrict__ wtx2elem,
-    float* __restrict__ wtx2param, const uint32_t* __restrict__ order,
-    uint32_t* __restrict__ err) {
-  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= num_wtx) return;
-  const uint32_t w = order ? order[i] : i;
-  if (w >= num_wtx) {
+__device__ __forceinline__ bool box_holds(const float* __restrict__ b, const V3& q) {
+  const float2* p = reinterpret_cast<const float2*>(b);
+  const float2 u = p[0], v = p[1], w = p[2];  // lo.x lo.y | lo.z hi.x | hi.y hi.z
+  return u.x <= q.x && q.x <= v.y && u.y <= q.y && q.y <= w.x && v.x <= q.z && q.z <= w.y;
+}
+
+enum : int { kElemOut = 0, kElemIn = 1, kElemBad = 2 };
+
+// Whether element e holds the point, and its parametric coordinates there.
+__device__ __forceinline__ int elem_test(const MeshView& m, uint32_t e, const V3& q, float c[3],
+                                         uint32_t* __restrict__ err) {
+  if (e >= m.num_elem) {
     raise_error(err, DMSH_DEVERR_INDEX);
-    return;
+    return kElemBad;
   }
-  const V3 q{wtx2xyz[(size_t)w * 3], wtx2xyz[(size_t)w * 3 + 1], wtx2xyz[(size_t)w * 3 + 2]};
-  uint32_t found = DMSH_U32MAX;
-  float pco[3] = {0.f, 0.f, 0.f};
-  const uint32_t num_node = m.num_elem ? 2 * m.num_elem - 1 : 0;
+  const uint32_t i0 = m.elem2idx[e], i1 = m.elem2idx[e + 1];
+  const uint32_t n = i1 - i0;
+  if (i1 < i0 || i1 > m.num_idx) {
+    raise_error(err, DMSH_DEVERR_INDEX);
+    return kElemBad;
+  }
+  if (n != 4 && n != 5 && n != 6 && n != 8) return kElemOut;
+  // all eight slots by constant index (registers, not scratch)
+  V3 p[8];
+  bool ok = true;
+#pragma unroll
+  for (uint32_t k = 0; k < 8; ++k) {
+    p[k] = V3{0.f, 0.f, 0.f};
+    if (k < n) {
+      const uint32_t v = m.idx2vtx[i0 + k];
+      if (v >= m.num_vtx) {
+        ok = false;
+      } else {
+        const float* x = m.xyz + (size_t)v * 3;
+        p[k] = V3{x[0] - q.x, x[1] - q.y, x[2] - q.z};
+      }
+    }
+  }
+  if (!ok) {
+    raise_error(err, DMSH_DEVERR_INDEX);
+    return kElemBad;
+  }
+  return param_coord(p, n, c) ? kElemIn : kElemOut;
+}
+
+// The walk without a stack.  Returns the element or DMSH_U32MAX.
+__device__ __forceinline__ uint32_t search_climb(const MeshView& m,
+                                                 const uint32_t* __restrict__ bvhnodes,
+                                                 const float* __restrict__ aabb, const V3& q,
+                                                 float pco[3], uint32_t* __restrict__ err) {
+  const uint32_t num_node = 2 * m.num_elem - 1;
   uint32_t node = 0;
-  bool down = num_node > 0;
+  bool down = true;
   const uint64_t max_steps = 2ull * num_node + 2;
-  for (uint64_t steps = 0; num_node > 0; ++steps) {
+  for (uint64_t steps = 0;; ++steps) {
     if (steps > max_steps || node >= num_node) {
       raise_error(err, DMSH_DEVERR_INDEX);
-      break;
+      return DMSH_U32MAX;
     }
     const uint32_t* row = bvhnodes + (size_t)node * 3;
     if (down) {
-      const float* b = aabb + (size_t)node * 6;
-      const bool in = b[0] <= q.x && q.x <= b[3] && b[1] <= q.y && q.y <= b[4] && b[2] <= q.z &&
-                      q.z <= b[5];
-      if (in) {
+      if (box_holds(aabb + (size_t)node * 6, q)) {
         if (row[2] == DMSH_U32MAX) {
-          const uint32_t e = row[1];
-          if (e >= m.num_elem) {
-            raise_error(err, DMSH_DEVERR_INDEX);
-            break;
-          }
-          const uint32_t i0 = m.elem2idx[e], i1 = m.elem2idx[e + 1];
-          const uint32_t n = i1 - i0;
-          if (i1 < i0 || i1 > m.num_idx) {
-            raise_error(err, DMSH_DEVERR_INDEX);
-            break;
-          }
-          if (n == 4 || n == 5 || n == 6 || n == 8) {
-            // all eight slots by constant index (registers, not scratch)
-            V3 p[8];
-            bool ok = true;
-#pragma unroll
-            for (uint32_t k = 0; k < 8; ++k) {
-              p[k] = V3{0.f, 0.f, 0.f};
-              if (k < n) {
-                const uint32_t v = m.idx2vtx[i0 + k];
-                if (v >= m.num_vtx) {
-                  ok = false;
-                } else {
-                  const float* x = m.xyz + (size_t)v * 3;
-                  p[k] = V3{x[0] - q.x, x[1] - q.y, x[2] - q.z};
-                }
-              }
-            }
-            if (!ok) {
-              raise_error(err, DMSH_DEVERR_INDEX);
-              break;
-            }
-            float c[3];
-            if (param_coord(p, n, c)) {
-              found = e;
-              pco[0] = c[0];
-              pco[1] = c[1];
-              pco[2] = c[2];
-              break;
-            }
-          }
+          const int st = elem_test(m, row[1], q, pco, err);
+          if (st != kElemOut) return st == kElemIn ? row[1] : DMSH_U32MAX;
           down = false;  // leaf done: climb
           continue;
         }
@@ -362,10 +355,10 @@ static __global__ __launch_bounds__(256) void k_search_elem_contain_points(
     }
     // climbing from `node`
     const uint32_t par = row[0];
-    if (par == DMSH_U32MAX) break;  // back at the root: not found
+    if (par == DMSH_U32MAX) return DMSH_U32MAX;  // back at the root: not found
     if (par >= num_node) {
       raise_error(err, DMSH_DEVERR_INDEX);
-      break;
+      return DMSH_U32MAX;
     }
     const uint32_t* prow = bvhnodes + (size_t)par * 3;
     if (prow[1] == node) {
@@ -375,6 +368,96 @@ static __global__ __launch_bounds__(256) void k_search_elem_contain_points(
       node = par;
     }
   }
+}
+
+// One thread per query point; with `order`, thread i takes query order[i].
+// A wave's lanes first walk each to its next leaf whose box holds the point,
+// then test their elements together: the Newton solves are most of the work,
+// and in a loop that did whatever each lane was at they ran for a few lanes at
+// a time.  A node's children are read together, rows and boxes, so a level
+// costs one round trip.  2^20 points in 66 000 mixed elements: 1467 -> 844 us.
+constexpr int kSearchFrames = 32;
+constexpr int kSearchThreads = 256;
+
+static __global__ __launch_bounds__(kSearchThreads) void k_search_elem_contain_points(
+    MeshView m, const uint32_t* __restrict__ bvhnodes, const float* __restrict__ aabb,
+    uint32_t num_wtx, const float* __restrict__ wtx2xyz, uint32_t* __restrict__ wtx2elem,
+    float* __restrict__ wtx2param, const uint32_t* __restrict__ order,
+    uint32_t* __restrict__ err) {
+  __shared__ uint32_t s_frame[kSearchFrames][kSearchThreads];
+  const uint32_t i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= num_wtx) return;
+  const uint32_t w = order ? order[i] : i;
+  if (w >= num_wtx) {
+    raise_error(err, DMSH_DEVERR_INDEX);
+    return;
+  }
+  const V3 q{wtx2xyz[(size_t)w * 3], wtx2xyz[(size_t)w * 3 + 1], wtx2xyz[(size_t)w * 3 + 2]};
+  uint32_t found = DMSH_U32MAX;
+  float pco[3] = {0.f, 0.f, 0.f};
+  const uint32_t num_node = m.num_elem ? 2 * m.num_elem - 1 : 0;
+  // The node at hand holds the point: its children (c0, c1), or its element
+  // (c0) and DMSH_U32MAX.
+  uint32_t c0 = 0u, c1 = 0u;
+  int sp = 0;
+  bool on = num_node > 0 && box_holds(aabb, q), climb = false;
+  if (on) {
+    c0 = bvhnodes[1];
+    c1 = bvhnodes[2];
+  }
+  uint32_t steps = 0;  // a walk visits a node once; the cap ends one in a broken tree
+  while (on) {
+    // to the next leaf that holds the point
+    while (on && c1 != DMSH_U32MAX) {
+      if (c0 >= num_node || c1 >= num_node || ++steps > num_node) {
+        raise_error(err, DMSH_DEVERR_INDEX);
+        on = false;
+        break;
+      }
+      const uint32_t *r0 = bvhnodes + (size_t)c0 * 3, *r1 = bvhnodes + (size_t)c1 * 3;
+      const uint32_t a0 = r0[1], a1 = r0[2], b0 = r1[1], b1 = r1[2];
+      const bool in0 = box_holds(aabb + (size_t)c0 * 6, q);
+      const bool in1 = box_holds(aabb + (size_t)c1 * 6, q);
+      if (in0 && in1) {
+        if (sp == kSearchFrames) {
+          on = false;
+          climb = true;
+          break;
+        }
+        s_frame[sp++][threadIdx.x] = c1;
+      }
+      if (in0) {
+        c0 = a0;
+        c1 = a1;
+      } else if (in1) {
+        c0 = b0;
+        c1 = b1;
+      } else if (sp > 0) {
+        const uint32_t* row = bvhnodes + (size_t)s_frame[--sp][threadIdx.x] * 3;
+        c0 = row[1];
+        c1 = row[2];
+      } else {
+        on = false;
+      }
+    }
+    if (!on) break;
+    float c[3];
+    const int st = elem_test(m, c0, q, c, err);
+    if (st == kElemIn) {
+      found = c0;
+      pco[0] = c[0];
+      pco[1] = c[1];
+      pco[2] = c[2];
+    }
+    on = st == kElemOut && sp > 0;
+    if (on) {
+      const uint32_t* row = bvhnodes + (size_t)s_frame[--sp][threadIdx.x] * 3;
+      c0 = row[1];
+      c1 = row[2];
+    }
+  }
+  if (climb) found = search_climb(m, bvhnodes, aabb, q, pco, err);
+  if (found == DMSH_U32MAX) pco[0] = pco[1] = pco[2] = 0.f;
   wtx2elem[w] = found;
   wtx2param[(size_t)w * 3] = pco[0];
   wtx2param[(size_t)w * 3 + 1] = pco[1];
@@ -390,17 +473,17 @@ static __global__ __launch_bounds__(256) void k_interpolate_at_points(
   const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
   if (w >= num_wtx) return;
   float* o = out + (size_t)w * num_vdim;
-  for (uint32_t d = 0; d < num_vdim; ++d) o[d] = 0.f;
   const uint32_t e = wtx2elem[w];
-  if (e == DMSH_U32MAX) return;
-  if (e >= m.num_elem) {
-    raise_error(err, DMSH_DEVERR_INDEX);
-    return;
-  }
-  const uint32_t i0 = m.elem2idx[e], i1 = m.elem2idx[e + 1];
-  if (i1 < i0 || i1 > m.num_idx) {
-    raise_error(err, DMSH_DEVERR_INDEX);
-    return;
+  uint32_t i0 = 0u, i1 = 0u;
+  if (e != DMSH_U32MAX) {
+    if (e < m.num_elem) {
+      i0 = m.elem2idx[e];
+      i1 = m.elem2idx[e + 1];
+    }
+    if (e >= m.num_elem || i1 < i0 || i1 > m.num_idx) {
+      raise_error(err, DMSH_DEVERR_INDEX);
+      i0 = i1 = 0u;
+    }
   }
   const uint32_t n = i1 - i0;
   const float r = wtx2param[(size_t)w * 3], s = wtx2param[(size_t)w * 3 + 1],
@@ -416,16 +499,44 @@ static __global__ __launch_bounds__(256) void k_interpolate_at_points(
     case 5: shape_pyramid(r, s, t, sf, nullptr, nullptr, nullptr); break;
     case 6: shape_prism(r, s, t, sf, nullptr, nullptr, nullptr); break;
     case 8: shape_hex(r, s, t, sf, nullptr, nullptr, nullptr); break;
-    default: return;
+    default:
+      for (uint32_t d = 0; d < num_vdim; ++d) o[d] = 0.f;
+      return;
   }
-  for (uint32_t k = 0; k < n; ++k) {
-    const uint32_t v = m.idx2vtx[i0 + k];
-    if (v >= m.num_vtx) {
-      raise_error(err, DMSH_DEVERR_INDEX);
-      continue;
+  uint32_t v[8];
+#pragma unroll
+  for (uint32_t k = 0; k < 8; ++k) {
+    v[k] = DMSH_U32MAX;  // no term
+    if (k < n) {
+      v[k] = m.idx2vtx[i0 + k];
+      if (v[k] >= m.num_vtx) {
+        raise_error(err, DMSH_DEVERR_INDEX);
+        v[k] = DMSH_U32MAX;
+      }
     }
-    const float* val = vtx2val + (size_t)v * num_vdim;
-    for (uint32_t d = 0; d < num_vdim; ++d) o[d] += sf[k] * val[d];
+  }
+  // two values at a time: the reads of all nodes go out together, and the sums
+  // (in node order) stay in registers
+  for (uint32_t d = 0; d < num_vdim; d += 2) {
+    const bool two = d + 1 < num_vdim;
+    float x[8][2];
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
+      x[k][0] = x[k][1] = 0.f;
+      if (v[k] == DMSH_U32MAX) continue;
+      const float* val = vtx2val + (size_t)v[k] * num_vdim + d;
+      x[k][0] = val[0];
+      if (two) x[k][1] = val[1];
+    }
+    float acc[2] = {0.f, 0.f};
+#pragma unroll
+    for (uint32_t k = 0; k < 8; ++k) {
+      if (v[k] == DMSH_U32MAX) continue;
+      acc[0] += sf[k] * x[k][0];
+      acc[1] += sf[k] * x[k][1];
+    }
+    o[d] = acc[0];
+    if (two) o[d + 1] = acc[1];
   }
 }
 
