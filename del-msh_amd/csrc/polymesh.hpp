@@ -259,13 +259,14 @@ struct MeshView {
   const float* xyz;
 };
 
-// 30-bit Morton code of each query point in the unit-cube fit of the root
-// box (aabb row 0), and the identity permutation: sorting by these codes puts
+// 30-bit Morton code, less its lowest `shift` bits, of each query point in the
+// unit-cube fit of the root box (aabb row 0), and the identity permutation: sorting by these codes puts
 // nearby queries in one wave, so its lanes walk the same branches and test
 // the same elements.  Only the processing order changes, not any result.
 static __global__ __launch_bounds__(256) void k_query_codes(uint32_t num_wtx,
                                                             const float* __restrict__ wtx2xyz,
                                                             const float* __restrict__ aabb,
+                                                            uint32_t shift,
                                                             uint32_t* __restrict__ keys,
                                                             uint32_t* __restrict__ idx) {
   const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
@@ -275,7 +276,8 @@ static __global__ __launch_bounds__(256) void k_query_codes(uint32_t num_wtx,
   float T[16] = {s, 0.f, 0.f, 0.f, 0.f, s, 0.f, 0.f, 0.f, 0.f, s, 0.f,
                  -aabb[0] * s, -aabb[1] * s, -aabb[2] * s, 1.f};
   keys[w] = morton3_transformed<uint32_t>(T, wtx2xyz[(size_t)w * 3], wtx2xyz[(size_t)w * 3 + 1],
-                                          wtx2xyz[(size_t)w * 3 + 2]);
+                                          wtx2xyz[(size_t)w * 3 + 2]) >>
+            shift;
   idx[w] = w;
 }
 
