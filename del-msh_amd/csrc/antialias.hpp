@@ -210,19 +210,42 @@ static __global__ __launch_bounds__(256) void k_zero_u64(unsigned long long* __r
     p[i] = 0ull;
 }
 
-static __global__ __launch_bounds__(64) void k_aa_keys(EdgeArgs a,
-                                                       unsigned long long* __restrict__ keys) {
-  const uint32_t e = (blockIdx.x * blockDim.x + threadIdx.x) / kEdgeLanes;
-  const uint32_t sub = threadIdx.x % kEdgeLanes;
-  if (e >= a.num_cedge) return;
+// The writes of contour edge e, by the lanes of its group, as keys (edge, then
+// step and pair) into the pixels' maxima.
+__device__ __forceinline__ void keys_of_edge(const EdgeArgs& a, uint32_t e, uint32_t sub,
+                                             unsigned long long* __restrict__ keys) {
+  const unsigned long long hi = (unsigned long long)(e + 1) << 32;
   float m[16], q0[2], q1[2];
   uint32_t i0, i1;
   if (!edge_setup(a, e, m, i0, i1, q0, q1)) return;
-  const unsigned long long hi = (unsigned long long)(e + 1) << 32;
   const bool done = walk(q0, q1, sub, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t seq) {
     atomicMax(keys + (rc < 0.5f ? pr.p0 : pr.p1), hi | seq);
   });
   if (!done && sub == 0u) raise_error(a.err, DMSH_DEVERR_WALK);
+}
+
+// The values of its writes that hold their pixel's key.
+__device__ __forceinline__ void values_of_edge(const EdgeArgs& a, uint32_t e, uint32_t sub,
+                                               const unsigned long long* __restrict__ keys,
+                                               const float* __restrict__ vin,
+                                               float* __restrict__ vout) {
+  const unsigned long long hi = (unsigned long long)(e + 1) << 32;
+  float m[16], q0[2], q1[2];
+  uint32_t i0, i1;
+  if (!edge_setup(a, e, m, i0, i1, q0, q1)) return;
+  walk(q0, q1, sub, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t seq) {
+    const uint32_t p = rc < 0.5f ? pr.p0 : pr.p1;
+    if (keys[p] != (hi | seq)) return;
+    const float r0 = rc < 0.5f ? 0.5f + rc : rc - 0.5f;
+    vout[p] = r0 * vin[pr.p0] + (1.f - r0) * vin[pr.p1];
+  });
+}
+
+static __global__ __launch_bounds__(64) void k_aa_keys(EdgeArgs a,
+                                                       unsigned long long* __restrict__ keys) {
+  const uint32_t e = (blockIdx.x * blockDim.x + threadIdx.x) / kEdgeLanes;
+  if (e < a.num_cedge)
+    keys_of_edge(a, e, threadIdx.x % kEdgeLanes, keys);
 }
 
 static __global__ __launch_bounds__(64) void k_aa_write(EdgeArgs a,
@@ -230,18 +253,8 @@ static __global__ __launch_bounds__(64) void k_aa_write(EdgeArgs a,
                                                         const float* __restrict__ vin,
                                                         float* __restrict__ vout) {
   const uint32_t e = (blockIdx.x * blockDim.x + threadIdx.x) / kEdgeLanes;
-  const uint32_t sub = threadIdx.x % kEdgeLanes;
-  if (e >= a.num_cedge) return;
-  float m[16], q0[2], q1[2];
-  uint32_t i0, i1;
-  if (!edge_setup(a, e, m, i0, i1, q0, q1)) return;
-  const unsigned long long hi = (unsigned long long)(e + 1) << 32;
-  walk(q0, q1, sub, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t seq) {
-    const uint32_t p = rc < 0.5f ? pr.p0 : pr.p1;
-    if (keys[p] != (hi | seq)) return;
-    const float r0 = rc < 0.5f ? 0.5f + rc : rc - 0.5f;
-    vout[p] = r0 * vin[pr.p0] + (1.f - r0) * vin[pr.p1];
-  });
+  if (e < a.num_cedge)
+    values_of_edge(a, e, threadIdx.x % kEdgeLanes, keys, vin, vout);
 }
 
 __device__ __forceinline__ void proj_jacobian_xy(const float* m, const float* p, float J[2][3]) {
@@ -256,12 +269,11 @@ __device__ __forceinline__ void proj_jacobian_xy(const float* m, const float* p,
   }
 }
 
-static __global__ __launch_bounds__(64) void k_aa_bwd(EdgeArgs a, const float* __restrict__ val,
-                                                      const float* __restrict__ dldw,
-                                                      float* __restrict__ dldw_vtx2xyz) {
-  const uint32_t e = (blockIdx.x * blockDim.x + threadIdx.x) / kEdgeLanes;
-  const uint32_t sub = threadIdx.x % kEdgeLanes;
-  if (e >= a.num_cedge) return;
+// dL/d(vertices) of contour edge e, by the lanes of its group.
+__device__ __forceinline__ void bwd_of_edge(const EdgeArgs& a, uint32_t e, uint32_t sub,
+                                            const float* __restrict__ val,
+                                            const float* __restrict__ dldw,
+                                            float* __restrict__ dldw_vtx2xyz) {
   float m[16], q0[2], q1[2];
   uint32_t i0, i1;
   if (!edge_setup(a, e, m, i0, i1, q0, q1)) return;
@@ -293,6 +305,13 @@ static __global__ __launch_bounds__(64) void k_aa_bwd(EdgeArgs a, const float* _
       unsafeAtomicAdd(dldw_vtx2xyz + (size_t)i1 * 3 + j, g1[j]);
     }
   }
+}
+
+static __global__ __launch_bounds__(64) void k_aa_bwd(EdgeArgs a, const float* __restrict__ val,
+                                                      const float* __restrict__ dldw,
+                                                      float* __restrict__ dldw_vtx2xyz) {
+  const uint32_t e = (blockIdx.x * blockDim.x + threadIdx.x) / kEdgeLanes;
+  if (e < a.num_cedge) bwd_of_edge(a, e, threadIdx.x % kEdgeLanes, val, dldw, dldw_vtx2xyz);
 }
 
 // ---------------------------------------------------------------------------
@@ -372,10 +391,10 @@ static __global__ __launch_bounds__(256) void k_contour_count(ContourArgs a,
   if (threadIdx.x == 0) block_count[blockIdx.x] = s_w[0] + s_w[1] + s_w[2] + s_w[3];
 }
 
-// pass 2: one block turns the block counts into exclusive offsets (+ total)
-static __global__ __launch_bounds__(1024) void k_scan_counts(uint32_t* __restrict__ block_count,
-                                                             uint32_t num_blocks,
-                                                             uint32_t* __restrict__ total) {
+// pass 2: one block of 1024 threads turns the block counts into exclusive
+// offsets (+ total)
+__device__ __forceinline__ void scan_counts(uint32_t* __restrict__ block_count,
+                                            uint32_t num_blocks, uint32_t* __restrict__ total) {
   __shared__ uint32_t s_w[16];
   __shared__ uint32_t s_carry;
   if (threadIdx.x == 0) s_carry = 0;
@@ -400,6 +419,12 @@ static __global__ __launch_bounds__(1024) void k_scan_counts(uint32_t* __restric
     __syncthreads();
   }
   if (threadIdx.x == 0) *total = s_carry;
+}
+
+static __global__ __launch_bounds__(1024) void k_scan_counts(uint32_t* __restrict__ block_count,
+                                                             uint32_t num_blocks,
+                                                             uint32_t* __restrict__ total) {
+  scan_counts(block_count, num_blocks, total);
 }
 
 // pass 3: scatter the selected vertex pairs in edge order

@@ -2,6 +2,7 @@
 #include <algorithm>
 
 #include "antialias.hpp"
+#include "batch_aa.hpp"
 
 using namespace dmsh;
 
@@ -24,6 +25,34 @@ inline bool carve_contour(Arena& a, uint32_t num_edge, ContourLayout& L) {
   L.n2w = a.take<float>(17);
   L.flags = a.take<uint32_t>(num_edge ? num_edge : 1);
   L.block_count = a.take<uint32_t>(num_edge ? contour_blocks(num_edge) : 1);
+  return a.ok();
+}
+
+struct BatchContourLayout {
+  float* n2w;
+  uint64_t* wave_mask;
+  uint32_t* block_count;
+  uint32_t* bad;
+};
+
+inline bool carve_batch_contour(Arena& a, uint32_t num_mesh, uint32_t total_edge,
+                                BatchContourLayout& L) {
+  const uint32_t nb = contour_blocks(total_edge);
+  L.n2w = a.take<float>((size_t)num_mesh * 17);
+  L.wave_mask = a.take<uint64_t>((size_t)nb * 4 + 1);
+  L.block_count = a.take<uint32_t>((size_t)nb + 1);
+  L.bad = a.take<uint32_t>(1);
+  return a.ok();
+}
+
+struct BatchAaLayout {
+  unsigned long long* keys;
+  uint32_t* bad;
+};
+
+inline bool carve_batch_aa(Arena& a, uint32_t total_pix, BatchAaLayout& L) {
+  L.keys = a.take<unsigned long long>((size_t)total_pix + 1);
+  L.bad = a.take<uint32_t>(1);
   return a.ok();
 }
 
@@ -123,6 +152,125 @@ int dmsh_antialias_bwd(void* stream, uint32_t num_cedge, const uint32_t* cedge2v
                   img_w, img_h, pix2tri, err};
   launch("k_aa_bwd", aa::k_aa_bwd, dim3(edge_blocks(num_cedge)), dim3(64), 0, as_stream(stream),
                      ea, pix2val, dldw_pix2val, dldw_vtx2xyz);
+  return launch_status();
+}
+
+size_t dmsh_batch_contour_workspace_bytes(uint32_t num_mesh, uint32_t total_edge) {
+  Arena a{nullptr, ~(size_t)0, 0};
+  BatchContourLayout L;
+  carve_batch_contour(a, num_mesh, total_edge, L);
+  return a.off + 256;
+}
+
+int dmsh_batch_contour(void* stream, uint32_t num_mesh, uint32_t total_tri, uint32_t total_vtx,
+                       uint32_t total_edge, const uint32_t* mesh2tri, const uint32_t* mesh2vtx,
+                       const uint32_t* tri2vtx, const float* vtx2xyz,
+                       const float* transforms_world2ndc, const uint32_t* mesh2edge,
+                       const uint32_t* edge2vtx, const uint32_t* edge2tri, uint32_t* mesh2cedge,
+                       uint32_t* cedge2vtx, void* ws, size_t ws_bytes) {
+  if (num_mesh == 0 || !mesh2tri || !mesh2vtx || !mesh2edge || !transforms_world2ndc || !mesh2cedge)
+    return DMSH_ERR_INVALID;
+  if (total_edge > 0 && (!tri2vtx || !vtx2xyz || !edge2vtx || !edge2tri || !cedge2vtx))
+    return DMSH_ERR_INVALID;
+  if (!ws || ws_bytes < dmsh_batch_contour_workspace_bytes(num_mesh, total_edge))
+    return DMSH_ERR_WORKSPACE;
+  Arena ar{static_cast<char*>(ws), ws_bytes, 0};
+  BatchContourLayout L;
+  if (!carve_batch_contour(ar, num_mesh, total_edge, L)) return DMSH_ERR_WORKSPACE;
+  uint32_t* err = device_error_word();
+  if (!err) return DMSH_ERR_HIP;
+  hipStream_t s = as_stream(stream);
+  const uint32_t nb = contour_blocks(total_edge);
+  const baa::ContourBatch b{num_mesh,  mesh2tri, mesh2vtx, tri2vtx,
+                            vtx2xyz,   total_edge, mesh2edge, edge2vtx,
+                            edge2tri,  transforms_world2ndc, L.n2w, L.bad, err};
+  launch("k_batch_contour_init", baa::k_batch_contour_init, dim3(1), dim3(1024), 0, s, b,
+         total_tri, total_vtx);
+  int st = launch_status();
+  if (st != DMSH_OK) return st;
+  if (nb) {
+    launch("k_batch_contour_count", baa::k_batch_contour_count, dim3(nb), dim3(256), 0, s, b,
+           L.wave_mask, L.block_count);
+    if ((st = launch_status()) != DMSH_OK) return st;
+  }
+  // also writes the total when there is no edge (0)
+  launch("k_scan_counts", aa::k_scan_counts, dim3(1), dim3(1024), 0, s, L.block_count, nb,
+         mesh2cedge + num_mesh);
+  if ((st = launch_status()) != DMSH_OK) return st;
+  launch("k_batch_contour_scatter", baa::k_batch_contour_scatter,
+         dim3(nb + ceil_div(num_mesh, 256)), dim3(256), 0, s, b, nb, L.wave_mask, L.block_count,
+         mesh2cedge, cedge2vtx);
+  return launch_status();
+}
+
+size_t dmsh_batch_antialias_workspace_bytes(uint32_t total_pix) {
+  Arena a{nullptr, ~(size_t)0, 0};
+  BatchAaLayout L;
+  carve_batch_aa(a, total_pix, L);
+  return a.off + 256;
+}
+
+int dmsh_batch_antialias_fwd(void* stream, uint32_t num_mesh, uint32_t total_vtx,
+                             uint32_t total_pix, uint32_t num_cedge, const uint32_t* mesh2vtx,
+                             const float* vtx2xyz, const uint32_t* mesh2pix,
+                             const uint32_t* mesh2width, const uint32_t* mesh2cedge,
+                             const uint32_t* cedge2vtx, const float* transforms_world2pix,
+                             const uint32_t* pix2tri, const float* pix2vin, float* pix2vout,
+                             void* ws, size_t ws_bytes) {
+  if (total_pix == 0 || num_cedge == 0) return DMSH_OK;
+  if (num_mesh == 0 || num_cedge == DMSH_U32MAX) return DMSH_ERR_INVALID;
+  if (!mesh2vtx || !vtx2xyz || !mesh2pix || !mesh2width || !mesh2cedge || !cedge2vtx ||
+      !transforms_world2pix || !pix2tri || !pix2vin || !pix2vout)
+    return DMSH_ERR_INVALID;
+  if (!ws || ws_bytes < dmsh_batch_antialias_workspace_bytes(total_pix)) return DMSH_ERR_WORKSPACE;
+  Arena ar{static_cast<char*>(ws), ws_bytes, 0};
+  BatchAaLayout L;
+  if (!carve_batch_aa(ar, total_pix, L)) return DMSH_ERR_WORKSPACE;
+  uint32_t* err = device_error_word();
+  if (!err) return DMSH_ERR_HIP;
+  hipStream_t s = as_stream(stream);
+  const baa::Images b{num_mesh,   mesh2vtx,  vtx2xyz,              mesh2pix, mesh2width, num_cedge,
+                      mesh2cedge, cedge2vtx, transforms_world2pix, pix2tri,  L.bad,      err};
+  launch("k_batch_aa_init", baa::k_batch_aa_init,
+         dim3(std::min<uint32_t>(ceil_div(total_pix, 256), 4096) + 1), dim3(256), 0, s, b,
+         total_vtx, total_pix, L.keys, (uint64_t)total_pix);
+  int st = launch_status();
+  if (st != DMSH_OK) return st;
+  launch("k_batch_aa_keys", baa::k_batch_aa_keys, dim3(edge_blocks(num_cedge)), dim3(64), 0, s, b,
+         L.keys);
+  if ((st = launch_status()) != DMSH_OK) return st;
+  launch("k_batch_aa_write", baa::k_batch_aa_write, dim3(edge_blocks(num_cedge)), dim3(64), 0, s,
+         b, L.keys, pix2vin, pix2vout);
+  return launch_status();
+}
+
+int dmsh_batch_antialias_bwd(void* stream, uint32_t num_mesh, uint32_t total_vtx,
+                             uint32_t total_pix, uint32_t num_cedge, const uint32_t* mesh2vtx,
+                             const float* vtx2xyz, float* dldw_vtx2xyz, const uint32_t* mesh2pix,
+                             const uint32_t* mesh2width, const uint32_t* mesh2cedge,
+                             const uint32_t* cedge2vtx, const float* transforms_world2pix,
+                             const float* pix2val, const float* dldw_pix2val,
+                             const uint32_t* pix2tri, void* ws, size_t ws_bytes) {
+  if (total_pix == 0 || num_cedge == 0) return DMSH_OK;
+  if (num_mesh == 0 || num_cedge == DMSH_U32MAX) return DMSH_ERR_INVALID;
+  if (!mesh2vtx || !vtx2xyz || !dldw_vtx2xyz || !mesh2pix || !mesh2width || !mesh2cedge ||
+      !cedge2vtx || !transforms_world2pix || !pix2val || !dldw_pix2val || !pix2tri)
+    return DMSH_ERR_INVALID;
+  if (!ws || ws_bytes < dmsh_batch_antialias_workspace_bytes(0)) return DMSH_ERR_WORKSPACE;
+  Arena ar{static_cast<char*>(ws), ws_bytes, 0};
+  BatchAaLayout L;
+  if (!carve_batch_aa(ar, 0, L)) return DMSH_ERR_WORKSPACE;
+  uint32_t* err = device_error_word();
+  if (!err) return DMSH_ERR_HIP;
+  hipStream_t s = as_stream(stream);
+  const baa::Images b{num_mesh,   mesh2vtx,  vtx2xyz,              mesh2pix, mesh2width, num_cedge,
+                      mesh2cedge, cedge2vtx, transforms_world2pix, pix2tri,  L.bad,      err};
+  launch("k_batch_aa_init", baa::k_batch_aa_init, dim3(1), dim3(256), 0, s, b, total_vtx,
+         total_pix, L.keys, (uint64_t)0);
+  int st = launch_status();
+  if (st != DMSH_OK) return st;
+  launch("k_batch_aa_bwd", baa::k_batch_aa_bwd, dim3(edge_blocks(num_cedge)), dim3(64), 0, s, b,
+         pix2val, dldw_pix2val, dldw_vtx2xyz);
   return launch_status();
 }
 

@@ -14,6 +14,7 @@ import numpy as np
 import torch
 
 from .. import _lib
+from ..util_torch import assert_shape_dtype_device
 
 
 def _host_u32(a) -> np.ndarray:
@@ -381,15 +382,29 @@ def autotune(p: Pipeline, reps: int = 2, stacks=(12, 16, 20, 24, 32), wgs_per_cu
 # ---------------------------------------------------------------------------
 # differentiable anti-aliased silhouettes of a batch
 # ---------------------------------------------------------------------------
+class _ContourEdges(list):
+    """Each mesh's contour edges, as slices of the batch's compacted buffer
+    (mesh m's are rows mesh2cedge[m] .. mesh2cedge[m+1])."""
+
+    def __init__(self, cedge2vtx: torch.Tensor, mesh2cedge: torch.Tensor, offsets):
+        super().__init__(cedge2vtx[a:b] for a, b in zip(offsets, offsets[1:]))
+        self.own = tuple(self)
+        self.batch = (cedge2vtx, mesh2cedge, offsets[-1])
+
+    def intact(self) -> bool:
+        """Still the slices (a caller may put other edges in their place)."""
+        return len(self) == len(self.own) and all(a is b for a, b in zip(self, self.own))
+
+
 class SilhouetteBatch:
     """Anti-aliased silhouette images of a CSR mesh batch, one image per mesh
     (occupancy of the ray-cast, blended across the contour edges as
     DifferentiableAntialias does), and dL/d(vertex positions) of them.
 
     The "hit buffers" -- the batch's BVHs, pix2tri, the occupancy and the
-    contour edges -- come from hits(): one batched build and one batched
-    ray-cast for all meshes, then one contour extraction per mesh.  The mesh
-    edges are built once on the GPU (TriMesh3.make_edge2vtx / make_edge2tri)
+    contour edges -- come from hits(): one batched build, one batched ray-cast
+    and one batched contour extraction for all meshes.  The mesh edges are
+    built once on the GPU (TriMesh3.make_edge2vtx / make_edge2tri)
     and kept one direction per edge, so each silhouette edge is walked once
     and the gradient is that of the forward image.
 
@@ -407,16 +422,16 @@ class SilhouetteBatch:
         dev = p.device
         self.num_vtx = p.total_vtx
         n2w = ndc2world.detach().cpu().to(torch.float64)
-        self.world2ndc, self.world2pix, self.edges, self.shapes = [], [], [], []
+        self.shapes, edges, world2ndc, world2pix = [], [], [], []
         for m in range(p.num_mesh):
             a, b = int(p.mesh2pix_h[m]), int(p.mesh2pix_h[m + 1])
             w = int(p.mesh2width_h[m])
             h = (b - a) // w if w else 0
             self.shapes.append((h, w))
             w2n = torch.linalg.inv(n2w[m])
-            self.world2ndc.append(w2n.to(torch.float32).contiguous().to(dev))
-            self.world2pix.append((from_transform_ndc2pix((w, h), dtype=torch.float64) @ w2n)
-                                  .to(torch.float32).contiguous().to(dev))
+            world2ndc.append(w2n.to(torch.float32))
+            world2pix.append((from_transform_ndc2pix((w, h), dtype=torch.float64) @ w2n)
+                             .to(torch.float32))
             t0, t1 = int(p.mesh2tri_h[m]), int(p.mesh2tri_h[m + 1])
             v0, v1 = int(p.mesh2vtx_h[m]), int(p.mesh2vtx_h[m + 1])
             tri = p.tri2vtx[t0:t1]
@@ -424,96 +439,113 @@ class SilhouetteBatch:
                 e2v = make_edge2vtx(tri, v1 - v0)
                 e2t = make_edge2tri(tri, v1 - v0, e2v)
                 keep = e2v[:, 0].to(torch.int64) < e2v[:, 1].to(torch.int64)
-                rows = lambda a: a.view(torch.int32)[keep].view(torch.uint32).contiguous()
-                self.edges.append((rows(e2v), rows(e2t)))
+                edges.append((e2v.view(torch.int32)[keep], e2t.view(torch.int32)[keep]))
             else:
-                z = torch.zeros((0, 2), dtype=torch.uint32, device=dev)
-                self.edges.append((z, z))
-
-    def _slices(self, m: int):
-        p = self.pipe
-        return ((int(p.mesh2tri_h[m]), int(p.mesh2tri_h[m + 1])),
-                (int(p.mesh2vtx_h[m]), int(p.mesh2vtx_h[m + 1])),
-                (int(p.mesh2pix_h[m]), int(p.mesh2pix_h[m + 1])))
+                z = torch.zeros((0, 2), dtype=torch.int32, device=dev)
+                edges.append((z, z))
+        self._ragged = any(h * w != int(n) for (h, w), n in
+                           zip(self.shapes, np.diff(p.mesh2pix_h.astype(np.int64))))
+        # row-major per mesh, and all meshes' edges back to back
+        self._world2ndc = torch.stack(world2ndc).to(dev)
+        self._world2pix = torch.stack(world2pix).to(dev)
+        self.world2ndc = list(self._world2ndc)
+        self.world2pix = list(self._world2pix)
+        self._edge2vtx, self._edge2tri = (
+            torch.cat([e[k] for e in edges]).contiguous().view(torch.uint32) for k in (0, 1))
+        offs = np.cumsum([0] + [int(e[0].shape[0]) for e in edges])
+        self._mesh2edge = torch.from_numpy(offs.astype(np.uint32)).to(dev)
+        self.edges = [(self._edge2vtx[a:b], self._edge2tri[a:b])
+                      for a, b in zip(offs.tolist(), offs[1:].tolist())]
 
     def hits(self, vtx2xyz: torch.Tensor) -> dict:
-        """BVHs + pix2tri (batched), occupancy, contour edges per mesh.  The
-        meshes' contour extractions are enqueued back to back into slices of
-        one buffer, sharing one workspace, and their counts are read with one
-        synchronization (the same kernels and results as one call per mesh)."""
-        from .. import _lib
-        from ..Edge2Vtx import contour_for_triangle_mesh_into
-
+        """BVHs + pix2tri, occupancy and each mesh's contour edges, every stage
+        batched; the contour counts are read with one synchronization."""
         p = self.pipe
         p.set_vertices(vtx2xyz)
         p.run()
         pix2tri = p.pix2tri[: p.total_pix].clone()
         occ = (pix2tri != 0xFFFFFFFF).to(torch.float32)
-        v = p.vtx2xyz
         dev = pix2tri.device
-        sizes = [int(self.edges[m][0].shape[0]) for m in range(p.num_mesh)]
-        offs = [0]
-        for n in sizes:
-            offs.append(offs[-1] + n)
-        cbuf = torch.empty((max(offs[-1], 1), 2), dtype=torch.uint32, device=dev)
-        counts = torch.zeros((max(p.num_mesh, 1),), dtype=torch.uint32, device=dev)
-        ws = _lib.workspace(_lib.lib().dmsh_contour_workspace_bytes(max(sizes + [1])), dev)
-        live = []
-        for m in range(p.num_mesh):
-            (t0, t1), (v0, v1), _ = self._slices(m)
-            e2v, e2t = self.edges[m]
-            if t1 == t0 or e2v.shape[0] == 0:
-                continue
-            contour_for_triangle_mesh_into(p.tri2vtx[t0:t1], v[v0:v1],
-                                           self.world2ndc[m].T.contiguous().flatten(), e2v, e2t,
-                                           cbuf[offs[m]:offs[m + 1]], counts[m:m + 1], ws)
-            live.append(m)
-        counts_h = counts.view(torch.int32).cpu().tolist()
-        cedges = []
-        for m in range(p.num_mesh):
-            if m in live:
-                cedges.append(cbuf[offs[m]:offs[m] + counts_h[m]])
-            else:
-                cedges.append(self.edges[m][0])
-        return {"pix2tri": pix2tri, "occ": occ, "cedges": cedges}
+        L = _lib.lib()
+        num_edge = self._edge2vtx.shape[0]
+        cedge2vtx = torch.empty((max(num_edge, 1), 2), dtype=torch.uint32, device=dev)
+        mesh2cedge = torch.empty((p.num_mesh + 1,), dtype=torch.uint32, device=dev)
+        world2ndc = self._world2ndc.transpose(1, 2).contiguous()
+        ws = _lib.workspace(L.dmsh_batch_contour_workspace_bytes(p.num_mesh, num_edge), dev)
+        _lib.check(L.dmsh_batch_contour(
+            _lib.stream_of(dev), p.num_mesh, p.total_tri, p.total_vtx, num_edge,
+            _lib.ptr(p.mesh2tri), _lib.ptr(p.mesh2vtx), _lib.ptr(p.tri2vtx), _lib.ptr(p.vtx2xyz),
+            _lib.ptr(world2ndc), _lib.ptr(self._mesh2edge), _lib.ptr(self._edge2vtx),
+            _lib.ptr(self._edge2tri), _lib.ptr(mesh2cedge), _lib.ptr(cedge2vtx), _lib.ptr(ws),
+            ws.numel()), "dmsh_batch_contour")
+        offsets = mesh2cedge.view(torch.int32).cpu().tolist()
+        return {"pix2tri": pix2tri, "occ": occ,
+                "cedges": _ContourEdges(cedge2vtx, mesh2cedge, offsets)}
 
     @staticmethod
     def hit_bytes(hits: dict) -> int:
         return (hits["pix2tri"].numel() * 4 + hits["occ"].numel() * 4 +
                 sum(c.numel() * 4 for c in hits["cedges"]))
 
-    def images(self, vtx2xyz: torch.Tensor, hits: dict) -> torch.Tensor:
-        from ..DifferentiableAntialias.torch import antialias
+    def _contours(self, cedges):
+        """(cedge2vtx, mesh2cedge, their number) of each mesh's edges."""
+        if isinstance(cedges, _ContourEdges) and cedges.intact():
+            return cedges.batch
+        for c in cedges:
+            assert_shape_dtype_device(c, (c.shape[0], 2), torch.uint32, self.pipe.device)
+        offs = np.cumsum([0] + [int(cedges[m].shape[0]) for m in range(self.pipe.num_mesh)])
+        rows = torch.cat([cedges[m].view(torch.int32) for m in range(self.pipe.num_mesh)])
+        return (rows.contiguous().view(torch.uint32),
+                torch.from_numpy(offs.astype(np.uint32)).to(self.pipe.device), int(offs[-1]))
 
-        p = self.pipe
+    def _flat(self, t: torch.Tensor, dtype=torch.float32) -> torch.Tensor:
+        """The pixels of all images as one array."""
+        t = t.detach()[: self.pipe.total_pix].view(-1)
+        assert_shape_dtype_device(t, (self.pipe.total_pix,), dtype, self.pipe.device)
+        return t
+
+    def _antialias_args(self, vtx2xyz: torch.Tensor):
+        """The vertices and column-major transforms of an antialias call."""
+        if self._ragged:
+            raise RuntimeError("an image's pixel count is not a multiple of its width")
+        v = vtx2xyz[: self.num_vtx]
+        assert_shape_dtype_device(v, (self.num_vtx, 3), torch.float32, self.pipe.device)
+        _lib.require_gpu(v)
+        return v, self._world2pix.transpose(1, 2).contiguous()
+
+    def images(self, vtx2xyz: torch.Tensor, hits: dict) -> torch.Tensor:
+        p, L = self.pipe, _lib.lib()
         out = hits["occ"].clone()
-        v = vtx2xyz.detach()
-        for m in range(p.num_mesh):
-            _, (v0, v1), (a, b) = self._slices(m)
-            c = hits["cedges"][m]
-            if c.shape[0] == 0 or b == a:
-                continue
-            h, w = self.shapes[m]
-            out[a:b] = antialias(c, v[v0:v1], self.world2pix[m], hits["pix2tri"][a:b].view(h, w),
-                                 hits["occ"][a:b].view(h, w)).view(-1)
+        cedge2vtx, mesh2cedge, num_cedge = self._contours(hits["cedges"])
+        if num_cedge == 0 or p.total_pix == 0:
+            return out
+        v, world2pix = self._antialias_args(vtx2xyz.detach())
+        ws = _lib.workspace(L.dmsh_batch_antialias_workspace_bytes(p.total_pix), p.device)
+        _lib.check(L.dmsh_batch_antialias_fwd(
+            _lib.stream_of(p.device), p.num_mesh, self.num_vtx, p.total_pix, num_cedge,
+            _lib.ptr(p.mesh2vtx), _lib.ptr(v), _lib.ptr(p.mesh2pix), _lib.ptr(p.mesh2width),
+            _lib.ptr(mesh2cedge), _lib.ptr(cedge2vtx), _lib.ptr(world2pix),
+            _lib.ptr(self._flat(hits["pix2tri"], torch.uint32)),
+            _lib.ptr(self._flat(hits["occ"])), _lib.ptr(self._flat(out)), _lib.ptr(ws),
+            ws.numel()), "dmsh_batch_antialias_fwd")
         return out
 
     def vertex_gradient(self, vtx2xyz: torch.Tensor, hits: dict,
                         dldw: torch.Tensor) -> torch.Tensor:
-        from ..DifferentiableAntialias.torch import bwd_antialias
-
-        p = self.pipe
-        v = vtx2xyz.detach()
-        grad = torch.zeros_like(v)
-        for m in range(p.num_mesh):
-            _, (v0, v1), (a, b) = self._slices(m)
-            c = hits["cedges"][m]
-            if c.shape[0] == 0 or b == a:
-                continue
-            h, w = self.shapes[m]
-            grad[v0:v1] = bwd_antialias(c, v[v0:v1], self.world2pix[m],
-                                        hits["occ"][a:b].view(h, w), dldw[a:b].view(h, w),
-                                        hits["pix2tri"][a:b].view(h, w))
+        p, L = self.pipe, _lib.lib()
+        grad = torch.zeros_like(vtx2xyz.detach())
+        cedge2vtx, mesh2cedge, num_cedge = self._contours(hits["cedges"])
+        if num_cedge == 0 or p.total_pix == 0:
+            return grad
+        v, world2pix = self._antialias_args(vtx2xyz.detach())
+        ws = _lib.workspace(L.dmsh_batch_antialias_workspace_bytes(0), p.device)
+        _lib.check(L.dmsh_batch_antialias_bwd(
+            _lib.stream_of(p.device), p.num_mesh, self.num_vtx, p.total_pix, num_cedge,
+            _lib.ptr(p.mesh2vtx), _lib.ptr(v), _lib.ptr(grad), _lib.ptr(p.mesh2pix),
+            _lib.ptr(p.mesh2width), _lib.ptr(mesh2cedge), _lib.ptr(cedge2vtx),
+            _lib.ptr(world2pix), _lib.ptr(self._flat(hits["occ"])), _lib.ptr(self._flat(dldw)),
+            _lib.ptr(self._flat(hits["pix2tri"], torch.uint32)), _lib.ptr(ws), ws.numel()),
+            "dmsh_batch_antialias_bwd")
         return grad
 
 

@@ -132,6 +132,23 @@ _PROTOTYPES = {
         [c_void_p, c_u32, c_void_p, c_u32, c_void_p, c_void_p, c_void_p, c_u32, c_u32, c_void_p,
          c_void_p, c_void_p],
     ),
+    "dmsh_batch_contour_workspace_bytes": (c_size, [c_u32, c_u32]),
+    "dmsh_batch_contour": (
+        c_int,
+        [c_void_p, c_u32, c_u32, c_u32, c_u32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size],
+    ),
+    "dmsh_batch_antialias_workspace_bytes": (c_size, [c_u32]),
+    "dmsh_batch_antialias_fwd": (
+        c_int,
+        [c_void_p, c_u32, c_u32, c_u32, c_u32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size],
+    ),
+    "dmsh_batch_antialias_bwd": (
+        c_int,
+        [c_void_p, c_u32, c_u32, c_u32, c_u32, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
+         c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_size],
+    ),
     "dmsh_interpolate": (
         c_int, [c_void_p, c_void_p, c_u32, c_u32, c_u32, c_void_p, c_u32, c_void_p, c_u32, c_void_p,
                 c_void_p, c_void_p]),

@@ -395,6 +395,48 @@ int dmsh_antialias_bwd(void *stream, uint32_t num_cedge,
                        const float *dldw_pix2val, const uint32_t *pix2tri);
 
 /* ---------------------------------------------------------------------
+ * Contours and anti-aliased silhouettes of a CSR batch (offsets as for the
+ * batched build below): per mesh the results of
+ * dmsh_contour_for_triangle_mesh and dmsh_antialias_fwd / _bwd, each stage
+ * one launch for all meshes.  Edges [mesh2edge[m], mesh2edge[m+1]) are mesh
+ * m's, with vertex and triangle ids local to it; transforms are 16 floats
+ * column-major per mesh.  cedge2vtx needs room for total_edge pairs; mesh m's
+ * contour edges land in [mesh2cedge[m], mesh2cedge[m+1]) in edge order.  The
+ * antialias calls take num_cedge = mesh2cedge[num_mesh] (no edges: nothing is
+ * done), walk no edge of a mesh without pixels, and the backward accumulates
+ * and needs a workspace for 0 pixels.  Offsets that do not fit the totals,
+ * or a pixel count that is no multiple of its image's width, set
+ * DMSH_DEVERR_INDEX and no edge is found or walked.
+ * ------------------------------------------------------------------- */
+size_t dmsh_batch_contour_workspace_bytes(uint32_t num_mesh, uint32_t total_edge);
+int dmsh_batch_contour(void *stream, uint32_t num_mesh, uint32_t total_tri,
+                       uint32_t total_vtx, uint32_t total_edge,
+                       const uint32_t *mesh2tri, const uint32_t *mesh2vtx,
+                       const uint32_t *tri2vtx, const float *vtx2xyz,
+                       const float *transforms_world2ndc,
+                       const uint32_t *mesh2edge, const uint32_t *edge2vtx,
+                       const uint32_t *edge2tri, uint32_t *mesh2cedge,
+                       uint32_t *cedge2vtx, void *ws, size_t ws_bytes);
+size_t dmsh_batch_antialias_workspace_bytes(uint32_t total_pix);
+int dmsh_batch_antialias_fwd(void *stream, uint32_t num_mesh, uint32_t total_vtx,
+                             uint32_t total_pix, uint32_t num_cedge,
+                             const uint32_t *mesh2vtx, const float *vtx2xyz,
+                             const uint32_t *mesh2pix, const uint32_t *mesh2width,
+                             const uint32_t *mesh2cedge, const uint32_t *cedge2vtx,
+                             const float *transforms_world2pix,
+                             const uint32_t *pix2tri, const float *pix2vin,
+                             float *pix2vout, void *ws, size_t ws_bytes);
+int dmsh_batch_antialias_bwd(void *stream, uint32_t num_mesh, uint32_t total_vtx,
+                             uint32_t total_pix, uint32_t num_cedge,
+                             const uint32_t *mesh2vtx, const float *vtx2xyz,
+                             float *dldw_vtx2xyz, const uint32_t *mesh2pix,
+                             const uint32_t *mesh2width, const uint32_t *mesh2cedge,
+                             const uint32_t *cedge2vtx,
+                             const float *transforms_world2pix, const float *pix2val,
+                             const float *dldw_pix2val, const uint32_t *pix2tri,
+                             void *ws, size_t ws_bytes);
+
+/* ---------------------------------------------------------------------
  * Batched build and ray-cast: many triangle meshes of uneven size, each
  * stage one launch over all of them.  No reference counterpart (the
  * reference builds and casts one mesh per call,
