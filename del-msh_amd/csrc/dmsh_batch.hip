@@ -12,7 +12,7 @@ namespace {
 
 std::atomic<int> g_batch_stack{12};       // LDS frames per lane of the ray-cast
 std::atomic<int> g_batch_wgs_per_cu{32};  // persistent ray-cast waves per CU
-std::atomic<int> g_batch_sort_items{16};  // elements per thread of the digit passes
+std::atomic<int> g_batch_sort_items{16};  // tiles of the digit passes
 std::atomic<int> g_batch_sort_seg{1};     // segmented passes + finish (up to kSegMaxMeshes)
 std::atomic<int> g_batch_cast_waves{1};   // waves per ray-cast workgroup
 std::atomic<int> g_batch_treelet_grid{1024};

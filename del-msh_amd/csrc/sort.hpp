@@ -31,8 +31,14 @@
 namespace dmsh {
 namespace sortk {
 
-constexpr int kThreads = 256;  // 4 waves
-constexpr int kWideThreads = 512;             // wide tiles (see k_onesweep)
+constexpr int kTileUnit = 256;      // a tile is `items` (8, 12 or 16) times this many elements
+constexpr int kWideTileUnit = 512;  // a wide tile, times this many
+// A pass runs a tile on 16 waves.  Ranking is a chain of ballots and LDS reads
+// for every item of a thread, and at one or two tiles a CU nothing hides it:
+// with 256 threads of 16 items (wide tiles: 512 of 16) the three passes over
+// 14.5 M u64 keys took 562 us and a pass over a few thousand u32 keys 18.5 us;
+// with 1024 threads of 4 (8) they take 436 and 11 us.
+constexpr int kPassThreads = 1024;
 constexpr uint32_t kWideTilesFrom = 1u << 21;  // elements from which the default takes them
 constexpr int kRadixBits = 8;
 constexpr int kRadix = 1 << kRadixBits;
@@ -172,22 +178,28 @@ struct SegOff {
 
 // One digit pass.  IOTA: values are the element indices (first pass).  With
 // `n_dev`, the element
-// count is read from the device (the grid is sized for a capacity); blocks
-// whose ticket lies past the last tile exit before publishing anything, and
-// only earlier tiles are ever looked back at, so they wait on nobody.
-// THREADS: 256 (4 waves) or 512 (8 waves, for large inputs: half the tiles,
-// so half the same-address tickets and a look-back chain half as long).
+// count is read from the device (the grid is sized for a capacity); the blocks
+// past the number of tiles exit, and only earlier tickets' tiles are ever
+// looked back at, so nobody waits on them.
+// ITEMS: elements a thread; large inputs take wide tiles (half the tiles, so
+// half the same-address tickets and a look-back chain half as long).
 // SEG: a segmented pass (see SegOff); `hist` is not read.
-template <typename KeyT, int ITEMS, bool IOTA, int THREADS = kThreads, bool SEG = false>
-__global__ __launch_bounds__(THREADS) void k_onesweep(
+template <typename KeyT, int ITEMS, bool IOTA, bool SEG = false>
+__global__ __launch_bounds__(kPassThreads) void k_onesweep(
     const KeyT* __restrict__ kin, const uint32_t* __restrict__ vin, KeyT* __restrict__ kout,
     uint32_t* __restrict__ vout, uint32_t n, const uint32_t* __restrict__ n_dev, uint32_t shift,
     uint32_t dbits, const uint32_t* __restrict__ hist, uint32_t* __restrict__ status,
     uint32_t* __restrict__ ticket, uint32_t* __restrict__ err, SegOff seg) {
+  constexpr int THREADS = kPassThreads;
   static_assert(THREADS >= kRadix && THREADS % 64 == 0, "one thread per digit");
-  if (n_dev) n = *n_dev;
   constexpr int kTile = THREADS * ITEMS;
   constexpr uint32_t W = THREADS / 64;
+  if (n_dev) {
+    // as many workgroups as there are tiles take tickets, and no others: the
+    // atomics of a grid for the capacity would queue (15 ns each)
+    n = *n_dev;
+    if (blockIdx.x >= (n + (uint32_t)kTile - 1u) / (uint32_t)kTile) return;
+  }
   __shared__ uint32_t s_wcnt[W][kRadix];
   __shared__ uint32_t s_excl[kRadix];
   __shared__ uint32_t s_gbase[kRadix];
@@ -203,7 +215,7 @@ __global__ __launch_bounds__(THREADS) void k_onesweep(
   __syncthreads();
   const uint32_t tile = s_tile;
   const uint32_t tile_base = tile * (uint32_t)kTile;
-  if (tile_base >= n) return;  // past the data (a capacity-sized grid)
+  if (tile_base >= n) return;
   const uint32_t wave_base = tile_base + wave * 64u * ITEMS;
 
   KeyT key[ITEMS];
@@ -221,7 +233,8 @@ __global__ __launch_bounds__(THREADS) void k_onesweep(
   for (int i = 0; i < ITEMS; ++i) {
     const bool valid = dig[i] != 0xFFFFFFFFu;
     uint64_t m = __ballot(valid);
-    for (uint32_t b = 0; b < dbits; ++b) {
+#pragma unroll
+    for (uint32_t b = 0; b < (uint32_t)kRadixBits; ++b) {  // bits above dbits are 0 in all lanes
       const bool bit = (dig[i] >> b) & 1u;
       const uint64_t bb = __ballot(bit);
       m &= bit ? bb : ~bb;
@@ -763,16 +776,16 @@ inline int sort_small(hipStream_t s, const Src& src, uint32_t n, uint32_t key_bi
 
 template <typename KeyT>
 inline uint32_t num_tiles(uint32_t n) {
-  return ceil_div(n, (uint64_t)kThreads * Tune<KeyT>::kItems);
+  return ceil_div(n, (uint64_t)kTileUnit * Tune<KeyT>::kItems);
 }
 
-// Elements per thread of a digit pass: the default (Tune), or 8 / 12 / 16 for
+// The items of a digit pass's tile: the default (Tune), or 8 / 12 / 16 for
 // callers that tune it (the batched build); a workspace used with more than
 // one value is sized for the smallest, which has the most tiles.
 constexpr int kMinItems = 8;
 inline bool valid_items(int items) { return items == 8 || items == 12 || items == 16; }
 inline uint32_t num_tiles_items(uint32_t n, int items) {
-  return ceil_div(n, (uint64_t)kThreads * (uint64_t)items);
+  return ceil_div(n, (uint64_t)kTileUnit * (uint64_t)items);
 }
 
 inline uint32_t num_passes(uint32_t key_bits) { return ceil_div(key_bits, kRadixBits); }
@@ -839,34 +852,23 @@ inline int launch_pass_items(hipStream_t s, uint32_t n, uint32_t key_bits, const
   const uint32_t tiles = num_tiles_items(n, ITEMS);
   const uint32_t shift = SEG ? seg_shift : digit * kRadixBits;
   const uint32_t dbits = SEG ? (uint32_t)kRadixBits : pass_bits(key_bits, digit);
-  // each pass's status region is sized for 256-thread tiles
+  // each pass's status region is sized for the narrow tiles
   uint32_t* st = L.status + (size_t)slot * tiles * kRadix;
   const int wide_opt = refit_option(kSortWideTiles);
   const bool wide = wide_opt == 2 || (wide_opt == 1 && n >= kWideTilesFrom);
-  if (wide) {
-    const uint32_t wt = ceil_div(n, (uint64_t)kWideThreads * ITEMS);
-    if (iota) {
-      launch("k_onesweep", (k_onesweep<KeyT, ITEMS, true, kWideThreads, SEG>), dim3(wt),
-             dim3(kWideThreads), 0, s, sk, sv, dk, dv, n, n_dev, shift, dbits,
-             L.hist + digit * kRadix, st, L.tickets + slot, err, seg);
-    } else {
-      launch("k_onesweep", (k_onesweep<KeyT, ITEMS, false, kWideThreads, SEG>), dim3(wt),
-             dim3(kWideThreads), 0, s, sk, sv, dk, dv, n, n_dev, shift, dbits,
-             L.hist + digit * kRadix, st, L.tickets + slot, err, seg);
-    }
-  } else if (iota) {
-    launch("k_onesweep", (k_onesweep<KeyT, ITEMS, true, kThreads, SEG>), dim3(tiles), dim3(kThreads), 0, s, sk,
-           sv, dk, dv, n, n_dev, shift, dbits, L.hist + digit * kRadix, st, L.tickets + slot, err,
-           seg);
-  } else {
-    launch("k_onesweep", (k_onesweep<KeyT, ITEMS, false, kThreads, SEG>), dim3(tiles), dim3(kThreads), 0, s, sk,
-           sv, dk, dv, n, n_dev, shift, dbits, L.hist + digit * kRadix, st, L.tickets + slot, err,
-           seg);
-  }
+  auto pass = [&](auto kernel, uint32_t grid) {
+    launch("k_onesweep", kernel, dim3(grid), dim3(kPassThreads), 0, s, sk, sv, dk, dv, n, n_dev,
+           shift, dbits, L.hist + digit * kRadix, st, L.tickets + slot, err, seg);
+  };
+  const uint32_t wt = ceil_div(n, (uint64_t)kWideTileUnit * ITEMS);
+  if (wide && iota) pass(k_onesweep<KeyT, ITEMS / 2, true, SEG>, wt);
+  else if (wide) pass(k_onesweep<KeyT, ITEMS / 2, false, SEG>, wt);
+  else if (iota) pass(k_onesweep<KeyT, ITEMS / 4, true, SEG>, tiles);
+  else pass(k_onesweep<KeyT, ITEMS / 4, false, SEG>, tiles);
   return launch_status();
 }
 
-// items: elements per thread (0: the default of KeyT).
+// items: of the tile (0: the default of KeyT).
 template <typename KeyT>
 inline int launch_pass(hipStream_t s, uint32_t n, uint32_t key_bits, const Layout& L,
                        uint32_t digit, uint32_t slot, bool iota, const KeyT* sk,
@@ -993,7 +995,7 @@ inline int run_seg_passes_items(hipStream_t s, uint32_t n, uint32_t key_bits, ui
   return launch_status();
 }
 
-// items: elements per thread of the passes (8, 12 or 16).
+// items: of the passes' tiles (8, 12 or 16).
 template <typename KeyT>
 inline int run_seg_passes(hipStream_t s, uint32_t n, uint32_t key_bits, uint32_t code_bits,
                           const Layout& L, const uint32_t* seg_off, uint32_t seg_rows,

@@ -319,7 +319,7 @@ def autotune(p: Pipeline, reps: int = 2, stacks=(12, 16, 20, 24, 32), wgs_per_cu
     keeps the fastest (results do not depend on them).  The ray-cast is tuned
     over (LDS stack frames, ray-cast waves per CU), then over the workgroup
     size (waves per workgroup) at that pair; the build over (refit grid,
-    elements per thread of the radix-sort digit passes, the sort: three
+    the tile of the radix-sort digit passes in 256 elements, the sort: three
     segmented passes over the codes and the LDS finish, or one pass per 8-bit
     digit of the whole composite key).  Returns {"cast": {...}, "build":
     {...}, "trials": [...]}."""

@@ -462,7 +462,7 @@ int dmsh_batch_antialias_bwd(void *stream, uint32_t num_mesh, uint32_t total_vtx
  * 32; default 20),
  * "batch.wgs_per_cu" (persistent ray-cast workgroups per CU, 1..64),
  * "batch.treelet_grid" (refit workgroups, 1..65536),
- * "batch.sort_items" (elements per thread of the digit passes: 8, 12, 16),
+ * "batch.sort_items" (a digit pass's tile in 256 elements: 8, 12, 16),
  * "batch.cast_waves" (waves per ray-cast workgroup: 1, 2, 4),
  * "batch.sort_seg" (1, the default: up to 8192 meshes, the composite keys
  * are sorted inside their meshes by three passes over the code's top 24 bits
