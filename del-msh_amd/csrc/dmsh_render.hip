@@ -253,12 +253,13 @@ int dmsh_rasterized_edge_gradient_bwd(void* stream, const uint32_t* tri2vtx, uin
 
 
 namespace {
-// Workspace of the ordered edge-gradient backward for P pixel pairs:
-// offsets [P + 1], scan tile sums, then per record slot (3 per pair) the
-// vertex id, the record index and the term, and the sort's workspace.
+// Workspace of the ordered edge-gradient backward for P pixel pairs: an offset
+// per workgroup of 256 pairs (and their total), its found terms (3 slots per
+// pair), per record the vertex id, the record index and the term, and the
+// sort's workspace.
 struct EgLayout {
   uint32_t* off;
-  uint32_t* sums;
+  uint32_t* found;
   uint32_t* rec_vtx;
   uint32_t* rec_idx;
   float* rec_term;
@@ -277,9 +278,9 @@ uint32_t eg_key_bits(uint32_t num_vtx) {
 }
 
 bool eg_carve(Arena& a, uint32_t num_pair, uint32_t num_vtx, EgLayout& L) {
-  const uint32_t cap = 3u * num_pair;
-  L.off = a.take<uint32_t>((size_t)num_pair + 1);
-  L.sums = a.take<uint32_t>(topo::scan_tiles(num_pair));
+  const uint32_t cap = 3u * num_pair, blocks = ceil_div(num_pair, 256);
+  L.off = a.take<uint32_t>((size_t)blocks + 1);
+  L.found = a.take<uint32_t>((size_t)blocks * eg::kEgSlots);
   L.rec_vtx = a.take<uint32_t>(cap);
   L.rec_idx = a.take<uint32_t>(cap);
   L.rec_term = a.take<float>((size_t)cap * 3);
@@ -326,23 +327,24 @@ int dmsh_rasterized_edge_gradient_bwd_ordered(
   if (!err) return DMSH_ERR_HIP;
   hipStream_t s = as_stream(stream);
   const uint32_t cap = 3u * num_pair;
-  const uint32_t blocks = std::min<uint32_t>(ceil_div(num_pair, 256), 16384);
-  launch("k_eg_count", eg::k_eg_count, dim3(blocks), dim3(256), 0, s, tri2vtx, num_tri, vtx2xyz,
-         num_vtx, transform_world2pix, img_w, img_h, pix2tri, num_vdim, pix2val, dldw_pix2val,
-         num_pair, L.off, err);
+  const uint32_t blocks = ceil_div(num_pair, 256);
+  launch("k_eg_find", eg::k_eg_find, dim3(blocks), dim3(256), 0, s, tri2vtx, num_tri, vtx2xyz,
+         num_vtx, transform_world2pix, img_w, img_h, pix2tri, num_pair, L.off, L.found, err);
   int rc = launch_status();
   if (rc != DMSH_OK) return rc;
-  // in place: off[s] = records before pair s, off[num_pair] = all records
-  if ((rc = topo::launch_exclusive_scan(s, num_pair, L.off, L.off, L.sums)) != DMSH_OK) return rc;
+  launch("k_eg_scan", eg::k_eg_scan, dim3(1), dim3(1024), 0, s, L.off, blocks);
+  if ((rc = launch_status()) != DMSH_OK) return rc;
   launch("k_eg_records", eg::k_eg_records, dim3(blocks), dim3(256), 0, s, tri2vtx, num_tri,
          vtx2xyz, num_vtx, transform_world2pix, img_w, img_h, pix2tri, num_vdim, pix2val,
-         dldw_pix2val, num_pair, L.off, L.rec_vtx, L.rec_idx, L.rec_term, err);
+         dldw_pix2val, (const uint32_t*)L.off, (const uint32_t*)L.found, L.rec_vtx, L.rec_idx,
+         L.rec_term, err);
   if ((rc = launch_status()) != DMSH_OK) return rc;
-  rc = sortk::sort_pairs_device_count<uint32_t>(s, cap, L.off + num_pair, L.rec_vtx, L.rec_idx,
+  rc = sortk::sort_pairs_device_count<uint32_t>(s, cap, L.off + blocks, L.rec_vtx, L.rec_idx,
                                                 eg_key_bits(num_vtx), L.sort_ws, L.sort_bytes);
   if (rc != DMSH_OK) return rc;
-  launch("k_eg_sum", eg::k_eg_sum, dim3(std::min<uint32_t>(ceil_div(cap, 256), 16384)),
-         dim3(256), 0, s, (const uint32_t*)(L.off + num_pair), (const uint32_t*)L.rec_vtx,
+  // few pixel pairs have records: a grid for a sixteenth of the slots
+  launch("k_eg_sum", eg::k_eg_sum, dim3(std::min<uint32_t>(ceil_div(cap, 256 * 16), 16384)),
+         dim3(256), 0, s, (const uint32_t*)(L.off + blocks), (const uint32_t*)L.rec_vtx,
          (const uint32_t*)L.rec_idx, (const float*)L.rec_term, num_vtx, cap, dldw_vtx2xyz, err);
   return launch_status();
 }

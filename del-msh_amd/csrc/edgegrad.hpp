@@ -16,7 +16,7 @@
 // results agree with the serial CPU loop to rounding only.
 #pragma once
 
-#include "dmsh_common.hpp"
+#include "sort.hpp"
 
 namespace dmsh {
 namespace eg {
@@ -154,13 +154,18 @@ static __global__ __launch_bounds__(256) void k_edge_grad_bwd(
 //   outer and ih0 inner (pixel-y Jacobian), s = iw (H - 1) + ih0; then the
 //   horizontal pairs (iw0, ih)-(iw0 + 1, ih) with iw0 outer and ih inner
 //   (pixel-x Jacobian), s = W (H - 1) + iw0 H + ih.
-//   k_eg_count: terms per pair (0..3, one per vertex slot whose projection
-//   gradient exists), in pair order;  exclusive scan -> record offsets and
-//   the record count on the device;  k_eg_records: record r = (vertex id,
-//   r, the term's three floats), records in pair order and, inside a pair,
-//   in vertex-slot order (the loop's order);  a stable radix sort by vertex
-//   id keeps that order inside each vertex;  k_eg_sum: one thread per vertex
-//   adds its run to dldw_vtx2xyz left to right.
+//   k_eg_find: which terms a pair has (0..3, one per vertex slot whose
+//   projection gradient exists), packed to the front of the workgroup's slots
+//   in pair order and, inside a pair, in vertex-slot order (the loop's order);
+//   k_eg_scan: exclusive scan of the workgroups' counts;  k_eg_records: record
+//   r = (vertex id, r, the term's three floats), a thread a term;  a stable
+//   radix sort by vertex id keeps that order inside each vertex;  k_eg_sum:
+//   one thread per vertex adds its run to dldw_vtx2xyz left to right.
+// Of the 522 000 pairs of a 512 x 512 image of a 50 000-triangle sphere a few
+// thousand have terms: the find is bound by its projections and divisions, the
+// rest is latency.  Working every term out twice, once to
+// count it, and scanning a count a pair took 102 us of kernels; this, with the
+// faster sort passes, 69.
 // ---------------------------------------------------------------------------
 struct PairRef {
   size_t ip0, ip1;
@@ -194,13 +199,10 @@ __device__ __forceinline__ PairRef pair_of(uint32_t s, uint32_t img_w, uint32_t 
   return r;
 }
 
-// The pair's terms, as edge_pair computes them: returns the mask of vertex
-// slots of the receiving triangle `itri` that get a term; term[k] holds slot
-// k's three floats.
-__device__ __forceinline__ uint32_t pair_terms(const Ctx& c, const uint32_t* __restrict__ pix2tri,
-                                               uint32_t nv, const float* __restrict__ pix2val,
-                                               const float* __restrict__ dpix, const PairRef& r,
-                                               uint32_t& itri, float term[3][3]) {
+// Which terms the pair has, as edge_pair decides it: the mask of vertex slots of
+// the receiving triangle (that of the pair's second pixel if `second`).
+__device__ __forceinline__ uint32_t pair_mask(const Ctx& c, const uint32_t* __restrict__ pix2tri,
+                                              const PairRef& r, bool& second) {
   const uint32_t t0 = pix2tri[r.ip0], t1 = pix2tri[r.ip1];
   if (t0 == t1) return 0u;
   float b[3];
@@ -213,26 +215,38 @@ __device__ __forceinline__ uint32_t pair_terms(const Ctx& c, const uint32_t* __r
     return 0u;
   }
   if (in0 == in1) return 0u;  // neither: shared edge; both: intersection
+  // not inside, so the receiving triangle is there and has an area
+  second = in1;
+  const uint32_t* tv = c.tri2vtx + (size_t)(in1 ? t1 : t0) * 3;
+  uint32_t mask = 0u;
+#pragma unroll
+  for (int inode = 0; inode < 3; ++inode) {
+    float d[3];
+    if (proj_grad(c.m, c.xyz + (size_t)tv[inode] * 3, r.axis, d)) mask |= 1u << inode;
+  }
+  return mask;
+}
+
+// The term of vertex slot `inode`, and that vertex.
+__device__ __forceinline__ uint32_t pair_term(const Ctx& c, const uint32_t* __restrict__ pix2tri,
+                                              uint32_t nv, const float* __restrict__ pix2val,
+                                              const float* __restrict__ dpix, const PairRef& r,
+                                              bool second, uint32_t inode, float term[3]) {
   float dldpa = 0.f;
   for (uint32_t k = 0; k < nv; ++k) {
     const float v0 = pix2val[r.ip0 * nv + k], v1 = pix2val[r.ip1 * nv + k];
     const float g0 = dpix[r.ip0 * nv + k], g1 = dpix[r.ip1 * nv + k];
     dldpa += (g0 + g1) * 0.5f * (v0 - v1);
   }
-  itri = in1 ? t1 : t0;
-  if (bary(c, in1 ? r.pc1 : r.pc0, itri, b) != 1) return 0u;
-  const uint32_t* tv = c.tri2vtx + (size_t)itri * 3;
-  uint32_t mask = 0u;
+  const uint32_t itri = pix2tri[second ? r.ip1 : r.ip0];
+  float b[3] = {0.f, 0.f, 0.f}, d[3] = {0.f, 0.f, 0.f};
+  bary(c, second ? r.pc1 : r.pc0, itri, b);
+  const uint32_t iv = c.tri2vtx[(size_t)itri * 3 + inode];
+  proj_grad(c.m, c.xyz + (size_t)iv * 3, r.axis, d);
+  const float bi = inode == 0u ? b[0] : (inode == 1u ? b[1] : b[2]);
 #pragma unroll
-  for (int inode = 0; inode < 3; ++inode) {
-    float d[3];
-    if (!proj_grad(c.m, c.xyz + (size_t)tv[inode] * 3, r.axis, d)) continue;
-    term[inode][0] = b[inode] * d[0] * dldpa;
-    term[inode][1] = b[inode] * d[1] * dldpa;
-    term[inode][2] = b[inode] * d[2] * dldpa;
-    mask |= 1u << inode;
-  }
-  return mask;
+  for (int j = 0; j < 3; ++j) term[j] = bi * d[j] * dldpa;
+  return iv;
 }
 
 __device__ __forceinline__ Ctx make_ctx(const uint32_t* tri2vtx, uint32_t num_tri,
@@ -249,50 +263,90 @@ __device__ __forceinline__ Ctx make_ctx(const uint32_t* tri2vtx, uint32_t num_tr
   return c;
 }
 
-static __global__ __launch_bounds__(256) void k_eg_count(
+constexpr uint32_t kEgSlots = 3u * 256u;  // term slots of a workgroup's 256 pairs
+
+static __global__ __launch_bounds__(256) void k_eg_find(
     const uint32_t* __restrict__ tri2vtx, uint32_t num_tri, const float* __restrict__ xyz,
     uint32_t num_vtx, const float* __restrict__ T, uint32_t img_w, uint32_t img_h,
-    const uint32_t* __restrict__ pix2tri, uint32_t nv, const float* __restrict__ pix2val,
-    const float* __restrict__ dpix, uint32_t num_pair, uint32_t* __restrict__ cnt,
-    uint32_t* err) {
+    const uint32_t* __restrict__ pix2tri, uint32_t num_pair, uint32_t* __restrict__ block_count,
+    uint32_t* __restrict__ found, uint32_t* err) {
+  __shared__ uint32_t s_w[4];
   const Ctx c = make_ctx(tri2vtx, num_tri, xyz, num_vtx, T, err);
-  for (uint32_t s = blockIdx.x * blockDim.x + threadIdx.x; s < num_pair;
-       s += gridDim.x * blockDim.x) {
-    uint32_t itri;
-    float term[3][3];
-    const uint32_t mask = pair_terms(c, pix2tri, nv, pix2val, dpix, pair_of(s, img_w, img_h),
-                                     itri, term);
-    cnt[s] = (uint32_t)__builtin_popcount(mask);
+  const uint32_t s = blockIdx.x * 256u + threadIdx.x;
+  uint32_t mask = 0u;
+  bool second = false;
+  if (s < num_pair) mask = pair_mask(c, pix2tri, pair_of(s, img_w, img_h), second);
+  // terms before this thread's: the low and the high bit of the counts by ballots
+  const uint32_t count = (uint32_t)__builtin_popcount(mask);
+  const uint64_t lo = __ballot(count & 1u), hi = __ballot(count & 2u);
+  const uint32_t wave = threadIdx.x >> 6;
+  if ((threadIdx.x & 63u) == 0u) s_w[wave] = (uint32_t)__popcll(lo) + 2u * (uint32_t)__popcll(hi);
+  __syncthreads();
+  uint32_t r = mask_rank(lo) + 2u * mask_rank(hi), total = 0u;
+#pragma unroll
+  for (uint32_t w = 0; w < 4u; ++w) {
+    if (w < wave) r += s_w[w];
+    total += s_w[w];
   }
+  if (threadIdx.x == 0u) block_count[blockIdx.x] = total;
+  r += blockIdx.x * kEgSlots;
+#pragma unroll
+  for (uint32_t inode = 0; inode < 3u; ++inode)
+    if ((mask >> inode) & 1u) found[r++] = s << 3 | (second ? 4u : 0u) | inode;
 }
 
+// Counts -> exclusive offsets in place, the total at [n] (one workgroup, eight
+// counts a thread and round).
+static __global__ __launch_bounds__(1024) void k_eg_scan(uint32_t* __restrict__ count, uint32_t n) {
+  constexpr uint32_t K = 8u;
+  __shared__ uint32_t s_w[16];
+  uint32_t carry = 0u;
+  for (uint32_t base = 0; base < n; base += 1024u * K) {
+    uint32_t v[K], sum = 0u;
+    const uint32_t i0 = base + threadIdx.x * K;
+#pragma unroll
+    for (uint32_t k = 0; k < K; ++k) {
+      v[k] = i0 + k < n ? count[i0 + k] : 0u;
+      sum += v[k];
+    }
+    const uint32_t inc = sortk::wave_inclusive_scan(sum);
+    if ((threadIdx.x & 63u) == 63u) s_w[threadIdx.x >> 6] = inc;
+    __syncthreads();
+    uint32_t pre = carry + inc - sum;
+    for (uint32_t w = 0; w < 16u; ++w) {
+      if (w < (threadIdx.x >> 6)) pre += s_w[w];
+      carry += s_w[w];
+    }
+#pragma unroll
+    for (uint32_t k = 0; k < K; ++k) {
+      if (i0 + k < n) count[i0 + k] = pre;
+      pre += v[k];
+    }
+    __syncthreads();
+  }
+  if (threadIdx.x == 0u) count[n] = carry;
+}
+
+// The records: workgroup b's found terms from off[b] on.
 static __global__ __launch_bounds__(256) void k_eg_records(
     const uint32_t* __restrict__ tri2vtx, uint32_t num_tri, const float* __restrict__ xyz,
     uint32_t num_vtx, const float* __restrict__ T, uint32_t img_w, uint32_t img_h,
     const uint32_t* __restrict__ pix2tri, uint32_t nv, const float* __restrict__ pix2val,
-    const float* __restrict__ dpix, uint32_t num_pair, const uint32_t* __restrict__ off,
-    uint32_t* __restrict__ rec_vtx, uint32_t* __restrict__ rec_idx,
-    float* __restrict__ rec_term, uint32_t* err) {
-  // off [num_pair + 1]: the exclusive scan of k_eg_count's counts
+    const float* __restrict__ dpix, const uint32_t* __restrict__ off,
+    const uint32_t* __restrict__ found, uint32_t* __restrict__ rec_vtx,
+    uint32_t* __restrict__ rec_idx, float* __restrict__ rec_term, uint32_t* err) {
+  const uint32_t first = off[blockIdx.x], n = off[blockIdx.x + 1] - first;
+  if (threadIdx.x >= n) return;
   const Ctx c = make_ctx(tri2vtx, num_tri, xyz, num_vtx, T, err);
-  for (uint32_t s = blockIdx.x * blockDim.x + threadIdx.x; s < num_pair;
-       s += gridDim.x * blockDim.x) {
-    if (off[s + 1] == off[s]) continue;
-    uint32_t itri;
-    float term[3][3];
-    const uint32_t mask = pair_terms(c, pix2tri, nv, pix2val, dpix, pair_of(s, img_w, img_h),
-                                     itri, term);
-    uint32_t r = off[s];
-#pragma unroll
-    for (int inode = 0; inode < 3; ++inode) {
-      if (!((mask >> inode) & 1u)) continue;
-      rec_vtx[r] = tri2vtx[(size_t)itri * 3 + inode];
-      rec_idx[r] = r;
-      rec_term[(size_t)r * 3 + 0] = term[inode][0];
-      rec_term[(size_t)r * 3 + 1] = term[inode][1];
-      rec_term[(size_t)r * 3 + 2] = term[inode][2];
-      ++r;
-    }
+  for (uint32_t i = threadIdx.x; i < n; i += 256u) {
+    const uint32_t f = found[blockIdx.x * kEgSlots + i], r = first + i;
+    float term[3];
+    rec_vtx[r] = pair_term(c, pix2tri, nv, pix2val, dpix, pair_of(f >> 3, img_w, img_h),
+                           (f & 4u) != 0u, f & 3u, term);
+    rec_idx[r] = r;
+    rec_term[(size_t)r * 3 + 0] = term[0];
+    rec_term[(size_t)r * 3 + 1] = term[1];
+    rec_term[(size_t)r * 3 + 2] = term[2];
   }
 }
 
