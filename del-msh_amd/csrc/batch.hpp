@@ -296,6 +296,9 @@ constexpr uint32_t kSegTables = sortk::kTopPasses * sortk::kRadix;  // words per
 // in LDS and is flushed to hseg when a round reaches past it (then it starts
 // at the round's first mesh); a round spanning more meshes than the window
 // (meshes of fewer than 64 triangles) counts the rest with global atomics.
+// The window's first triangles and unit-cube fits sit in LDS too: a binary
+// search over the offsets and a fit (two divisions) a triangle were most of
+// the 181 us that 14.5 M triangles took; now 87.
 static __global__ __launch_bounds__(256) void k_batch_morton_seghist(
     const uint32_t* __restrict__ bad, uint32_t total_tri, uint32_t M,
     const uint32_t* __restrict__ mesh2tri, const float* __restrict__ cntr,
@@ -308,8 +311,24 @@ static __global__ __launch_bounds__(256) void k_batch_morton_seghist(
   const uint32_t t0 = blockIdx.x * per;
   if (t0 >= total_tri) return;  // uniform over the block
   const uint32_t t1 = total_tri - t0 < per ? total_tri : t0 + per;
+  __shared__ uint32_t s_first[kSegWindow + 1];  // first triangles of the window's meshes
+  __shared__ float s_fit[kSegWindow][4];        // scale and shift of their unit-cube fits
   for (uint32_t e = threadIdx.x; e < kW; e += blockDim.x) s_h[e] = 0u;
-  uint32_t wbase = find_segment(mesh2tri, M, t0);  // the window's first mesh (uniform)
+  uint32_t wbase;  // the window's first mesh (uniform)
+  auto open_window = [&](uint32_t t) {
+    wbase = find_segment(mesh2tri, M, t);
+    if (threadIdx.x <= kSegWindow) {
+      const uint32_t m = wbase + threadIdx.x;
+      s_first[threadIdx.x] = m < M ? mesh2tri[m] : total_tri;
+      if (threadIdx.x < kSegWindow && m < M) {
+        float T[16];
+        bld::fit_transform(keys6 + (size_t)m * 6, T);
+        s_fit[threadIdx.x][0] = T[0];
+        for (int d = 0; d < 3; ++d) s_fit[threadIdx.x][1 + d] = T[12 + d];
+      }
+    }
+  };
+  open_window(t0);
   auto flush = [&]() {
     for (uint32_t e = threadIdx.x; e < kW; e += blockDim.x) {
       const uint32_t v = s_h[e];
@@ -321,22 +340,30 @@ static __global__ __launch_bounds__(256) void k_batch_morton_seghist(
   __syncthreads();
   for (uint32_t r0 = t0; r0 < t1; r0 += blockDim.x) {
     const uint32_t rl = t1 - r0 < blockDim.x ? t1 - 1 : r0 + blockDim.x - 1;
-    const uint32_t mlast = find_segment(mesh2tri, M, rl);  // uniform
-    if (mlast - wbase >= kSegWindow) {
+    if (rl >= s_first[kSegWindow]) {
       __syncthreads();  // the window's counts are complete
       flush();
-      wbase = find_segment(mesh2tri, M, r0);
-      __syncthreads();  // zeroed before the round counts
+      open_window(r0);
+      __syncthreads();  // zeroed and opened before the round counts
     }
     const uint32_t t = r0 + threadIdx.x;
     if (t < t1) {
-      const uint32_t m = find_segment(mesh2tri, M, t);
+      // the last mesh of the window that starts at or before t
+      uint32_t w = 0u;
+#pragma unroll
+      for (uint32_t k = 1; k <= kSegWindow; ++k)
+        if (s_first[k] <= t) w = k;
       float T[16];
-      bld::fit_transform(keys6 + (size_t)m * 6, T);
+      uint32_t m = wbase + w;
+      if (w < kSegWindow) {
+        bld::set_fit(T, s_fit[w][0], s_fit[w] + 1);
+      } else {
+        m = find_segment(mesh2tri, M, t);
+        bld::fit_transform(keys6 + (size_t)m * 6, T);
+      }
       const float* p = cntr + (size_t)t * 3;
       const uint32_t code = morton3_transformed<uint32_t>(T, p[0], p[1], p[2]);
       codes[t] = ((uint64_t)m << kMeshKeyShift) | code;
-      const uint32_t w = m - wbase;
 #pragma unroll
       for (uint32_t q = 0; q < kP; ++q) {
         const uint32_t d = (code >> (kSegLow + q * sortk::kRadixBits)) & (kR - 1u);
@@ -440,51 +467,68 @@ static __global__ __launch_bounds__(256) void k_batch_seg_cols(
     if (i < cnt) O[(size_t)(m0 + i) * kR + d] = o[i] - col;
 }
 
-// The codes of one mesh (index 0 = the mesh's first) through a window over
-// all meshes' codes.
-template <typename KeyT>
+// The codes of one mesh (index 0 = the mesh's first) through a window over the
+// low words of all meshes' keys: the 30 code bits, and above them two bits of
+// the mesh, which its keys share.
 struct MeshCodes {
-  CodeWindow<KeyT> w;
-  uint32_t tb;
-  __device__ MeshCodes(const CodeWindow<KeyT>& w_, uint32_t tb_) : w(w_), tb(tb_) {}
-  __device__ __forceinline__ KeyT operator[](uint32_t j) const { return w[tb + j]; }
+  const __attribute__((address_space(1))) uint32_t* g;  // keys, as pairs of words
+  const __attribute__((address_space(3))) uint32_t* s;  // low words of keys [lo, lo + len)
+  uint32_t lo, len, tb;
+  __device__ MeshCodes(const uint64_t* keys, const uint32_t* lds, uint32_t lo_, uint32_t len_,
+                       uint32_t tb_)
+      : g((const __attribute__((address_space(1))) uint32_t*)keys),
+        s((const __attribute__((address_space(3))) uint32_t*)lds),
+        lo(lo_),
+        len(len_),
+        tb(tb_) {}
+  __device__ __forceinline__ uint32_t operator[](uint32_t j) const {
+    const uint32_t o = tb + j - lo;
+    if (o < len) return s[o];
+    return g[(size_t)(tb + j) * 2];
+  }
 };
 
 // Internal node g of all meshes (g < inner_off[M]), a thread each.  Node g
 // of mesh m searches the codes around mesh2tri[m] + (g - inner_off[m]), so a
 // block's nodes search one nearly contiguous run of codes: that run and
 // kTopoHalo codes either side sit in LDS (kWin codes at most; any other
-// code is read from memory), as in k_topology.
+// code is read from memory), as in k_topology.  The searches are bound by
+// their instructions, so they compare the codes' 32 bits; and as a block's
+// nodes are nearly always of one mesh, the others look for theirs from the
+// first node's on.  14.5 M triangles: 430 us with the 64-bit keys and three
+// searches for the mesh, 358 now.
 static __global__ __launch_bounds__(kTopoThreads) void k_batch_topology(
     const uint32_t* __restrict__ bad, uint32_t total_tri, uint32_t M,
     const uint32_t* __restrict__ mesh2tri, const uint32_t* __restrict__ inner_off,
     const uint32_t* __restrict__ node_off, uint32_t* __restrict__ bvhnodes,
     const uint64_t* __restrict__ codes, const uint32_t* __restrict__ idx, TreeletSink ts) {
   constexpr uint32_t kWin = 2 * kTopoHalo + 2 * kTopoThreads + 1;
-  __shared__ uint64_t s_c[kWin];
+  __shared__ uint32_t s_c[kWin];
   if (*bad) return;
   const uint32_t total_inner = inner_off[M];
   const uint32_t base = blockIdx.x * kTopoThreads;
   if (base >= total_inner || base >= total_tri) return;  // uniform over the block
   const uint32_t last_g = (total_inner - base < kTopoThreads ? total_inner : base + kTopoThreads) - 1u;
   const uint32_t m_first = find_segment(inner_off, M, base);
-  const uint32_t m_last = find_segment(inner_off, M, last_g);
+  const uint32_t m_last = inner_off[m_first + 1] > last_g
+                              ? m_first
+                              : m_first + find_segment(inner_off + m_first, M - m_first, last_g);
   const uint32_t a_lo = base + mesh2tri[m_first] - inner_off[m_first];
   const uint32_t a_hi = last_g + mesh2tri[m_last] - inner_off[m_last];
   const uint32_t lo = a_lo > kTopoHalo ? a_lo - kTopoHalo : 0u;
   uint32_t hi = total_tri - a_hi > kTopoHalo + 2u ? a_hi + kTopoHalo + 2u : total_tri;
   if (hi - lo > kWin) hi = lo + kWin;
-  for (uint32_t j = lo + threadIdx.x; j < hi; j += kTopoThreads) s_c[j - lo] = codes[j];
+  for (uint32_t j = lo + threadIdx.x; j < hi; j += kTopoThreads) s_c[j - lo] = (uint32_t)codes[j];
   __syncthreads();
   const uint32_t g = base + threadIdx.x;
   if (g > last_g) return;
-  const uint32_t m = find_segment(inner_off, M, g);
+  const uint32_t m = m_first + find_segment(inner_off + m_first, m_last - m_first + 1u, g);
   const uint32_t tb = mesh2tri[m], n = mesh2tri[m + 1] - tb;
-  const MeshCodes<uint64_t> c(CodeWindow<uint64_t>(codes, s_c, lo, hi - lo), tb);
+  const MeshCodes c(codes, s_c, lo, hi - lo, tb);
   const uint32_t i = g - inner_off[m];
   uint32_t first, last;
-  node_range<uint64_t>(c, n, i, first, last);
-  const uint32_t split = node_split<uint64_t>(c, first, last);
+  node_range<uint32_t>(c, n, i, first, last);
+  const uint32_t split = node_split<uint32_t>(c, first, last);
   topology_emit(n, i, first, last, split, bvhnodes + (size_t)node_off[m] * 3, idx + tb, tb, ts, m,
                 tb, inner_off[m]);
 }

@@ -160,6 +160,18 @@ __global__ __launch_bounds__(256) void k_centroid_aabb(uint32_t n,
   }
 }
 
+// Column-major scale and shift.
+__device__ __forceinline__ void set_fit(float T[16], float scale, const float shift[3]) {
+#pragma unroll
+  for (int k = 0; k < 16; ++k) T[k] = 0.f;
+  T[0] = scale;
+  T[5] = scale;
+  T[10] = scale;
+  T[15] = 1.f;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) T[12 + d] = shift[d];
+}
+
 // Column-major unit-cube fit of the reduced box: s = 1 / max extent,
 // translation -center * s + 0.5.
 __device__ __forceinline__ void fit_transform(const uint32_t* __restrict__ keys6, float T[16]) {
@@ -173,17 +185,13 @@ __device__ __forceinline__ void fit_transform(const uint32_t* __restrict__ keys6
   ext = fmax_sel(ext, mx[1] - mn[1]);
   ext = fmax_sel(ext, mx[2] - mn[2]);
   const float s = 1.f / ext;
-#pragma unroll
-  for (int k = 0; k < 16; ++k) T[k] = 0.f;
-  T[0] = s;
-  T[5] = s;
-  T[10] = s;
-  T[15] = 1.f;
+  float shift[3];
 #pragma unroll
   for (int d = 0; d < 3; ++d) {
     const float c = (mn[d] + mx[d]) * 0.5f;
-    T[12 + d] = (-c) * s + 0.5f;
+    shift[d] = (-c) * s + 0.5f;
   }
+  set_fit(T, s, shift);
 }
 
 // The reduced box of the copies, in every lane of the wave.
