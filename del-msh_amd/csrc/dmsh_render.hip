@@ -388,8 +388,10 @@ size_t dmsh_smooth_gradient_workspace_bytes(uint32_t img_w, uint32_t img_h) {
   if (img_w < 2 || img_h < 2) return 256;
   const SmoothGrids g = smooth_grids(img_w, img_h);
   Arena a{nullptr, ~(size_t)0, 0};
-  a.take<float>(g.nh);
-  a.take<float>(g.nv);
+  for (int k = 0; k < 2; ++k) {
+    a.take<float>(g.nh);
+    a.take<float>(g.nv);
+  }
   a.take<uint8_t>(g.nh);
   a.take<uint8_t>(g.nv);
   return a.off + 256;
@@ -407,6 +409,8 @@ int dmsh_smooth_gradient(void* stream, uint32_t img_w, uint32_t img_h, const uin
   Arena a{static_cast<char*>(ws), ws_bytes, 0};
   float* h2 = a.take<float>(g.nh);
   float* v2 = a.take<float>(g.nv);
+  float* h3 = a.take<float>(g.nh);
+  float* v3 = a.take<float>(g.nv);
   uint8_t* hm = a.take<uint8_t>(g.nh);
   uint8_t* vm = a.take<uint8_t>(g.nv);
   if (!a.ok()) return DMSH_ERR_WORKSPACE;
@@ -418,19 +422,19 @@ int dmsh_smooth_gradient(void* stream, uint32_t img_w, uint32_t img_h, const uin
   if ((rc = launch_status()) != DMSH_OK) return rc;
   const uint32_t steps = 2u * num_iter;
   const uint32_t launches = ceil_div(steps, (uint32_t)eg::kSmoothK);
-  // launches alternate buffers and must end in the caller's arrays
+  // launches alternate between the caller's arrays and a buffer and must end in
+  // the caller's: of an odd number the second goes to a third buffer, and a single
+  // one reads a copy
   float *hs = hedge2dldr, *vs = vedge2dldr, *hd = h2, *vd = v2;
-  if (launches % 2 == 1) {
+  if (launches == 1) {
     launch("k_copy_f32", eg::k_copy_f32, dim3(std::min<uint32_t>(ceil_div(g.nh, 256), 2048)),
            dim3(256), 0, s, hedge2dldr, h2, g.nh);
     if ((rc = launch_status()) != DMSH_OK) return rc;
     launch("k_copy_f32", eg::k_copy_f32, dim3(std::min<uint32_t>(ceil_div(g.nv, 256), 2048)),
            dim3(256), 0, s, vedge2dldr, v2, g.nv);
     if ((rc = launch_status()) != DMSH_OK) return rc;
-    hs = h2;
-    vs = v2;
-    hd = hedge2dldr;
-    vd = vedge2dldr;
+    std::swap(hs, hd);
+    std::swap(vs, vd);
   }
   for (uint32_t step0 = 0; step0 < steps; step0 += eg::kSmoothK) {
     const uint32_t n = std::min<uint32_t>(eg::kSmoothK, steps - step0);
@@ -441,6 +445,13 @@ int dmsh_smooth_gradient(void* stream, uint32_t img_w, uint32_t img_h, const uin
     if ((rc = launch_status()) != DMSH_OK) return rc;
     std::swap(hs, hd);
     std::swap(vs, vd);
+    if (step0 == 0 && launches % 2 == 1) {
+      hd = h3;
+      vd = v3;
+    } else if (step0 == eg::kSmoothK && launches % 2 == 1) {
+      hd = hedge2dldr;
+      vd = vedge2dldr;
+    }
   }
   return DMSH_OK;
 }

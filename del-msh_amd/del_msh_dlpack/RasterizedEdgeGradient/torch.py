@@ -81,10 +81,11 @@ def edge_gradient_and_type(tri2vtx: torch.Tensor, vtx2xyz: torch.Tensor,
     assert_shape_dtype_device(pix2val, (img_h, img_w, num_vdim), torch.float32, device)
     assert_shape_dtype_device(dldw_pix2val, (img_h, img_w, num_vdim), torch.float32, device)
     _lib.require_gpu(tri2vtx, vtx2xyz, transform_world2pix, pix2tri, pix2val, dldw_pix2val)
-    hedge2type = torch.zeros((img_h - 1, img_w), dtype=torch.uint8, device=device)
-    hedge2dldr = torch.zeros((img_h - 1, img_w), dtype=torch.float32, device=device)
-    vedge2type = torch.zeros((img_h, img_w - 1), dtype=torch.uint8, device=device)
-    vedge2dldr = torch.zeros((img_h, img_w - 1), dtype=torch.float32, device=device)
+    # the kernel writes every pixel edge
+    hedge2type = torch.empty((img_h - 1, img_w), dtype=torch.uint8, device=device)
+    hedge2dldr = torch.empty((img_h - 1, img_w), dtype=torch.float32, device=device)
+    vedge2type = torch.empty((img_h, img_w - 1), dtype=torch.uint8, device=device)
+    vedge2dldr = torch.empty((img_h, img_w - 1), dtype=torch.float32, device=device)
     from . import edge_gradient_and_type as native
 
     native(tri2vtx, vtx2xyz, transform_world2pix.T.contiguous().flatten(), pix2tri, pix2val,
