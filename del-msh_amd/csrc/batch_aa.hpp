@@ -7,10 +7,10 @@
 // the offsets, the contour edges are compacted over the whole batch in edge
 // order (so mesh m's are a contiguous run from mesh2cedge[m] on, in its own edge
 // order), and the walks of all meshes share a launch.  The arithmetic, and the
-// writes that win, are the single-mesh ones.  Eight meshes of 5,000 to 200,000 triangles (512 x 512
-// images), forward and recomputing backward: 212 launches and 2.52 ms before,
-// 67 and 1.63 ms now; what is left of it is the two casts and builds, and the
-// contours and walks take 0.13 ms.
+// writes that win, are the single-mesh ones.  Eight meshes of 5,000 to 200,000
+// triangles (512 x 512 images), forward and recomputing backward: 212 launches
+// and 2.52 ms before, 67 and 1.57 ms now; what is left is the two casts and
+// builds, and the contours and walks take 0.13 ms.
 #pragma once
 
 #include "antialias.hpp"

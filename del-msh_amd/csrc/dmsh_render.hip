@@ -60,7 +60,6 @@ void launch_pix2tri_waves(int waves, hipStream_t s, const rc::ImageSrc& src,
 void launch_pix2tri_any(int stack, int waves, hipStream_t s, const rc::ImageSrc& src,
                         const rc::CastState& st, uint32_t* pix2tri, float* pix2t) {
   switch (stack) {
-    case 8: launch_pix2tri_waves<8>(waves, s, src, st, pix2tri, pix2t); break;
     case 16: launch_pix2tri_waves<16>(waves, s, src, st, pix2tri, pix2t); break;
     case 20: launch_pix2tri_waves<20>(waves, s, src, st, pix2tri, pix2t); break;
     case 24: launch_pix2tri_waves<24>(waves, s, src, st, pix2tri, pix2t); break;
@@ -76,7 +75,7 @@ extern "C" {
 int dmsh_set_tuning(const char* key, int value) {
   if (!key) return DMSH_ERR_INVALID;
   if (std::strcmp(key, "pix2tri.stack") == 0) {
-    if (value != 8 && value != 12 && value != 16 && value != 20 && value != 24 && value != 32)
+    if (value != 12 && value != 16 && value != 20 && value != 24 && value != 32)
       return DMSH_ERR_INVALID;
     g_cast_stack.store(value);
     return DMSH_OK;

@@ -52,12 +52,12 @@ int dmsh_get_device_errors(uint32_t *bits_out);
 
 /* Process-wide launch tuning (no reference counterpart; set by the
  * autotuner).  Keys: "pix2tri.stack" (LDS frames per lane: 12, 16, 20, 24,
- * 32; default 20), "pix2tri.waves" (waves per workgroup: 1, 2, 4), and the
+ * 32; default 12), "pix2tri.waves" (waves per workgroup: 1, 2, 4), and the
  * refit's "refit.leaves_in_aabb" (0, 1), "refit.climb" (0, 1, 2; default 2),
  * "refit.queue" (0, 1), "refit.top" (0, 1), "refit.plan_cache" (0, 1),
  * "refit.compact" (levels climbed before the remaining climbs move to the
  * first lanes, 0..1023; default 0: never), and the sort's "sort.wide_tiles"
- * (digit passes in 512-thread tiles: 0 never, 1 from 2^21 elements (default),
+ * (digit passes in tiles twice as large: 0 never, 1 from 2^21 elements (default),
  * 2 always).  get returns -1 for an unknown key. */
 int dmsh_set_tuning(const char *key, int value);
 int dmsh_get_tuning(const char *key);
@@ -458,8 +458,8 @@ int dmsh_batch_antialias_bwd(void *stream, uint32_t num_mesh, uint32_t total_vtx
  * Ray-cast: image of mesh m = pixels [mesh2pix[m], mesh2pix[m+1]) of
  * pix2tri / pix2t (nullable), mesh2width[m] pixels wide, row 0 at the top,
  * cast with transforms_ndc2world + 16 m (column-major).
- * Tuning keys (results do not depend on them): "batch.stack" (16, 20, 24,
- * 32; default 20),
+ * Tuning keys (results do not depend on them): "batch.stack" (12, 16, 20,
+ * 24, 32; default 12),
  * "batch.wgs_per_cu" (persistent ray-cast workgroups per CU, 1..64),
  * "batch.treelet_grid" (refit workgroups, 1..65536),
  * "batch.sort_items" (a digit pass's tile in 256 elements: 8, 12, 16),
