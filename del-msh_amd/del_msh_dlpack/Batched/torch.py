@@ -382,18 +382,30 @@ def autotune(p: Pipeline, reps: int = 2, stacks=(12, 16, 20, 24, 32), wgs_per_cu
 # ---------------------------------------------------------------------------
 # differentiable anti-aliased silhouettes of a batch
 # ---------------------------------------------------------------------------
+class _Parts:
+    """The slices of one buffer that were handed out in a list, and where they
+    lay.  A caller may put other tensors in their place, or give them other
+    memory; the buffer is then no longer what the list holds."""
+
+    def __init__(self, tensors):
+        self.own = [(t, t.data_ptr()) for t in tensors]
+
+    def are(self, tensors) -> bool:
+        return len(tensors) == len(self.own) and all(
+            t is own and t.data_ptr() == at for t, (own, at) in zip(tensors, self.own))
+
+
 class _ContourEdges(list):
     """Each mesh's contour edges, as slices of the batch's compacted buffer
     (mesh m's are rows mesh2cedge[m] .. mesh2cedge[m+1])."""
 
     def __init__(self, cedge2vtx: torch.Tensor, mesh2cedge: torch.Tensor, offsets):
         super().__init__(cedge2vtx[a:b] for a, b in zip(offsets, offsets[1:]))
-        self.own = tuple(self)
-        self.batch = (cedge2vtx, mesh2cedge, offsets[-1])
+        self.parts = _Parts(self)
+        self.batch = (cedge2vtx, mesh2cedge, offsets)
 
     def intact(self) -> bool:
-        """Still the slices (a caller may put other edges in their place)."""
-        return len(self) == len(self.own) and all(a is b for a, b in zip(self, self.own))
+        return self.parts.are(self)
 
 
 class SilhouetteBatch:
@@ -407,6 +419,10 @@ class SilhouetteBatch:
     built once on the GPU (TriMesh3.make_edge2vtx / make_edge2tri)
     and kept one direction per edge, so each silhouette edge is walked once
     and the gradient is that of the forward image.
+
+    world2ndc and world2pix (4 x 4 float32), edges (edge2vtx, edge2tri) and
+    shapes (height, width) are lists with an entry per mesh; entries may be
+    written in place or replaced (another camera, other edges).
 
     No reference counterpart (the reference renders and differentiates one
     mesh per call)."""
@@ -443,19 +459,44 @@ class SilhouetteBatch:
             else:
                 z = torch.zeros((0, 2), dtype=torch.int32, device=dev)
                 edges.append((z, z))
-        self._ragged = any(h * w != int(n) for (h, w), n in
-                           zip(self.shapes, np.diff(p.mesh2pix_h.astype(np.int64))))
-        # row-major per mesh, and all meshes' edges back to back
+        # all meshes' transforms (row-major) and edges back to back, and slices
+        # of them in the lists
         self._world2ndc = torch.stack(world2ndc).to(dev)
         self._world2pix = torch.stack(world2pix).to(dev)
         self.world2ndc = list(self._world2ndc)
         self.world2pix = list(self._world2pix)
-        self._edge2vtx, self._edge2tri = (
-            torch.cat([e[k] for e in edges]).contiguous().view(torch.uint32) for k in (0, 1))
-        offs = np.cumsum([0] + [int(e[0].shape[0]) for e in edges])
-        self._mesh2edge = torch.from_numpy(offs.astype(np.uint32)).to(dev)
-        self.edges = [(self._edge2vtx[a:b], self._edge2tri[a:b])
-                      for a, b in zip(offs.tolist(), offs[1:].tolist())]
+        self._own_world2ndc, self._own_world2pix = _Parts(self.world2ndc), _Parts(self.world2pix)
+        self._edges = self._cat_edges(edges)
+        ends = np.cumsum([int(e[0].shape[0]) for e in edges]).tolist()
+        self.edges = [(self._edges[0][a:b], self._edges[1][a:b]) for a, b in zip([0] + ends, ends)]
+        self._own_edges = _Parts([t for e in self.edges for t in e])
+        self._own_shapes = list(self.shapes)
+        self._npix = np.diff(p.mesh2pix_h.astype(np.int64)).tolist()
+        self._whole = all(h * w == n for (h, w), n in zip(self.shapes, self._npix))
+
+    def _cat_edges(self, edges):
+        """(edge2vtx, edge2tri, mesh2edge) of all meshes' edges back to back."""
+        offs = np.cumsum([0] + [int(e[0].shape[0]) for e in edges]).astype(np.uint32)
+        rows = (torch.cat([e[k].view(torch.int32) for e in edges]).view(torch.uint32)
+                for k in (0, 1))
+        return (*rows, torch.from_numpy(offs).to(self.pipe.device))
+
+    def _edge_args(self):
+        """The edges as _cat_edges lays them out, and {mesh: contour edges} of
+        meshes whose own edges are taken as such: a mesh without triangles has
+        no normals to decide by."""
+        if self._own_edges.are([t for e in self.edges for t in e]):
+            return self._edges, {}
+        edges, given = [], {}
+        for m, (e2v, e2t) in enumerate(self.edges[: self.pipe.num_mesh]):
+            _lib.require_gpu(e2v, e2t)
+            assert e2v.is_contiguous() and e2t.is_contiguous()
+            assert e2v.shape == e2t.shape == (e2v.shape[0], 2), (e2v.shape, e2t.shape)
+            if self.pipe.mesh2tri_h[m + 1] == self.pipe.mesh2tri_h[m] and e2v.shape[0]:
+                given[m] = e2v
+                e2v, e2t = e2v[:0], e2t[:0]
+            edges.append((e2v, e2t))
+        return self._cat_edges(edges), given
 
     def hits(self, vtx2xyz: torch.Tensor) -> dict:
         """BVHs + pix2tri, occupancy and each mesh's contour edges, every stage
@@ -467,20 +508,30 @@ class SilhouetteBatch:
         occ = (pix2tri != 0xFFFFFFFF).to(torch.float32)
         dev = pix2tri.device
         L = _lib.lib()
-        num_edge = self._edge2vtx.shape[0]
+        (edge2vtx, edge2tri, mesh2edge), given = self._edge_args()
+        num_edge = edge2vtx.shape[0]
         cedge2vtx = torch.empty((max(num_edge, 1), 2), dtype=torch.uint32, device=dev)
         mesh2cedge = torch.empty((p.num_mesh + 1,), dtype=torch.uint32, device=dev)
-        world2ndc = self._world2ndc.transpose(1, 2).contiguous()
+        if self._own_world2ndc.are(self.world2ndc):
+            world2ndc = self._world2ndc.transpose(1, 2).contiguous()
+        else:
+            columns = [t.detach().T.contiguous().flatten() for t in self.world2ndc[: p.num_mesh]]
+            for t in columns:
+                _lib.require_gpu(t)
+                _lib.check_transform(t, "world2ndc")
+            world2ndc = torch.stack(columns)
         ws = _lib.workspace(L.dmsh_batch_contour_workspace_bytes(p.num_mesh, num_edge), dev)
         _lib.check(L.dmsh_batch_contour(
             _lib.stream_of(dev), p.num_mesh, p.total_tri, p.total_vtx, num_edge,
             _lib.ptr(p.mesh2tri), _lib.ptr(p.mesh2vtx), _lib.ptr(p.tri2vtx), _lib.ptr(p.vtx2xyz),
-            _lib.ptr(world2ndc), _lib.ptr(self._mesh2edge), _lib.ptr(self._edge2vtx),
-            _lib.ptr(self._edge2tri), _lib.ptr(mesh2cedge), _lib.ptr(cedge2vtx), _lib.ptr(ws),
-            ws.numel()), "dmsh_batch_contour")
+            _lib.ptr(world2ndc), _lib.ptr(mesh2edge), _lib.ptr(edge2vtx), _lib.ptr(edge2tri),
+            _lib.ptr(mesh2cedge), _lib.ptr(cedge2vtx), _lib.ptr(ws), ws.numel()),
+            "dmsh_batch_contour")
         offsets = mesh2cedge.view(torch.int32).cpu().tolist()
-        return {"pix2tri": pix2tri, "occ": occ,
-                "cedges": _ContourEdges(cedge2vtx, mesh2cedge, offsets)}
+        cedges = _ContourEdges(cedge2vtx, mesh2cedge, offsets)
+        for m, e2v in given.items():
+            cedges[m] = e2v
+        return {"pix2tri": pix2tri, "occ": occ, "cedges": cedges}
 
     @staticmethod
     def hit_bytes(hits: dict) -> int:
@@ -488,7 +539,7 @@ class SilhouetteBatch:
                 sum(c.numel() * 4 for c in hits["cedges"]))
 
     def _contours(self, cedges):
-        """(cedge2vtx, mesh2cedge, their number) of each mesh's edges."""
+        """(cedge2vtx, mesh2cedge, its entries) of each mesh's edges."""
         if isinstance(cedges, _ContourEdges) and cedges.intact():
             return cedges.batch
         for c in cedges:
@@ -496,7 +547,7 @@ class SilhouetteBatch:
         offs = np.cumsum([0] + [int(cedges[m].shape[0]) for m in range(self.pipe.num_mesh)])
         rows = torch.cat([cedges[m].view(torch.int32) for m in range(self.pipe.num_mesh)])
         return (rows.contiguous().view(torch.uint32),
-                torch.from_numpy(offs.astype(np.uint32)).to(self.pipe.device), int(offs[-1]))
+                torch.from_numpy(offs.astype(np.uint32)).to(self.pipe.device), offs.tolist())
 
     def _flat(self, t: torch.Tensor, dtype=torch.float32) -> torch.Tensor:
         """The pixels of all images as one array."""
@@ -504,26 +555,46 @@ class SilhouetteBatch:
         assert_shape_dtype_device(t, (self.pipe.total_pix,), dtype, self.pipe.device)
         return t
 
-    def _antialias_args(self, vtx2xyz: torch.Tensor):
-        """The vertices and column-major transforms of an antialias call."""
-        if self._ragged:
-            raise RuntimeError("an image's pixel count is not a multiple of its width")
+    def _antialias_args(self, vtx2xyz: torch.Tensor, offsets):
+        """The vertices, image widths and column-major transforms of an
+        antialias call over the contour edges of `offsets`."""
+        p = self.pipe
         v = vtx2xyz[: self.num_vtx]
-        assert_shape_dtype_device(v, (self.num_vtx, 3), torch.float32, self.pipe.device)
+        assert_shape_dtype_device(v, (self.num_vtx, 3), torch.float32, p.device)
         _lib.require_gpu(v)
-        return v, self._world2pix.transpose(1, 2).contiguous()
+        width = p.mesh2width
+        if not self._whole:
+            raise RuntimeError("an image's pixel count is not a multiple of its width")
+        if self.shapes != self._own_shapes:
+            # an image without contour edges is not walked: one row
+            width = np.array([max(n, 1) for n in self._npix], np.uint32)
+            for m, n in enumerate(self._npix):
+                if n == 0 or offsets[m] == offsets[m + 1]:
+                    continue
+                h, w = self.shapes[m]
+                if h * w != n:
+                    raise RuntimeError(f"image {m}: {n} pixels are not {h} rows of {w}")
+                width[m] = w
+            width = torch.from_numpy(width).to(p.device)
+        world2pix = self._world2pix
+        if not self._own_world2pix.are(self.world2pix):
+            for t in self.world2pix[: p.num_mesh]:
+                assert_shape_dtype_device(t, (4, 4), torch.float32, p.device)
+            world2pix = torch.stack(self.world2pix[: p.num_mesh])
+        return v, width, world2pix.transpose(1, 2).contiguous()
 
     def images(self, vtx2xyz: torch.Tensor, hits: dict) -> torch.Tensor:
         p, L = self.pipe, _lib.lib()
         out = hits["occ"].clone()
-        cedge2vtx, mesh2cedge, num_cedge = self._contours(hits["cedges"])
+        cedge2vtx, mesh2cedge, offsets = self._contours(hits["cedges"])
+        num_cedge = offsets[-1]
         if num_cedge == 0 or p.total_pix == 0:
             return out
-        v, world2pix = self._antialias_args(vtx2xyz.detach())
+        v, width, world2pix = self._antialias_args(vtx2xyz.detach(), offsets)
         ws = _lib.workspace(L.dmsh_batch_antialias_workspace_bytes(p.total_pix), p.device)
         _lib.check(L.dmsh_batch_antialias_fwd(
             _lib.stream_of(p.device), p.num_mesh, self.num_vtx, p.total_pix, num_cedge,
-            _lib.ptr(p.mesh2vtx), _lib.ptr(v), _lib.ptr(p.mesh2pix), _lib.ptr(p.mesh2width),
+            _lib.ptr(p.mesh2vtx), _lib.ptr(v), _lib.ptr(p.mesh2pix), _lib.ptr(width),
             _lib.ptr(mesh2cedge), _lib.ptr(cedge2vtx), _lib.ptr(world2pix),
             _lib.ptr(self._flat(hits["pix2tri"], torch.uint32)),
             _lib.ptr(self._flat(hits["occ"])), _lib.ptr(self._flat(out)), _lib.ptr(ws),
@@ -534,15 +605,16 @@ class SilhouetteBatch:
                         dldw: torch.Tensor) -> torch.Tensor:
         p, L = self.pipe, _lib.lib()
         grad = torch.zeros_like(vtx2xyz.detach())
-        cedge2vtx, mesh2cedge, num_cedge = self._contours(hits["cedges"])
+        cedge2vtx, mesh2cedge, offsets = self._contours(hits["cedges"])
+        num_cedge = offsets[-1]
         if num_cedge == 0 or p.total_pix == 0:
             return grad
-        v, world2pix = self._antialias_args(vtx2xyz.detach())
+        v, width, world2pix = self._antialias_args(vtx2xyz.detach(), offsets)
         ws = _lib.workspace(L.dmsh_batch_antialias_workspace_bytes(0), p.device)
         _lib.check(L.dmsh_batch_antialias_bwd(
             _lib.stream_of(p.device), p.num_mesh, self.num_vtx, p.total_pix, num_cedge,
             _lib.ptr(p.mesh2vtx), _lib.ptr(v), _lib.ptr(grad), _lib.ptr(p.mesh2pix),
-            _lib.ptr(p.mesh2width), _lib.ptr(mesh2cedge), _lib.ptr(cedge2vtx),
+            _lib.ptr(width), _lib.ptr(mesh2cedge), _lib.ptr(cedge2vtx),
             _lib.ptr(world2pix), _lib.ptr(self._flat(hits["occ"])), _lib.ptr(self._flat(dldw)),
             _lib.ptr(self._flat(hits["pix2tri"], torch.uint32)), _lib.ptr(ws), ws.numel()),
             "dmsh_batch_antialias_bwd")

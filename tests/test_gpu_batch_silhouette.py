@@ -78,3 +78,68 @@ def test_batch_equals_single_meshes(gpu, num_mesh):
     hits["cedges"] = [c.clone() for c in sb.hits(v)["cedges"]]
     assert torch.equal(sb.images(v, hits), want_img) and not torch.equal(half, want_img)
     assert _lib.device_errors() == 0
+
+
+def _single(sb, m, hits, m2v, m2p, v, dldw):
+    """Image and gradient of mesh m by the single-mesh entry points."""
+    p = slice(int(m2p[m]), int(m2p[m + 1]))
+    vm, c = v[int(m2v[m]):int(m2v[m + 1])], hits["cedges"][m]
+    im = lambda a: a[p].view(*sb.shapes[m])
+    pix, occ = im(hits["pix2tri"]), im(hits["occ"])
+    return (DifferentiableAntialias.antialias(c, vm, sb.world2pix[m], pix, occ).view(-1),
+            DifferentiableAntialias.bwd_antialias(c, vm, sb.world2pix[m], occ, im(dldw), pix))
+
+
+REPLACED = [(what, how) for what in ("world2ndc", "world2pix", "edges", "shapes")
+            for how in ("entry", "list")]
+REPLACED += [("world2ndc", "in place"), ("world2ndc", "data"), ("world2pix", "in place"),
+             ("world2pix", "data"), ("edges", "data")]
+
+
+@pytest.mark.parametrize("what,how", REPLACED)
+def test_replaced_entries_are_used(gpu, what, how):
+    """Another camera, other edges or another image shape in place of a mesh's
+    own, by whichever way the caller puts it there."""
+    m2t, m2v, tri, vtx, m2p, width, n2w = _batch(5)
+    g = lambda a: torch.from_numpy(a).to(gpu)
+    t, v = g(tri), g(vtx)
+    dldw = g(np.random.default_rng(1).normal(size=int(m2p[-1])).astype(np.float32))
+    sb = Batched.SilhouetteBatch(m2t, m2v, t, v, m2p, width, n2w)
+    before = sb.hits(v)
+    img_before = sb.images(v, before)
+    m = 3
+    if what == "edges":
+        new = tuple(e[::3].contiguous() for e in sb.edges[m])
+    elif what == "shapes":
+        new = (1, sb.shapes[m][0] * sb.shapes[m][1])
+    else:  # the mesh turned about x and moved aside
+        turn = torch.tensor([[1, 0, 0, 0.1], [0, 0.8, -0.6, 0], [0, 0.6, 0.8, 0], [0, 0, 0, 1.0]])
+        new = (getattr(sb, what)[m].cpu() @ turn).to(gpu)
+    entries = getattr(sb, what)
+    if how == "entry":
+        entries[m] = new
+    elif how == "list":
+        setattr(sb, what, [new if k == m else e for k, e in enumerate(entries)])
+    elif how == "in place":
+        entries[m].copy_(new)
+    else:
+        for old, data in zip(entries[m], new) if what == "edges" else [(entries[m], new)]:
+            old.data = data
+    hits = sb.hits(v)
+    for k in range(5):
+        if sb.edges[k][0].shape[0] == 0:
+            continue
+        want = contour_for_triangle_mesh(
+            t[int(m2t[k]):int(m2t[k + 1])], v[int(m2v[k]):int(m2v[k + 1])],
+            sb.world2ndc[k].T.contiguous().flatten(), *sb.edges[k])
+        assert torch.equal(hits["cedges"][k].view(torch.int32), want.view(torch.int32))
+    same = torch.equal(hits["cedges"][m].view(torch.int32), before["cedges"][m].view(torch.int32))
+    assert same == (what in ("world2pix", "shapes"))
+    img, grad = sb.images(v, hits), sb.vertex_gradient(v, hits, dldw)
+    want_img, want_grad = _single(sb, m, hits, m2v, m2p, v, dldw)
+    p, q = slice(int(m2p[m]), int(m2p[m + 1])), slice(int(m2v[m]), int(m2v[m + 1]))
+    assert torch.equal(img[p], want_img) and not torch.equal(img[p], img_before[p])
+    assert torch.equal(img[:p.start], img_before[:p.start])
+    # the bound of test_batch_equals_single_meshes
+    assert float((grad[q] - want_grad).abs().max()) <= 1800 * 2.0 ** -24 * float(want_grad.abs().max())
+    assert _lib.device_errors() == 0
