@@ -563,9 +563,7 @@ class SilhouetteBatch:
         assert_shape_dtype_device(v, (self.num_vtx, 3), torch.float32, p.device)
         _lib.require_gpu(v)
         width = p.mesh2width
-        if not self._whole:
-            raise RuntimeError("an image's pixel count is not a multiple of its width")
-        if self.shapes != self._own_shapes:
+        if not self._whole or self.shapes != self._own_shapes:
             # an image without contour edges is not walked: one row
             width = np.array([max(n, 1) for n in self._npix], np.uint32)
             for m, n in enumerate(self._npix):

@@ -143,3 +143,30 @@ def test_replaced_entries_are_used(gpu, what, how):
     # the bound of test_batch_equals_single_meshes
     assert float((grad[q] - want_grad).abs().max()) <= 1800 * 2.0 ** -24 * float(want_grad.abs().max())
     assert _lib.device_errors() == 0
+
+
+def test_broken_rows_of_an_image_without_contours(gpu):
+    """An image whose pixels are not whole rows stops only a call that has to
+    walk its contour edges."""
+    m2t, m2v, tri, vtx, m2p, width, n2w = _batch(4)
+    g = lambda a: torch.from_numpy(a).to(gpu)
+    t, v = g(tri), g(vtx)
+    dldw = g(np.random.default_rng(1).normal(size=int(m2p[-1])).astype(np.float32))
+    whole = Batched.SilhouetteBatch(m2t, m2v, t, v, m2p, width, n2w)
+    hits = whole.hits(v)
+    want = whole.images(v, hits), whole.vertex_gradient(v, hits, dldw)
+    for m, ok in ((1, True), (3, False)):  # the emptied mesh, and one with contours
+        broken = width.copy()
+        broken[m] += 1
+        assert int(m2p[m + 1] - m2p[m]) % int(broken[m]) != 0
+        sb = Batched.SilhouetteBatch(m2t, m2v, t, v, m2p, broken, n2w)
+        if ok:
+            assert torch.equal(sb.images(v, hits), want[0])
+            # the bound of test_batch_equals_single_meshes
+            bound = 1800 * 2.0 ** -24 * float(want[1].abs().max())
+            assert float((sb.vertex_gradient(v, hits, dldw) - want[1]).abs().max()) <= bound
+        else:
+            for call in (lambda: sb.images(v, hits), lambda: sb.vertex_gradient(v, hits, dldw)):
+                with pytest.raises(RuntimeError):
+                    call()
+    assert _lib.device_errors() == 0
