@@ -51,6 +51,11 @@ constexpr uint32_t kMaxCastWaves = 8192;        // 32 waves on each of 256 CUs
 constexpr uint32_t kXcds = 8;
 constexpr uint32_t kCastCounts = 32 + 32 * kXcds;  // words of CastState::counts
 
+// Bounds of what the regular test serves: boxes and origins within kRegularMax
+// and, on one axis, a reciprocal within kRegularInv give a finite t there, as
+// 2 * 2^62 * 2^64 = 2^127 is below the largest float.
+constexpr float kRegularMax = 0x1p62f, kRegularInv = 0x1p64f;
+
 enum : int { kTraceOk = 0, kTraceOverflow = 1, kTraceBadIndex = 2 };
 
 struct alignas(16) InnerNode {
@@ -118,7 +123,7 @@ __device__ __forceinline__ void store_inner(InnerNode* __restrict__ inner, uint3
     bool fin = true;
 #pragma unroll
     for (int k = 0; k < 6; ++k)
-      fin = fin && fabsf(b0[k]) < __builtin_inff() && fabsf(b1[k]) < __builtin_inff();
+      fin = fin && fabsf(b0[k]) <= kRegularMax && fabsf(b1[k]) <= kRegularMax;
 #pragma unroll
     for (int k = 0; k < 3; ++k) fin = fin && b0[k] <= b0[k + 3] && b1[k] <= b1[k + 3];
     if (!fin) atomicOr(nonfinite, 1u);
@@ -130,8 +135,8 @@ __device__ __forceinline__ void store_inner(InnerNode* __restrict__ inner, uint3
 // c1): parts 0..2 hold the children's bounds x0..x3 (box 0 bounds 0-3;
 // bounds 4, 5 of box 0 and 0, 1 of box 1; box 1 bounds 2-5), part 3 the
 // refs.  A record whose children do not fit the layout raises (part 0), is
-// the one every ray misses and sets *nonfinite, as a part with a bound that is
-// not finite does (the boxes here are the refit's own: with finite bounds
+// the one every ray misses and sets *nonfinite, as a part with a bound outside
+// +-kRegularMax does (the boxes here are the refit's own: with finite bounds
 // lo <= hi).  Writing the four parts from consecutive threads makes a
 // wave's store one contiguous kilobyte.
 __device__ __forceinline__ uint4 inner_part_bits(uint32_t part, uint32_t c0, uint32_t c1,
@@ -155,8 +160,8 @@ __device__ __forceinline__ uint4 inner_part_bits(uint32_t part, uint32_t c0, uin
                       __float_as_uint(e.w));
   }
   if (part == 3u) return make_uint4(r0, r1, 0u, 0u);
-  const bool fin = fabsf(x0) < __builtin_inff() && fabsf(x1) < __builtin_inff() &&
-                   fabsf(x2) < __builtin_inff() && fabsf(x3) < __builtin_inff();
+  const bool fin = fabsf(x0) <= kRegularMax && fabsf(x1) <= kRegularMax &&
+                   fabsf(x2) <= kRegularMax && fabsf(x3) <= kRegularMax;
   if (!fin) atomicOr(nonfinite, 1u);
   return make_uint4(__float_as_uint(x0), __float_as_uint(x1), __float_as_uint(x2),
                     __float_as_uint(x3));
@@ -314,17 +319,18 @@ __device__ __forceinline__ void leaf_test(const Packed& pk, uint32_t slot, const
   tri_out = has ? __float_as_uint(lt.c.y) : DMSH_U32MAX;
 }
 
-// Slab test for a regular ray (see regular_ray) against a finite box with
-// lo <= hi.  The plane a ray enters through is lo for a positive reciprocal and
-// hi for a negative one: with lo <= hi and correctly rounded (so monotone)
-// subtraction and product that t is the smaller of the two, so selecting the
-// plane gives what the general test's compare-and-select gives, up to the sign
-// of a zero, which no later comparison can see.  A parallel axis carries the
+// Slab test for a regular ray (see regular_ray) against a box within
+// +-kRegularMax with lo <= hi.  The plane a ray enters through is lo for a
+// positive reciprocal and hi for a negative one: with lo <= hi and correctly
+// rounded (so monotone) subtraction and product that t is the smaller of the
+// two, so selecting the plane gives what the general test's compare-and-select
+// gives, up to the sign of a zero, which no later comparison can see.  A
+// parallel axis carries the
 // reciprocal +inf: lo < o gives -inf, lo > o gives +inf, and lo == o gives NaN,
 // which fmaxf ignores as it would -inf (for hi: fminf, +inf); so an origin
-// outside the slab leaves tmin = +inf or tmax = -inf and misses (the ray has an
-// axis that is not parallel, whose t is finite or of the missing sign), and one
-// inside leaves the axis out, as the general test does.
+// inside the slab leaves the axis out, as the general test does, and one
+// outside leaves tmax = -inf, or tmin = +inf with the finite tmax of the axis
+// whose t cannot overflow (regular_ray sees to one), and misses.
 __device__ __forceinline__ bool slab_hit_regular(const RaySlab& r, const bool neg[3],
                                                  const float lo[3], const float hi[3],
                                                  float& tmin_out, float& tmax_out) {
@@ -341,16 +347,16 @@ __device__ __forceinline__ bool slab_hit_regular(const RaySlab& r, const bool ne
   return !(tmin > tmax) && !(tmax < 0.f);
 }
 
-// Whether slab_hit_regular serves this ray: a finite origin, and per axis a
-// finite nonzero reciprocal or a direction of exactly 0, not 0 on all three.
-// Makes the reciprocals of parallel axes +inf.
+// Whether slab_hit_regular serves this ray: an origin within the bound, per axis
+// a nonzero reciprocal that is finite or of a parallel axis, and one of them
+// within its bound.  Makes the reciprocals of parallel axes +inf.
 __device__ __forceinline__ bool regular_ray(RaySlab& r, bool neg[3]) {
   bool ok = true, some = false;
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
     const float a = fabsf(r.inv[i]);
-    ok = ok && a > 0.f && fabsf(r.o[i]) < __builtin_inff();  // false for a NaN
-    some = some || a < __builtin_inff();
+    ok = ok && a > 0.f && fabsf(r.o[i]) <= kRegularMax;  // false for a NaN
+    some = some || a <= kRegularInv;
   }
   ok = ok && some;
 #pragma unroll
@@ -436,8 +442,8 @@ __device__ __forceinline__ int trace_loop(const Packed& pk, const RaySlab& r, co
   return kTraceOk;
 }
 
-// regular: every packed child box is finite with lo <= hi (checked while
-// packing).
+// regular: every packed child box lies within +-kRegularMax with lo <= hi
+// (checked while packing).
 template <class Stack>
 __device__ __forceinline__ int trace(const Packed& pk, const float org[3], const float dir[3],
                                      Stack& stk, Hit& out, bool regular) {

@@ -4,8 +4,8 @@
 //
 // Packed tree of N triangles (dmsh_packed_bytes): inner nodes [N-1] (64 B),
 // leaves [N] (48 B), the root box (6 floats), then a word that is nonzero
-// when a box of the tree is not finite -- the traversal layout of
-// raycast.hpp, so a cast reads nothing else.
+// when a box of the tree needs the general slab test (rc::store_inner) -- the
+// traversal layout of raycast.hpp, so a cast reads nothing else.
 #pragma once
 
 #include "batch.hpp"
@@ -90,7 +90,7 @@ struct PackSrc {
 };
 
 // After a build that packed as it refit: each mesh's root box and its
-// non-finite flag into its packed buffer.
+// slab-test flag into its packed buffer.
 static __global__ __launch_bounds__(256) void k_pack_roots(uint32_t M,
                                                            const uint32_t* __restrict__ mesh2tri,
                                                            const uint32_t* __restrict__ node_off,
@@ -108,7 +108,7 @@ static __global__ __launch_bounds__(256) void k_pack_roots(uint32_t M,
   *packed_flag(dst[m], n) = nonfinite[m];
 }
 
-// The per-mesh non-finite flags into the packed buffers (after the pack).
+// The per-mesh slab-test flags into the packed buffers (after the pack).
 static __global__ __launch_bounds__(256) void k_pack_flags(uint32_t M,
                                                            const uint32_t* __restrict__ mesh2tri,
                                                            const uint64_t* __restrict__ dst,
@@ -121,7 +121,7 @@ static __global__ __launch_bounds__(256) void k_pack_flags(uint32_t M,
 }
 
 // Internal nodes of a CSR batch of trees into their packed buffers; also the
-// root boxes and a per-mesh flag for non-finite boxes.
+// root boxes and a per-mesh flag for boxes that need the general slab test.
 static __global__ __launch_bounds__(256) void k_pack_to_buffers(
     bat::BatchTrees b, uint32_t total_tri, const uint32_t* __restrict__ inner_off,
     const uint64_t* __restrict__ dst, uint32_t* __restrict__ nonfinite,

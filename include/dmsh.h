@@ -497,7 +497,8 @@ int dmsh_batch_pix2tri(void *stream, uint32_t num_mesh, uint32_t total_tri,
  * dmsh_batch_pack packs the trees of a CSR batch (as built by
  * dmsh_batch_build_trimesh3, same offsets) into one self-contained buffer
  * per mesh of dmsh_packed_bytes(N_m) bytes at device address packed[m];
- * nonfinite[m] (written) is nonzero when a box of that tree is not finite.
+ * nonfinite[m] (written) is nonzero when the tree's rays need the general slab
+ * test: a box that is inverted, not finite or beyond +-2^62, or a broken row.
  * A packed tree is all a ray-cast reads, so it is what a cache keeps.
  *
  * dmsh_cast_requests ray-casts requests[0..num_req) (a device array) into

@@ -73,3 +73,32 @@ def test_rays_without_direction(gpu, oracle):
     tri = np.arange(60, dtype=np.uint32).reshape(20, 3)
     n2w = np.diag([1.0, 1.0, 0.0, 1.0]).astype(np.float32)
     _cast_equals_oracle(gpu, oracle, tri, vtx, n2w, 16, 16)
+
+
+# in turn: rays and boxes, only the rays, only the boxes beyond what the regular
+# slab test serves; and the mesh's own boxes
+@pytest.mark.parametrize("length,far", [(2e-25, 1e20), (2e-25, 1e15), (1e-19, 1e20), (2e-25, 0)])
+def test_box_beyond_the_range_of_t(gpu, oracle, length, far):
+    """Rays so short that a box's planes lie at t = +inf, beside a parallel axis
+    whose slab they miss, in a caller's own boxes: the general test misses such
+    a box, whatever the triangles in it."""
+    size = 1e13
+    rng = np.random.default_rng(5)
+    tri, vtx = [], []
+    for k in range(40):
+        x, y, z = *rng.uniform(-size, size, 2), -1.0 - k
+        tri.append([3 * k, 3 * k + 1, 3 * k + 2])
+        vtx += [[x - size, y - size, z], [x + size, y - size, z], [x, y + size, z]]
+    tri, vtx = np.array(tri, np.uint32), np.array(vtx, np.float32)
+    bn, aabb = oracle.build_trimesh3(tri, vtx)
+    n2w = np.diag([2 * size, 2 * size, 0.5 * length, 1.0]).astype(np.float32)
+    if far:  # all leaves but every fourth
+        leaf = np.flatnonzero(bn[:, 2] == 0xFFFFFFFF)
+        aabb[leaf[np.arange(len(leaf)) % 4 != 0]] = np.array(
+            [3 * size, aabb[0, 1], -2 * far, 4 * size, aabb[0, 4], -far], np.float32)
+    dev = [torch.from_numpy(a).to(gpu) for a in (tri, vtx, bn, aabb, n2w)]
+    pix, t = Pix2Tri.by_raycasting_with_coeff(*dev, (24, 24))
+    want, want_t, _ = oracle.pix2tri(tri, vtx, bn, aabb, n2w.T.reshape(-1), 24, 24, num_threads=4)
+    assert np.array_equal(pix.cpu().numpy(), want)
+    assert np.array_equal(t.cpu().numpy().view(np.uint32), want_t.view(np.uint32))
+    assert 200 < (want != 0xFFFFFFFF).sum() < 576 and _lib.device_errors() == 0
