@@ -179,7 +179,6 @@ __device__ __forceinline__ bool walk(const float q0[2], const float q1[2], uint3
 
 struct EdgeArgs {
   const uint32_t* __restrict__ cedge2vtx;
-  uint32_t num_cedge;
   const float* __restrict__ xyz;
   uint32_t num_vtx;
   const float* __restrict__ T;  // world2pix, column-major
@@ -241,20 +240,33 @@ __device__ __forceinline__ void values_of_edge(const EdgeArgs& a, uint32_t e, ui
   });
 }
 
-static __global__ __launch_bounds__(64) void k_aa_keys(EdgeArgs a,
-                                                       unsigned long long* __restrict__ keys) {
-  const uint32_t e = (blockIdx.x * blockDim.x + threadIdx.x) / kEdgeLanes;
-  if (e < a.num_cedge)
-    keys_of_edge(a, e, threadIdx.x % kEdgeLanes, keys);
+// The contour edges of one launch: kEdgeLanes threads each, within the 2^32
+// threads that a launch may have.
+struct EdgeSlice {
+  uint32_t first, count;
+};
+constexpr uint32_t kEdgeSlice = 1u << 27;
+static_assert((uint64_t)kEdgeSlice * kEdgeLanes < (1ull << 32), "threads of a launch");
+
+// The edge of the thread's group, false past the slice's last.
+__device__ __forceinline__ bool group_edge(const EdgeSlice& es, uint32_t& e) {
+  const uint32_t i = blockIdx.x * (64u / kEdgeLanes) + threadIdx.x / kEdgeLanes;
+  e = es.first + i;
+  return i < es.count;
 }
 
-static __global__ __launch_bounds__(64) void k_aa_write(EdgeArgs a,
+static __global__ __launch_bounds__(64) void k_aa_keys(EdgeSlice es, EdgeArgs a,
+                                                       unsigned long long* __restrict__ keys) {
+  uint32_t e;
+  if (group_edge(es, e)) keys_of_edge(a, e, threadIdx.x % kEdgeLanes, keys);
+}
+
+static __global__ __launch_bounds__(64) void k_aa_write(EdgeSlice es, EdgeArgs a,
                                                         const unsigned long long* __restrict__ keys,
                                                         const float* __restrict__ vin,
                                                         float* __restrict__ vout) {
-  const uint32_t e = (blockIdx.x * blockDim.x + threadIdx.x) / kEdgeLanes;
-  if (e < a.num_cedge)
-    values_of_edge(a, e, threadIdx.x % kEdgeLanes, keys, vin, vout);
+  uint32_t e;
+  if (group_edge(es, e)) values_of_edge(a, e, threadIdx.x % kEdgeLanes, keys, vin, vout);
 }
 
 __device__ __forceinline__ void proj_jacobian_xy(const float* m, const float* p, float J[2][3]) {
@@ -307,11 +319,12 @@ __device__ __forceinline__ void bwd_of_edge(const EdgeArgs& a, uint32_t e, uint3
   }
 }
 
-static __global__ __launch_bounds__(64) void k_aa_bwd(EdgeArgs a, const float* __restrict__ val,
+static __global__ __launch_bounds__(64) void k_aa_bwd(EdgeSlice es, EdgeArgs a,
+                                                      const float* __restrict__ val,
                                                       const float* __restrict__ dldw,
                                                       float* __restrict__ dldw_vtx2xyz) {
-  const uint32_t e = (blockIdx.x * blockDim.x + threadIdx.x) / kEdgeLanes;
-  if (e < a.num_cedge) bwd_of_edge(a, e, threadIdx.x % kEdgeLanes, val, dldw, dldw_vtx2xyz);
+  uint32_t e;
+  if (group_edge(es, e)) bwd_of_edge(a, e, threadIdx.x % kEdgeLanes, val, dldw, dldw_vtx2xyz);
 }
 
 // ---------------------------------------------------------------------------

@@ -155,41 +155,40 @@ static __global__ __launch_bounds__(256) void k_batch_aa_init(
 // Calls fn(the mesh's args, its contour edge, lane of the group, its first
 // pixel, its first vertex) for the group's contour edge of the batch.
 template <class Fn>
-__device__ __forceinline__ void with_cedge(const Images& b, Fn fn) {
-  const uint32_t g = (blockIdx.x * blockDim.x + threadIdx.x) / aa::kEdgeLanes;
-  if (g >= b.num_cedge || *b.bad != 0u) return;
+__device__ __forceinline__ void with_cedge(const aa::EdgeSlice& es, const Images& b, Fn fn) {
+  uint32_t g;
+  if (!aa::group_edge(es, g) || *b.bad != 0u) return;
   const uint32_t m = bat::find_segment(b.mesh2cedge, b.M, g);
   const uint32_t p0 = b.mesh2pix[m], n = b.mesh2pix[m + 1] - p0, w = b.mesh2width[m];
   if (n == 0u) return;
   const uint32_t c0 = b.mesh2cedge[m], v0 = b.mesh2vtx[m];
-  const aa::EdgeArgs a{b.cedge2vtx + (size_t)c0 * 2, b.mesh2cedge[m + 1] - c0,
-                       b.xyz + (size_t)v0 * 3,       b.mesh2vtx[m + 1] - v0,
-                       b.w2p + (size_t)m * 16,       w,
-                       n / w,                        b.pix2tri + p0,
-                       b.err};
+  const aa::EdgeArgs a{b.cedge2vtx + (size_t)c0 * 2, b.xyz + (size_t)v0 * 3,
+                       b.mesh2vtx[m + 1] - v0,       b.w2p + (size_t)m * 16,
+                       w,                            n / w,
+                       b.pix2tri + p0,               b.err};
   fn(a, g - c0, threadIdx.x % aa::kEdgeLanes, p0, v0);
 }
 
 static __global__ __launch_bounds__(64) void k_batch_aa_keys(
-    Images b, unsigned long long* __restrict__ keys) {
-  with_cedge(b, [&](const aa::EdgeArgs& a, uint32_t e, uint32_t sub, uint32_t p0, uint32_t) {
+    aa::EdgeSlice es, Images b, unsigned long long* __restrict__ keys) {
+  with_cedge(es, b, [&](const aa::EdgeArgs& a, uint32_t e, uint32_t sub, uint32_t p0, uint32_t) {
     aa::keys_of_edge(a, e, sub, keys + p0);
   });
 }
 
 static __global__ __launch_bounds__(64) void k_batch_aa_write(
-    Images b, const unsigned long long* __restrict__ keys, const float* __restrict__ vin,
-    float* __restrict__ vout) {
-  with_cedge(b, [&](const aa::EdgeArgs& a, uint32_t e, uint32_t sub, uint32_t p0, uint32_t) {
+    aa::EdgeSlice es, Images b, const unsigned long long* __restrict__ keys,
+    const float* __restrict__ vin, float* __restrict__ vout) {
+  with_cedge(es, b, [&](const aa::EdgeArgs& a, uint32_t e, uint32_t sub, uint32_t p0, uint32_t) {
     aa::values_of_edge(a, e, sub, keys + p0, vin + p0, vout + p0);
   });
 }
 
-static __global__ __launch_bounds__(64) void k_batch_aa_bwd(Images b,
+static __global__ __launch_bounds__(64) void k_batch_aa_bwd(aa::EdgeSlice es, Images b,
                                                             const float* __restrict__ val,
                                                             const float* __restrict__ dldw,
                                                             float* __restrict__ dldw_vtx2xyz) {
-  with_cedge(b, [&](const aa::EdgeArgs& a, uint32_t e, uint32_t sub, uint32_t p0, uint32_t v0) {
+  with_cedge(es, b, [&](const aa::EdgeArgs& a, uint32_t e, uint32_t sub, uint32_t p0, uint32_t v0) {
     aa::bwd_of_edge(a, e, sub, val + p0, dldw + p0, dldw_vtx2xyz + (size_t)v0 * 3);
   });
 }

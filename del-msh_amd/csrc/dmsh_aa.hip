@@ -14,9 +14,19 @@ struct ContourLayout {
   uint32_t* block_count;
 };
 
-// blocks of 64 threads, kEdgeLanes an edge
-inline uint32_t edge_blocks(uint32_t num_cedge) {
-  return ceil_div(num_cedge, 64u / aa::kEdgeLanes);
+// Launches a kernel over num_cedge contour edges in blocks of 64 threads,
+// kEdgeLanes an edge.
+template <typename... KArgs, typename... Args>
+int launch_edges(const char* label, void (*kernel)(aa::EdgeSlice, KArgs...), uint32_t num_cedge,
+                 hipStream_t s, const Args&... args) {
+  int st = DMSH_OK;
+  for (aa::EdgeSlice es{0u, 0u}; st == DMSH_OK && es.first < num_cedge; es.first += es.count) {
+    es.count = std::min(num_cedge - es.first, aa::kEdgeSlice);
+    launch(label, kernel, dim3(ceil_div(es.count, 64u / aa::kEdgeLanes)), dim3(64), 0, s, es,
+           args...);
+    st = launch_status();
+  }
+  return st;
 }
 
 inline uint32_t contour_blocks(uint32_t num_edge) { return ceil_div(num_edge, 256); }
@@ -127,13 +137,11 @@ int dmsh_antialias_fwd(void* stream, uint32_t num_cedge, const uint32_t* cedge2v
                      dim3(256), 0, s, keys, num_pix);
   int st = launch_status();
   if (st != DMSH_OK) return st;
-  aa::EdgeArgs ea{cedge2vtx, num_cedge, vtx2xyz, num_vtx, transform_world2pix,
-                  img_w, img_h, pix2tri, err};
-  launch("k_aa_keys", aa::k_aa_keys, dim3(edge_blocks(num_cedge)), dim3(64), 0, s, ea, keys);
-  if ((st = launch_status()) != DMSH_OK) return st;
-  launch("k_aa_write", aa::k_aa_write, dim3(edge_blocks(num_cedge)), dim3(64), 0, s, ea, keys,
-                     pix2vin, pix2vout);
-  return launch_status();
+  const aa::EdgeArgs ea{cedge2vtx, vtx2xyz, num_vtx, transform_world2pix,
+                        img_w, img_h, pix2tri, err};
+  st = launch_edges("k_aa_keys", aa::k_aa_keys, num_cedge, s, ea, keys);
+  if (st != DMSH_OK) return st;
+  return launch_edges("k_aa_write", aa::k_aa_write, num_cedge, s, ea, keys, pix2vin, pix2vout);
 }
 
 int dmsh_antialias_bwd(void* stream, uint32_t num_cedge, const uint32_t* cedge2vtx,
@@ -148,11 +156,10 @@ int dmsh_antialias_bwd(void* stream, uint32_t num_cedge, const uint32_t* cedge2v
     return DMSH_ERR_INVALID;
   uint32_t* err = device_error_word();
   if (!err) return DMSH_ERR_HIP;
-  aa::EdgeArgs ea{cedge2vtx, num_cedge, vtx2xyz, num_vtx, transform_world2pix,
-                  img_w, img_h, pix2tri, err};
-  launch("k_aa_bwd", aa::k_aa_bwd, dim3(edge_blocks(num_cedge)), dim3(64), 0, as_stream(stream),
-                     ea, pix2val, dldw_pix2val, dldw_vtx2xyz);
-  return launch_status();
+  const aa::EdgeArgs ea{cedge2vtx, vtx2xyz, num_vtx, transform_world2pix,
+                        img_w, img_h, pix2tri, err};
+  return launch_edges("k_aa_bwd", aa::k_aa_bwd, num_cedge, as_stream(stream), ea, pix2val,
+                      dldw_pix2val, dldw_vtx2xyz);
 }
 
 size_t dmsh_batch_contour_workspace_bytes(uint32_t num_mesh, uint32_t total_edge) {
@@ -236,12 +243,11 @@ int dmsh_batch_antialias_fwd(void* stream, uint32_t num_mesh, uint32_t total_vtx
          total_vtx, total_pix, L.keys, (uint64_t)total_pix);
   int st = launch_status();
   if (st != DMSH_OK) return st;
-  launch("k_batch_aa_keys", baa::k_batch_aa_keys, dim3(edge_blocks(num_cedge)), dim3(64), 0, s, b,
-         L.keys);
-  if ((st = launch_status()) != DMSH_OK) return st;
-  launch("k_batch_aa_write", baa::k_batch_aa_write, dim3(edge_blocks(num_cedge)), dim3(64), 0, s,
-         b, L.keys, pix2vin, pix2vout);
-  return launch_status();
+  if ((st = launch_edges("k_batch_aa_keys", baa::k_batch_aa_keys, num_cedge, s, b, L.keys)) !=
+      DMSH_OK)
+    return st;
+  return launch_edges("k_batch_aa_write", baa::k_batch_aa_write, num_cedge, s, b, L.keys, pix2vin,
+                      pix2vout);
 }
 
 int dmsh_batch_antialias_bwd(void* stream, uint32_t num_mesh, uint32_t total_vtx,
@@ -269,9 +275,8 @@ int dmsh_batch_antialias_bwd(void* stream, uint32_t num_mesh, uint32_t total_vtx
          total_pix, L.keys, (uint64_t)0);
   int st = launch_status();
   if (st != DMSH_OK) return st;
-  launch("k_batch_aa_bwd", baa::k_batch_aa_bwd, dim3(edge_blocks(num_cedge)), dim3(64), 0, s, b,
-         pix2val, dldw_pix2val, dldw_vtx2xyz);
-  return launch_status();
+  return launch_edges("k_batch_aa_bwd", baa::k_batch_aa_bwd, num_cedge, s, b, pix2val,
+                      dldw_pix2val, dldw_vtx2xyz);
 }
 
 }  // extern "C"

@@ -7,6 +7,7 @@ import pytest
 import torch
 
 from del_msh_dlpack import _lib
+import del_msh_dlpack.Batched.torch as Batched
 import del_msh_dlpack.DifferentiableAntialias.torch as DifferentiableAntialias
 
 pytestmark = pytest.mark.gpu
@@ -49,4 +50,41 @@ def test_walks_equal_the_serial_walk(gpu, oracle, seed, cover):
     # addition is off by 2^-24 of a partial sum, and those stay within a few
     # times the largest gradient
     assert np.abs(got - want).max() <= 480 * 2.0 ** -24 * 4 * np.abs(want).max()
+    assert _lib.device_errors() == 0
+
+
+def test_edges_past_one_launch(gpu):
+    """More edges than a launch has groups of lanes: the first and the last ones
+    are real, those between have a vertex that is not finite and are skipped."""
+    rng = np.random.default_rng(2)
+    vtx, edge = _edges(rng)
+    skipped = len(vtx) - 1
+    assert not np.isfinite(vtx[skipped]).all()
+    g = lambda a: torch.from_numpy(a).to(gpu)
+    many = torch.full((2 ** 28 + 3, 2), skipped, dtype=torch.int32, device=gpu)
+    half = len(edge) // 2
+    many[:half] = g(edge[:half].view(np.int32))
+    many[half - len(edge):] = g(edge[half:].view(np.int32))
+    many = many.view(torch.uint32)
+    pix = g(np.where(rng.random((H, W)) < 0.8, 3, 0xFFFFFFFF).astype(np.uint32))
+    val = g(rng.random((H, W), dtype=np.float32))
+    dldw = g(rng.normal(size=(H, W)).astype(np.float32))
+    eye, v = torch.eye(4, device=gpu), g(vtx)
+    want = DifferentiableAntialias.antialias(g(edge), v, eye, pix, val)
+    assert not torch.equal(want, val)
+    assert torch.equal(DifferentiableAntialias.antialias(many, v, eye, pix, val), want)
+    want_grad = DifferentiableAntialias.bwd_antialias(g(edge), v, eye, val, dldw, pix)
+    grad = DifferentiableAntialias.bwd_antialias(many, v, eye, val, dldw, pix)
+    # the bound of the test above
+    bound = 480 * 2.0 ** -24 * 4 * float(want_grad.abs().max())
+    assert float((grad - want_grad).abs().max()) <= bound
+    # and as a batch of one mesh with an image of its own
+    tri = torch.zeros((1, 3), dtype=torch.uint32, device=gpu)
+    sb = Batched.SilhouetteBatch([0, 1], [0, len(vtx)], tri, v, [0, W * H], [W],
+                                 torch.eye(4)[None])
+    sb.world2pix[0] = eye
+    hits = {"pix2tri": pix.view(-1), "occ": val.view(-1), "cedges": [many]}
+    assert torch.equal(sb.images(v, hits), want.view(-1))
+    grad = sb.vertex_gradient(v, hits, dldw.view(-1))
+    assert float((grad - want_grad).abs().max()) <= bound
     assert _lib.device_errors() == 0
