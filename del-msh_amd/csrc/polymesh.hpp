@@ -281,9 +281,12 @@ static __global__ __launch_bounds__(256) void k_query_codes(uint32_t num_wtx,
   idx[w] = w;
 }
 
+// Two floats read at once from where a caller's array of floats lies.
+using UnalignedPair = float __attribute__((ext_vector_type(2), aligned(4)));
+
 __device__ __forceinline__ bool box_holds(const float* __restrict__ b, const V3& q) {
-  const float2* p = reinterpret_cast<const float2*>(b);
-  const float2 u = p[0], v = p[1], w = p[2];  // lo.x lo.y | lo.z hi.x | hi.y hi.z
+  const UnalignedPair* p = reinterpret_cast<const UnalignedPair*>(b);
+  const UnalignedPair u = p[0], v = p[1], w = p[2];  // lo.x lo.y | lo.z hi.x | hi.y hi.z
   return u.x <= q.x && q.x <= v.y && u.y <= q.y && q.y <= w.x && v.x <= q.z && q.z <= w.y;
 }
 

@@ -6,7 +6,7 @@ import numpy as np
 import pytest
 import torch
 
-from del_msh_dlpack import _lib
+from del_msh_dlpack import _lib, primitives
 import del_msh_dlpack.PolyhedronMesh.torch as PolyhedronMesh
 
 pytestmark = pytest.mark.gpu
@@ -40,3 +40,25 @@ def test_deep_walks(gpu, oracle, copies, flip, vdim):
     want_val = oracle.polyhedron_interpolate(off, iv, val, want, want_par)
     assert np.array_equal(got.cpu().numpy().view(np.uint32), want_val.view(np.uint32))
     assert _lib.device_errors() == 0
+
+
+def test_arrays_at_a_four_byte_boundary(gpu, oracle):
+    """The tree and the points as slices of larger buffers, aligned to their
+    elements and to nothing more."""
+    off, iv, x = primitives.mixed_hex_grid(4, 4, 4, seed=2)
+    rng = np.random.default_rng(0)
+    q = rng.uniform(-0.2, 4.2, (500, 3)).astype(np.float32)
+    bn, _ = oracle.build_points(oracle.polyhedron_elem2center(off, iv, x))
+    aabb = oracle.polyhedron_refit(bn, off, iv, x)
+
+    def shifted(a):
+        b = torch.empty(a.size + 1, dtype=torch.from_numpy(a).dtype, device=gpu)[1:].view(a.shape)
+        assert b.data_ptr() % 8 == 4 and b.is_contiguous()
+        return b.copy_(torch.from_numpy(a))
+
+    elem, par = PolyhedronMesh.search_elem_contain_points(
+        *map(shifted, (off, iv, x.astype(np.float32), bn, aabb, q)))
+    want, want_par = oracle.polyhedron_search(off, iv, x, bn, aabb, q)
+    assert np.array_equal(elem.cpu().numpy(), want)
+    assert np.array_equal(par.cpu().numpy().view(np.uint32), want_par.view(np.uint32))
+    assert (want != 0xFFFFFFFF).sum() > 300 and _lib.device_errors() == 0
