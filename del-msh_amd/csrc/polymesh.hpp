@@ -259,25 +259,46 @@ struct MeshView {
   const float* xyz;
 };
 
-// 30-bit Morton code, less its lowest `shift` bits, of each query point in the
-// unit-cube fit of the root box (aabb row 0), and the identity permutation: sorting by these codes puts
-// nearby queries in one wave, so its lanes walk the same branches and test
-// the same elements.  Only the processing order changes, not any result.
+// Code of `bits` bits of each query point in the root box (aabb row 0), and the
+// identity permutation: sorting by these codes puts nearby queries in one wave,
+// so its lanes walk the same branches and test the same elements.  Only the
+// processing order changes, not any result.
+// The code is the path to the point's cell as the box is halved, at level l
+// along every axis longer than 2^-l of the longest: a Morton code without the
+// bits that are 0 in the whole box.  (With those bits in it, 16 bits divided a
+// plate into 2048 cells and a wire into 32, and 2^20 points in plates, rods and
+// wires of 50,000 to 240,000 elements took 4 to 24 % longer than with 30 bits.)
 static __global__ __launch_bounds__(256) void k_query_codes(uint32_t num_wtx,
                                                             const float* __restrict__ wtx2xyz,
                                                             const float* __restrict__ aabb,
-                                                            uint32_t shift,
+                                                            uint32_t bits,
                                                             uint32_t* __restrict__ keys,
                                                             uint32_t* __restrict__ idx) {
+  constexpr uint32_t kLevels = 24;
   const uint32_t w = blockIdx.x * blockDim.x + threadIdx.x;
   if (w >= num_wtx) return;
-  float ext = fmax_sel(fmax_sel(aabb[3] - aabb[0], aabb[4] - aabb[1]), aabb[5] - aabb[2]);
+  const float ext = fmax_sel(fmax_sel(aabb[3] - aabb[0], aabb[4] - aabb[1]), aabb[5] - aabb[2]);
   const float s = ext > 0.f ? 1.f / ext : 1.f;
-  float T[16] = {s, 0.f, 0.f, 0.f, 0.f, s, 0.f, 0.f, 0.f, 0.f, s, 0.f,
-                 -aabb[0] * s, -aabb[1] * s, -aabb[2] * s, 1.f};
-  keys[w] = morton3_transformed<uint32_t>(T, wtx2xyz[(size_t)w * 3], wtx2xyz[(size_t)w * 3 + 1],
-                                          wtx2xyz[(size_t)w * 3 + 2]) >>
-            shift;
+  uint32_t cell[3], from[3];  // the point's cell at the last level; the first level along an axis
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const float x = (wtx2xyz[(size_t)w * 3 + d] - aabb[d]) * s;
+    cell[d] = (uint32_t)(fminf(fmaxf(x, 0.f), 1.f - 0x1p-24f) * 0x1p24f);
+    // r in (2^-l, 2^(1 - l)] has, made a little smaller, the exponent of 2^-l
+    const float r = (aabb[3 + d] - aabb[d]) * s * (1.f - 0x1p-20f);
+    const int l = 127 - (int)((__float_as_uint(r) >> 23) & 255u);
+    from[d] = __builtin_amdgcn_readfirstlane(l < 1 ? 1u : (uint32_t)l);
+  }
+  uint32_t code = 0u, n = 0u;
+  for (uint32_t l = 1; l <= kLevels && n < bits; ++l) {
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      if (l < from[d] || n == bits) continue;
+      code = code << 1 | ((cell[d] >> (kLevels - l)) & 1u);
+      ++n;
+    }
+  }
+  keys[w] = code;
   idx[w] = w;
 }
 

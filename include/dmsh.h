@@ -691,8 +691,8 @@ int dmsh_bvhnode2aabb_polyhedron(void *stream, uint32_t num_bvhnode, const uint3
                                  const float *vtx2xyz, float *bvhnode2aabb, void *ws,
                                  size_t ws_bytes);
 /* ws (optional, dmsh_polyhedron_search_workspace_bytes(num_wtx)): with it,
- * sets of 65536 or more query points are searched in the Morton order of the
- * points in the root box (only the order of work changes, not any result);
+ * sets of 65536 or more query points are searched in the order of their cells
+ * in the root box (only the order of work changes, not any result);
  * ws == NULL searches in the given order. */
 size_t dmsh_polyhedron_search_workspace_bytes(uint32_t num_wtx);
 int dmsh_polyhedron_search_elem_contain_points(void *stream, uint32_t num_elem,

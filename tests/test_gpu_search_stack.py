@@ -62,3 +62,26 @@ def test_arrays_at_a_four_byte_boundary(gpu, oracle):
     assert np.array_equal(elem.cpu().numpy(), want)
     assert np.array_equal(par.cpu().numpy().view(np.uint32), want_par.view(np.uint32))
     assert (want != 0xFFFFFFFF).sum() > 300 and _lib.device_errors() == 0
+
+
+@pytest.mark.parametrize("dims", [(12, 12, 12), (60, 40, 1), (1, 900, 1), (3, 1, 500), (1, 1, 1)])
+@pytest.mark.parametrize("scale", [1.0, 1e-30, 1e30, 0.0])
+def test_order_of_queries_in_boxes_of_every_shape(gpu, oracle, dims, scale):
+    """Queries enough to be put in order: in cubes, plates, rods and a mesh that
+    is drawn together in a point, inside, outside and not finite."""
+    off, iv, x = primitives.mixed_hex_grid(*dims, seed=3)
+    x = (x * scale).astype(np.float32)
+    rng = np.random.default_rng(1)
+    q = (rng.uniform(-0.1, 1.1, (1000, 3)) * np.array(dims) * scale).astype(np.float32)
+    q[::97] = np.nan
+    q[::101, 1] = np.inf
+    bn, _ = oracle.build_points(oracle.polyhedron_elem2center(off, iv, x))
+    aabb = oracle.polyhedron_refit(bn, off, iv, x)
+    want, want_par = oracle.polyhedron_search(off, iv, x, bn, aabb, q)
+    assert scale != 1.0 or (want != 0xFFFFFFFF).sum() > 300
+    which = rng.permutation(np.arange(70000) % 1000)
+    elem, par = PolyhedronMesh.search_elem_contain_points(
+        *(torch.from_numpy(a).to(gpu) for a in (off, iv, x, bn, aabb, q[which])))
+    assert np.array_equal(elem.cpu().numpy(), want[which])
+    assert np.array_equal(par.cpu().numpy().view(np.uint32), want_par[which].view(np.uint32))
+    assert _lib.device_errors() == 0
