@@ -133,7 +133,7 @@ void launch_cast(hipStream_t s, uint32_t max_tiles, const Src& src, const rc::Ca
                  uint32_t* pix2tri, float* pix2t) {
   auto go = [&](auto kernel, const char* label, int frames, uint32_t w) {
     const uint32_t per_cu =
-        std::min((uint32_t)g_batch_wgs_per_cu.load(), rc::resident_waves(frames));
+        std::min((uint32_t)g_batch_wgs_per_cu.load(), rc::resident_waves(frames, (int)w));
     const uint32_t waves = std::min(rc::cast_waves(max_tiles), (uint32_t)device_cu_count() * per_cu);
     launch(label, kernel, dim3(ceil_div(waves, w)), dim3(64 * w), 0, s, src, st, pix2tri, pix2t);
   };

@@ -550,12 +550,17 @@ inline uint32_t max_tiles(uint64_t num_pix, uint64_t images) {
 // Waves of a launch over at most `tiles` tiles, and the words of spill area
 // each of them owns.
 inline uint32_t cast_waves(uint32_t tiles) { return tiles < kMaxCastWaves ? tiles : kMaxCastWaves; }
-// Waves per CU that fit its 160 KB of LDS with S frames a lane (of the 32 that
-// their registers allow): a wave of the grid that starts late holds its fixed
-// share of the tiles back.
-constexpr uint32_t resident_waves(int S) {
-  return 160u * 1024u / (uint32_t)(S * 512) < 32u ? 160u * 1024u / (uint32_t)(S * 512) : 32u;
+// Waves per CU in workgroups of W that fit its 160 KB of LDS with S frames a
+// lane (of the 32 waves that their registers allow).  A grid of more would start
+// the last workgroups when others have ended, and those with their own first
+// tiles.
+constexpr uint32_t resident_waves(int S, int W) {
+  const uint32_t by_lds = 160u * 1024u / (uint32_t)(S * 512 * W), by_regs = 32u / (uint32_t)W;
+  return (by_lds < by_regs ? by_lds : by_regs) * (uint32_t)W;
 }
+static_assert(resident_waves(12, 1) == 26 && resident_waves(12, 2) == 26 &&
+                  resident_waves(12, 4) == 24 && resident_waves(32, 4) == 8,
+              "whole workgroups");
 constexpr size_t kSpillPerWave = (size_t)kSpillFrames * 64;
 
 struct CastState {
