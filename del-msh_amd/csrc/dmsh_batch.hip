@@ -139,6 +139,7 @@ void launch_cast(hipStream_t s, uint32_t max_tiles, const Src& src, const rc::Ca
   };
   auto with_waves = [&](auto frames) {
     constexpr int S = decltype(frames)::value;
+    static_assert(S >= rc::kMinFrames, "fewer frames, more waves than the spill area is for");
     switch (g_batch_cast_waves.load()) {
       case 2: go(Cast<S, 2>::kernel(), Cast<S, 2>::label(), S, 2u); break;
       case 4: go(Cast<S, 4>::kernel(), Cast<S, 4>::label(), S, 4u); break;
@@ -150,7 +151,7 @@ void launch_cast(hipStream_t s, uint32_t max_tiles, const Src& src, const rc::Ca
     case 20: with_waves(std::integral_constant<int, 20>()); break;
     case 24: with_waves(std::integral_constant<int, 24>()); break;
     case 32: with_waves(std::integral_constant<int, 32>()); break;
-        default: with_waves(std::integral_constant<int, 12>()); break;
+    default: with_waves(std::integral_constant<int, 12>()); break;
   }
 }
 

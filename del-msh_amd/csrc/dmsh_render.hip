@@ -42,6 +42,7 @@ inline bool carve_cast(Arena& a, uint32_t num_tri, uint32_t img_w, uint32_t img_
 template <int S, int W>
 void launch_pix2tri(hipStream_t s, const rc::ImageSrc& src, const rc::CastState& st,
                     uint32_t* pix2tri, float* pix2t) {
+  static_assert(S >= rc::kMinFrames, "fewer frames, more waves than the spill area is for");
   const uint32_t waves = std::min(rc::cast_waves(src.tiles),
                                   (uint32_t)device_cu_count() * rc::resident_waves(S, W));
   launch("k_pix2tri", (rc::k_pix2tri<S, W>), dim3(ceil_div(waves, W)), dim3(64 * W), 0, s, src, st, pix2tri, pix2t);

@@ -47,7 +47,6 @@ constexpr uint32_t kIndexMask = 0x3FFFFFFFu;
 constexpr uint32_t kMaxTri = 0x3FFFFFFFu;    // child refs hold 30-bit indices
 constexpr int kSpillFrames = 64;                // spilled frames per lane
 constexpr uint32_t kDeepFrames = 64u * kSpillFrames;  // a lone lane's frames
-constexpr uint32_t kMaxCastWaves = 8192;        // 32 waves on each of 256 CUs
 constexpr uint32_t kXcds = 8;
 constexpr uint32_t kCastCounts = 32 + 32 * kXcds;  // words of CastState::counts
 
@@ -547,9 +546,6 @@ inline uint32_t max_tiles(uint64_t num_pix, uint64_t images) {
   const uint64_t t = num_pix * 9u / 64u + 2u * images + 1u;
   return t < num_pix ? (uint32_t)t : (uint32_t)num_pix;
 }
-// Waves of a launch over at most `tiles` tiles, and the words of spill area
-// each of them owns.
-inline uint32_t cast_waves(uint32_t tiles) { return tiles < kMaxCastWaves ? tiles : kMaxCastWaves; }
 // Waves per CU in workgroups of W that fit its 160 KB of LDS with S frames a
 // lane (of the 32 waves that their registers allow).  A grid of more would start
 // the last workgroups when others have ended, and those with their own first
@@ -561,6 +557,12 @@ constexpr uint32_t resident_waves(int S, int W) {
 static_assert(resident_waves(12, 1) == 26 && resident_waves(12, 2) == 26 &&
                   resident_waves(12, 4) == 24 && resident_waves(32, 4) == 8,
               "whole workgroups");
+// Waves of a launch over at most `tiles` tiles with any number of frames, and
+// the words of spill area each of them owns: 32 KB, so 208 MiB from 6656 tiles
+// (a 649 x 649 image) on.
+constexpr int kMinFrames = 12;
+constexpr uint32_t kMaxCastWaves = 256u * resident_waves(kMinFrames, 1);
+inline uint32_t cast_waves(uint32_t tiles) { return tiles < kMaxCastWaves ? tiles : kMaxCastWaves; }
 constexpr size_t kSpillPerWave = (size_t)kSpillFrames * 64;
 
 struct CastState {

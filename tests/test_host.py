@@ -160,3 +160,21 @@ def test_tuning_keys_accept_and_reject_without_a_gpu():
         finally:
             assert L.dmsh_set_tuning(key, old) == 0
     assert L.dmsh_set_tuning(b"refit.no_such_key", 1) != 0
+
+
+def test_cast_workspaces_hold_the_waves_that_a_launch_can_start():
+    """32 KB of stack a wave, for 26 waves (12 frames a lane) on each of 256 CUs,
+    whatever the image; one wave a tile in small images; never less for a larger
+    image, as one workspace serves images of several sizes."""
+    L = _lib.lib()
+    wave, most, slack = 32 << 10, 26 * 256 * (32 << 10), 1 << 17
+    sizes = [(1, 1), (8, 8), (64, 64), (256, 256), (512, 512), (649, 649), (2048, 2048),
+             (1, 1 << 20), (1 << 14, 1 << 14)]
+    for f in (lambda w, h: L.dmsh_pix2tri_workspace_bytes(0, w, h),
+              lambda w, h: L.dmsh_batch_pix2tri_workspace_bytes(1, 0, w * h),
+              lambda w, h: L.dmsh_cast_requests_workspace_bytes(1, w * h)):
+        for w, h in sizes:
+            tiles = -(-w // 8) * -(-h // 8)
+            assert min(tiles * wave, most) <= f(w, h) <= most + slack, (w, h)
+        assert f(8, 8) <= 16 * wave + slack
+        assert all(f(n, n) <= f(n + 1, n + 1) for n in range(1, 1000, 7))
