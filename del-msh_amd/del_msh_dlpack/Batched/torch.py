@@ -84,7 +84,7 @@ class Pipeline:
             self.pix2tri = torch.empty(max(self.total_pix, 1), dtype=torch.uint32, device=dev)
             self.pix2t = (torch.empty(max(self.total_pix, 1), dtype=torch.float32, device=dev)
                           if with_coeff else None)
-            self.ws_cast = _lib.workspace(
+            self.ws_cast = None if packed else _lib.workspace(
                 L.dmsh_batch_pix2tri_workspace_bytes(self.num_mesh, self.total_tri,
                                                      self.total_pix), dev)
         self.packed = bool(packed)

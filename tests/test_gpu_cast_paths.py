@@ -5,7 +5,8 @@ import numpy as np
 import pytest
 import torch
 
-from del_msh_dlpack import _lib
+from del_msh_dlpack import _lib, primitives
+import del_msh_dlpack.Batched.torch as Batched
 import del_msh_dlpack.Pix2Tri.torch as Pix2Tri
 
 pytestmark = pytest.mark.gpu
@@ -102,3 +103,25 @@ def test_box_beyond_the_range_of_t(gpu, oracle, length, far):
     assert np.array_equal(pix.cpu().numpy(), want)
     assert np.array_equal(t.cpu().numpy().view(np.uint32), want_t.view(np.uint32))
     assert 200 < (want != 0xFFFFFFFF).sum() < 576 and _lib.device_errors() == 0
+
+
+def test_packed_pipeline_holds_one_cast_workspace(gpu):
+    """A pipeline that casts from packed buffers keeps the workspace of that cast
+    and not the unpacked cast's as well."""
+    b = primitives.batch_meshes(4, seed=1, tri_range=(32, 200), pix_range=(500 ** 2, 600 ** 2))
+    g = lambda a: torch.from_numpy(a).to(gpu)
+    tri, vtx = g(b["tri2vtx"]), g(b["vtx2xyz"])
+    need = _lib.lib().dmsh_cast_requests_workspace_bytes(4, int(b["mesh2pix"][-1]))
+    assert need > 100 << 20
+    torch.cuda.synchronize()
+    before = torch.cuda.memory_allocated(gpu)
+    p = Batched.Pipeline(b["mesh2tri"], b["mesh2vtx"], tri, vtx, b["mesh2pix"], b["mesh2width"],
+                         torch.from_numpy(b["ndc2world"]), packed=True)
+    assert torch.cuda.memory_allocated(gpu) - before < 1.5 * need
+    p.run()
+    loop = Batched.PerMeshLoop(p)
+    loop.build()
+    loop.cast()
+    assert torch.equal(p.pix2tri.view(torch.int32), loop.pix2tri.view(torch.int32))
+    assert torch.equal(p.pix2t.view(torch.int32), loop.pix2t.view(torch.int32))
+    assert _lib.device_errors() == 0
