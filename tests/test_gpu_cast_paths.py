@@ -23,24 +23,62 @@ def _cast_equals_oracle(gpu, oracle, tri, vtx, n2w, w, h):
     return want
 
 
-# 12 frames in LDS, 64 more in the spill area, then a lone lane's stack
-@pytest.mark.parametrize("sheets", [11, 13, 14, 60, 77, 79, 200])
-@pytest.mark.parametrize("size", [(8, 8), (33, 17)])
-def test_stack_beyond_lds_and_spill(gpu, oracle, sheets, size):
-    """Sheets in one Morton cell, listed far to near, put a frame on the stack
-    for every sheet."""
+def _sheets(count):
+    """Sheets in one Morton cell, listed far to near, that put a frame on the
+    stack for every sheet."""
     tri, vtx = [], []
-    for k in range(sheets):
-        z = -0.001 + k * (0.0016 / sheets)
+    for k in range(count):
+        z = -0.001 + k * (0.0016 / count)
         tri.append([len(vtx), len(vtx) + 1, len(vtx) + 2])
         vtx += [[-0.5, -0.5, z], [0.6, -0.45, z], [-0.45, 0.6, z]]
     for s in (-1.0, 1.0):
         tri.append([len(vtx), len(vtx) + 1, len(vtx) + 2])
         vtx += [[s * 4, s * 4, 0], [s * 4 + 0.01, s * 4, 0], [s * 4, s * 4 + 0.01, 0]]
-    n2w = np.diag([1.0, 1.0, 1.0, 1.0]).astype(np.float32)
-    want = _cast_equals_oracle(gpu, oracle, np.array(tri, np.uint32), np.array(vtx, np.float32),
-                               n2w, *size)
+    return np.array(tri, np.uint32), np.array(vtx, np.float32)
+
+
+# 12 frames in LDS, 64 more in the spill area, then a lone lane's stack
+@pytest.mark.parametrize("sheets", [11, 13, 14, 60, 77, 79, 200])
+@pytest.mark.parametrize("size", [(8, 8), (33, 17)])
+def test_stack_beyond_lds_and_spill(gpu, oracle, sheets, size):
+    want = _cast_equals_oracle(gpu, oracle, *_sheets(sheets), np.eye(4, dtype=np.float32), *size)
     assert (want == sheets - 1).any()
+
+
+@pytest.mark.parametrize("waves", [1, 2, 4])
+@pytest.mark.parametrize("stack", [12, 16, 32])
+def test_stacks_of_wide_workgroups(gpu, oracle, waves, stack):
+    """Waves that share a workgroup keep their frames apart, in LDS, in the spill
+    area and as lone lanes, in every cast: images whose number of tiles is no
+    multiple of the waves, rays that need 10 to 200 frames in all waves at once."""
+    meshes = [_sheets(k) for k in (10, 20, 70, 90, 200)]
+    sizes = [(41, 29), (8, 8), (57, 57), (23, 100), (64, 9)]
+    eye = np.eye(4, dtype=np.float32)
+    csr = lambda n: np.concatenate([[0], np.cumsum(n)]).astype(np.uint32)
+    m2t, m2v = csr([len(t) for t, _ in meshes]), csr([len(v) for _, v in meshes])
+    m2p = csr([w * h for w, h in sizes])
+    tri, vtx = (torch.from_numpy(np.concatenate(a)).to(gpu) for a in zip(*meshes))
+    L = _lib.lib()
+    keys = ((L.dmsh_set_tuning, L.dmsh_get_tuning, b"pix2tri.waves", waves),
+            (L.dmsh_set_tuning, L.dmsh_get_tuning, b"pix2tri.stack", stack),
+            (L.dmsh_batch_set_tuning, L.dmsh_batch_get_tuning, b"batch.cast_waves", waves),
+            (L.dmsh_batch_set_tuning, L.dmsh_batch_get_tuning, b"batch.stack", stack))
+    old = [get(key) for _, get, key, _ in keys]
+    try:
+        for put, _, key, value in keys:
+            assert put(key, value) == 0
+        want = [_cast_equals_oracle(gpu, oracle, *mesh, eye, *size)
+                for mesh, size in zip(meshes, sizes)]
+        for packed in (False, True):
+            p = Batched.Pipeline(m2t, m2v, tri, vtx, m2p, [w for w, _ in sizes],
+                                 torch.eye(4).repeat(len(sizes), 1, 1), packed=packed)
+            p.run()
+            for m, image in enumerate(want):
+                assert np.array_equal(p.mesh_image(m)[0].cpu().numpy(), image)
+    finally:
+        for (put, _, key, _), value in zip(keys, old):
+            assert put(key, value) == 0
+    assert _lib.device_errors() == 0
 
 
 @pytest.mark.parametrize("flip", [(1, 1, 1), (-1, 1, 1), (1, 1, -1)])

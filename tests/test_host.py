@@ -131,7 +131,7 @@ def test_tuning_keys_accept_and_reject_without_a_gpu():
     batch = {b"batch.sort_items": ((8, 12, 16), (0, 4, 10, 32)),
              b"batch.cast_waves": ((1, 2, 4), (0, 3, 8)),
              b"batch.sort_seg": ((0, 1), (2, -1)),
-             b"batch.stack": ((16, 20, 24, 32), (8, 17)),
+             b"batch.stack": ((12, 16, 20, 24, 32), (8, 17)),
              b"batch.treelet_grid": ((1, 1024), (0, 70000))}
     for key, (good, bad) in batch.items():
         old = L.dmsh_batch_get_tuning(key)
@@ -150,6 +150,16 @@ def test_tuning_keys_accept_and_reject_without_a_gpu():
         assert L.dmsh_set_tuning(key, 1 - old) == 0 and L.dmsh_get_tuning(key) == 1 - old
         assert L.dmsh_set_tuning(key, 2) != 0 and L.dmsh_get_tuning(key) == 1 - old
         assert L.dmsh_set_tuning(key, old) == 0
+    for key, good, bad in ((b"pix2tri.stack", (12, 16, 20, 24, 32), (8, 17)),
+                           (b"pix2tri.waves", (1, 2, 4), (0, 3, 8))):
+        old = L.dmsh_get_tuning(key)
+        try:
+            for v in good:
+                assert L.dmsh_set_tuning(key, v) == 0 and L.dmsh_get_tuning(key) == v
+            for v in bad:
+                assert L.dmsh_set_tuning(key, v) != 0 and L.dmsh_get_tuning(key) == good[-1]
+        finally:
+            assert L.dmsh_set_tuning(key, old) == 0
     for key, top in ((b"refit.climb", 2), (b"refit.compact", 1023), (b"sort.wide_tiles", 2)):
         old = L.dmsh_get_tuning(key)
         try:
