@@ -205,14 +205,6 @@ inline bool carve_req(Arena& a, uint32_t R, uint32_t num_pix, ReqLayout& L) {
   return a.ok();
 }
 
-int device_cus() {
-  int dev = 0, cus = 0;
-  if (hipGetDevice(&dev) != hipSuccess) return 256;
-  if (hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-    return 256;
-  return cus > 0 ? cus : 256;
-}
-
 }  // namespace
 
 extern "C" {

@@ -6,7 +6,6 @@
 #include "edgegrad.hpp"
 #include "raycast.hpp"
 #include "sort.hpp"
-#include "topo.hpp"
 
 using namespace dmsh;
 

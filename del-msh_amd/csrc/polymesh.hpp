@@ -37,7 +37,6 @@
 #pragma once
 
 #include "dmsh_common.hpp"
-#include "morton.hpp"
 
 namespace dmsh {
 namespace poly {

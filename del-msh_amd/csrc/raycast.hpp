@@ -55,7 +55,7 @@ constexpr uint32_t kCastCounts = 32 + 32 * kXcds;  // words of CastState::counts
 // 2 * 2^62 * 2^64 = 2^127 is below the largest float.
 constexpr float kRegularMax = 0x1p62f, kRegularInv = 0x1p64f;
 
-enum : int { kTraceOk = 0, kTraceOverflow = 1, kTraceBadIndex = 2 };
+enum : int { kTraceOk = 0, kTraceOverflow = 1 };
 
 struct alignas(16) InnerNode {
   float4 a;  // c0.lo.xyz, c0.hi.x

@@ -9,7 +9,7 @@ import torch
 from del_msh_dlpack import _lib, primitives
 import del_msh_dlpack.Batched.torch as Batched
 import del_msh_dlpack.DifferentiableAntialias.torch as DifferentiableAntialias
-from del_msh_dlpack.Edge2Vtx import contour_for_triangle_mesh
+from del_msh_dlpack.Edge2Vtx import contour_for_triangle_mesh, contour_for_triangle_mesh_into
 
 pytestmark = pytest.mark.gpu
 
@@ -169,4 +169,26 @@ def test_broken_rows_of_an_image_without_contours(gpu):
             for call in (lambda: sb.images(v, hits), lambda: sb.vertex_gradient(v, hits, dldw)):
                 with pytest.raises(RuntimeError):
                     call()
+    assert _lib.device_errors() == 0
+
+
+def test_contours_into_a_callers_buffers(gpu):
+    """contour_for_triangle_mesh_into: several meshes' contours back to back
+    without a read in between, in a workspace for the largest."""
+    m2t, m2v, tri, vtx, m2p, width, n2w = _batch(6)
+    g = lambda a: torch.from_numpy(a).to(gpu)
+    t, v = g(tri), g(vtx)
+    sb = Batched.SilhouetteBatch(m2t, m2v, t, v, m2p, width, n2w)
+    live = [m for m in range(6) if sb.edges[m][0].shape[0]]
+    size = [sb.edges[m][0].shape[0] for m in live]
+    ws = _lib.workspace(_lib.lib().dmsh_contour_workspace_bytes(max(size)), gpu)
+    count = torch.zeros(len(live), dtype=torch.uint32, device=gpu)
+    out = [torch.empty((n, 2), dtype=torch.uint32, device=gpu) for n in size]
+    args = [(t[int(m2t[m]):int(m2t[m + 1])], v[int(m2v[m]):int(m2v[m + 1])],
+             sb.world2ndc[m].T.contiguous().flatten(), *sb.edges[m]) for m in live]
+    for k, a in enumerate(args):
+        contour_for_triangle_mesh_into(*a, out[k], count[k:k + 1], ws)
+    for n, c, a in zip(count.cpu().numpy().tolist(), out, args):
+        want = contour_for_triangle_mesh(*a)
+        assert torch.equal(c[:n].view(torch.int32), want.view(torch.int32))
     assert _lib.device_errors() == 0
