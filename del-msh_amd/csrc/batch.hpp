@@ -10,8 +10,8 @@
 // topology and the treelet refit run on each segment with local indices.
 // Output rows of mesh m start at node_off[m] = sum_{j<m} (2 N_j - 1).
 //
-// The ray-cast hands 8x8 pixel tiles of all meshes to a resident grid of
-// waves through a counter per XCD, over the XCD's own contiguous run of tiles,
+// The ray-cast hands 8x8 pixel tiles of all meshes to a resident grid of waves
+// in chunks that go to the XCDs in turn, with a counter per XCD (rc::TileDeal),
 // so meshes of every size share the chip evenly and neighbouring tiles stay in
 // one L2.
 #pragma once

@@ -486,8 +486,9 @@ __device__ __forceinline__ bool fixed_type(uint8_t t) { return t == 2 || t == 3;
 // writes the tile back to the other buffer.  After s half-steps every cell at
 // least s cells inside the loaded region holds exactly the value the global
 // iteration gives, so the tile itself (K cells inside) is exact after up to
-// K half-steps.  Launches alternate between two buffers because tiles read
-// each other's cells as halo.
+// K half-steps.  A launch reads one buffer and writes another because tiles read
+// each other's cells as halo; the launches alternate between two, and an odd
+// number of three or more takes a third, so that the last ends in the caller's.
 constexpr int kSmoothK = 16;
 constexpr int kSmoothTR = 32;
 constexpr int kSmoothTC = 64;

@@ -10,6 +10,8 @@ start at mesh2node[m] = sum_{j<m} (2 N_j - 1).
 
 from __future__ import annotations
 
+import operator
+
 import numpy as np
 import torch
 
@@ -388,11 +390,13 @@ class _Parts:
     memory; the buffer is then no longer what the list holds."""
 
     def __init__(self, tensors):
-        self.own = [(t, t.data_ptr()) for t in tensors]
+        self.own = list(tensors)
+        self.at = list(map(torch.Tensor.data_ptr, self.own))
 
     def are(self, tensors) -> bool:
-        return len(tensors) == len(self.own) and all(
-            t is own and t.data_ptr() == at for t, (own, at) in zip(tensors, self.own))
+        # (asked several times a step, with the GPU waiting)
+        return (len(tensors) == len(self.own) and all(map(operator.is_, tensors, self.own))
+                and list(map(torch.Tensor.data_ptr, tensors)) == self.at)
 
 
 class _ContourEdges(list):
@@ -400,7 +404,8 @@ class _ContourEdges(list):
     (mesh m's are rows mesh2cedge[m] .. mesh2cedge[m+1])."""
 
     def __init__(self, cedge2vtx: torch.Tensor, mesh2cedge: torch.Tensor, offsets):
-        super().__init__(cedge2vtx[a:b] for a, b in zip(offsets, offsets[1:]))
+        super().__init__(torch.split_with_sizes(
+            cedge2vtx[: offsets[-1]], [b - a for a, b in zip(offsets, offsets[1:])]))
         self.parts = _Parts(self)
         self.batch = (cedge2vtx, mesh2cedge, offsets)
 

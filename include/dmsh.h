@@ -462,7 +462,8 @@ int dmsh_batch_antialias_bwd(void *stream, uint32_t num_mesh, uint32_t total_vtx
  * cast with transforms_ndc2world + 16 m (column-major).
  * Tuning keys (results do not depend on them): "batch.stack" (12, 16, 20,
  * 24, 32; default 12),
- * "batch.wgs_per_cu" (persistent ray-cast workgroups per CU, 1..64),
+ * "batch.wgs_per_cu" (persistent ray-cast waves per CU, 1..64; at most those
+ * whose frames fit its LDS start, 26 with 12 frames; default 32),
  * "batch.treelet_grid" (refit workgroups, 1..65536),
  * "batch.sort_items" (a digit pass's tile in 256 elements: 8, 12, 16),
  * "batch.cast_waves" (waves per ray-cast workgroup: 1, 2, 4),
