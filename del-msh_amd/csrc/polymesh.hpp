@@ -400,7 +400,7 @@ __device__ __forceinline__ uint32_t search_climb(const MeshView& m,
 // then test their elements together: the Newton solves are most of the work,
 // and in a loop that did whatever each lane was at they ran for a few lanes at
 // a time.  A node's children are read together, rows and boxes, so a level
-// costs one round trip.  2^20 points in 66 000 mixed elements: 1467 -> 844 us.
+// costs one round trip.  2^20 points in 52,000 mixed elements: 1467 -> 729 us.
 constexpr int kSearchFrames = 32;
 constexpr int kSearchThreads = 256;
 
