@@ -37,8 +37,8 @@ def _sheets(count):
     return np.array(tri, np.uint32), np.array(vtx, np.float32)
 
 
-# 12 frames in LDS, 64 more in the spill area, then a lone lane's stack
-@pytest.mark.parametrize("sheets", [11, 13, 14, 60, 77, 79, 200])
+# 12 frames in LDS, 60 more in the spill area by sixes, then a lone lane's stack
+@pytest.mark.parametrize("sheets", [11, 12, 13, 14, 18, 19, 20, 25, 60, 71, 72, 73, 74, 77, 79, 200])
 @pytest.mark.parametrize("size", [(8, 8), (33, 17)])
 def test_stack_beyond_lds_and_spill(gpu, oracle, sheets, size):
     want = _cast_equals_oracle(gpu, oracle, *_sheets(sheets), np.eye(4, dtype=np.float32), *size)
