@@ -37,9 +37,10 @@ constexpr int kWideTileUnit = 512;  // a wide tile, times this many
 // for every item of a thread, and at one or two tiles a CU nothing hides it:
 // with 256 threads of 16 items (wide tiles: 512 of 16) the three passes over
 // 14.5 M u64 keys took 562 us and a pass over a few thousand u32 keys 18.5 us;
-// with 1024 threads of 4 (8) they take 436 and 11 us.
+// with 1024 threads of 8 they took 436, and the small pass with 4 takes 11.
 constexpr int kPassThreads = 1024;
-constexpr uint32_t kWideTilesFrom = 1u << 21;  // elements from which the default takes them
+// A wide tile of u32 keys past one a CU, on 8 waves: two workgroups fit a CU.
+constexpr int kLongThreads = 512;
 constexpr int kRadixBits = 8;
 constexpr int kRadix = 1 << kRadixBits;
 constexpr int kMaxPasses = 8;
@@ -181,16 +182,14 @@ struct SegOff {
 // count is read from the device (the grid is sized for a capacity); the blocks
 // past the number of tiles exit, and only earlier tickets' tiles are ever
 // looked back at, so nobody waits on them.
-// ITEMS: elements a thread; large inputs take wide tiles (half the tiles, so
-// half the same-address tickets and a look-back chain half as long).
+// ITEMS: elements a thread; for the tile see tile_for.
 // SEG: a segmented pass (see SegOff); `hist` is not read.
-template <typename KeyT, int ITEMS, bool IOTA, bool SEG = false>
-__global__ __launch_bounds__(kPassThreads) void k_onesweep(
+template <typename KeyT, int ITEMS, bool IOTA, bool SEG = false, int THREADS = kPassThreads>
+__global__ __launch_bounds__(THREADS) void k_onesweep(
     const KeyT* __restrict__ kin, const uint32_t* __restrict__ vin, KeyT* __restrict__ kout,
     uint32_t* __restrict__ vout, uint32_t n, const uint32_t* __restrict__ n_dev, uint32_t shift,
     uint32_t dbits, const uint32_t* __restrict__ hist, uint32_t* __restrict__ status,
     uint32_t* __restrict__ ticket, uint32_t* __restrict__ err, SegOff seg) {
-  constexpr int THREADS = kPassThreads;
   static_assert(THREADS >= kRadix && THREADS % 64 == 0, "one thread per digit");
   constexpr int kTile = THREADS * ITEMS;
   constexpr uint32_t W = THREADS / 64;
@@ -233,8 +232,7 @@ __global__ __launch_bounds__(kPassThreads) void k_onesweep(
   for (int i = 0; i < ITEMS; ++i) {
     const bool valid = dig[i] != 0xFFFFFFFFu;
     uint64_t m = __ballot(valid);
-#pragma unroll
-    for (uint32_t b = 0; b < (uint32_t)kRadixBits; ++b) {  // bits above dbits are 0 in all lanes
+    for (uint32_t b = 0; b < dbits; ++b) {
       const bool bit = (dig[i] >> b) & 1u;
       const uint64_t bb = __ballot(bit);
       m &= bit ? bb : ~bb;
@@ -843,6 +841,32 @@ inline int launch_fill(hipStream_t s, uint32_t* p, size_t count, uint32_t value)
 // and ticket.  iota: the values are the element indices.
 // SEG: a segmented pass over the 8 bits at `shift` (digit then only names
 // the status region's histogram slot, which is not read).
+enum class Tile { kNarrow, kWide, kLong };
+
+// The tile of a pass: narrow, wide, or wide on kLongThreads.  A round of the
+// grid is a tile a CU (of long ones two), and the last round costs as much as a
+// full one.  So wide tiles pay while they are one round and narrow ones more than
+// one and a half: 2^21 u64 keys of 63 bits take 127 us with narrow tiles and 117
+// with wide ones, 1.2 M 104 and 106, 2.2 M 138 and 151.  Past that u64 keys take
+// narrow tiles (4.0 M 192 us, 194 with wide, 207 with long; 16 M 590, 640 and
+// 750).  u32 keys take long ones while they are one round (3.1 M keys of 30 bits
+// 165 us, 177 with narrow, 184 with wide) and from two full rounds on (12 M 406,
+// 440, 472), in between narrow ones (5.2 M 253 long, 240 narrow, 259 wide).
+// A count on the device is mostly far below the capacity, whose tiles exit:
+// narrow.
+template <typename KeyT>
+inline Tile tile_for(uint32_t n, int items, bool device_count) {
+  const int opt = refit_option(kSortWideTiles);
+  const uint32_t cus = (uint32_t)device_cu_count();
+  const uint32_t wide = ceil_div(n, (uint64_t)kWideTileUnit * (uint64_t)items);
+  const bool long_tiles = sizeof(KeyT) == 4 && wide > cus;
+  if (opt == 0 || (opt == 1 && device_count)) return Tile::kNarrow;
+  if (opt == 2) return long_tiles ? Tile::kLong : Tile::kWide;
+  if (wide <= cus)
+    return 2u * num_tiles_items(n, items) > 3u * cus ? Tile::kWide : Tile::kNarrow;
+  return long_tiles && (wide <= 2u * cus || wide >= 4u * cus) ? Tile::kLong : Tile::kNarrow;
+}
+
 template <typename KeyT, int ITEMS, bool SEG = false>
 inline int launch_pass_items(hipStream_t s, uint32_t n, uint32_t key_bits, const Layout& L,
                              uint32_t digit, uint32_t slot, bool iota, const KeyT* sk,
@@ -854,17 +878,22 @@ inline int launch_pass_items(hipStream_t s, uint32_t n, uint32_t key_bits, const
   const uint32_t dbits = SEG ? (uint32_t)kRadixBits : pass_bits(key_bits, digit);
   // each pass's status region is sized for the narrow tiles
   uint32_t* st = L.status + (size_t)slot * tiles * kRadix;
-  const int wide_opt = refit_option(kSortWideTiles);
-  const bool wide = wide_opt == 2 || (wide_opt == 1 && n >= kWideTilesFrom);
-  auto pass = [&](auto kernel, uint32_t grid) {
-    launch("k_onesweep", kernel, dim3(grid), dim3(kPassThreads), 0, s, sk, sv, dk, dv, n, n_dev,
-           shift, dbits, L.hist + digit * kRadix, st, L.tickets + slot, err, seg);
+  auto pass = [&](auto first, auto later, uint32_t grid, int threads) {
+    launch("k_onesweep", iota ? first : later, dim3(grid), dim3(threads), 0, s, sk, sv, dk, dv, n,
+           n_dev, shift, dbits, L.hist + digit * kRadix, st, L.tickets + slot, err, seg);
   };
-  const uint32_t wt = ceil_div(n, (uint64_t)kWideTileUnit * ITEMS);
-  if (wide && iota) pass(k_onesweep<KeyT, ITEMS / 2, true, SEG>, wt);
-  else if (wide) pass(k_onesweep<KeyT, ITEMS / 2, false, SEG>, wt);
-  else if (iota) pass(k_onesweep<KeyT, ITEMS / 4, true, SEG>, tiles);
-  else pass(k_onesweep<KeyT, ITEMS / 4, false, SEG>, tiles);
+  const uint32_t wide_tiles = ceil_div(n, (uint64_t)kWideTileUnit * ITEMS);
+  const Tile tile = tile_for<KeyT>(n, ITEMS, n_dev != nullptr);
+  if (tile == Tile::kNarrow) {
+    pass(k_onesweep<KeyT, ITEMS / 4, true, SEG>, k_onesweep<KeyT, ITEMS / 4, false, SEG>, tiles,
+         kPassThreads);
+  } else if (tile == Tile::kWide) {
+    pass(k_onesweep<KeyT, ITEMS / 2, true, SEG>, k_onesweep<KeyT, ITEMS / 2, false, SEG>,
+         wide_tiles, kPassThreads);
+  } else if constexpr (sizeof(KeyT) == 4) {
+    pass(k_onesweep<KeyT, ITEMS, true, SEG, kLongThreads>,
+         k_onesweep<KeyT, ITEMS, false, SEG, kLongThreads>, wide_tiles, kLongThreads);
+  }
   return launch_status();
 }
 
