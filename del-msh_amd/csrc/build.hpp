@@ -367,7 +367,7 @@ inline int build(hipStream_t s, uint32_t n, const uint32_t* tri2vtx, uint32_t nu
                      L.keys6, err);
   if ((rc = launch_status()) != DMSH_OK) return rc;
   KeyT* codes = static_cast<KeyT*>(L.codes);
-  if (n <= sortk::small_capacity<KeyT>()) {
+  if (n <= sortk::small_capacity<KeyT>(kb)) {
     rc = sortk::sort_small<KeyT>(s, MortonSrc<KeyT>{TRI ? L.cntr : xyz, L.keys6, {}}, n, kb, codes,
                                  L.idx, static_cast<KeyT*>(L.sort.alt_keys), L.sort.alt_vals);
     if (rc != DMSH_OK) return rc;

@@ -604,13 +604,18 @@ __global__ __launch_bounds__(kGroupThreads) void k_sort_groups(
 // ---------------------------------------------------------------------------
 constexpr int kSmallThreads = 1024;
 constexpr uint32_t kChunk = 4u * kSmallThreads;
-// Every element searches every chunk, so the time grows with n^2 and meets the
-// digit passes': a build of 60 000 triangles with 30-bit codes takes 94 us (122
-// with digit passes), of 98 000 123 (125); with 63-bit codes, of 40 000 100
-// (108), of 60 000 114 (112).
+// Elements up to which the chunks are faster than P digit passes.  Every element
+// searches every chunk, so the merge's time grows with n^2, a chunk's sort with P,
+// and the passes' with P up to four digits (beyond, three passes and the finish
+// serve all).  u32 keys of 8 / 16 / 24 / 30 bits take the same time either way at
+// 20 / 28 / 45 / 53 thousand elements (21 / 30 / 47 / 54 us; 98,000 keys of 16
+// bits 72 us in chunks and 33 in passes), u64 keys of 40 / 63 bits at 38 / 25
+// thousand (50 us); builds of triangles likewise, 30-bit codes at 58,000 (100 us),
+// 63-bit ones at 22,000 (92).
 template <typename KeyT>
-__host__ __device__ constexpr uint32_t small_capacity() {
-  return kChunk * (sizeof(KeyT) == 4 ? 24u : 10u);
+__host__ __device__ constexpr uint32_t small_capacity(uint32_t key_bits) {
+  const uint32_t P = (key_bits + (uint32_t)kRadixBits - 1u) / (uint32_t)kRadixBits;
+  return kChunk * (P <= 4u ? (sizeof(KeyT) == 4 ? 3u : 2u) * P + 1u : 14u - P);
 }
 
 template <typename KeyT>
@@ -753,7 +758,7 @@ __global__ __launch_bounds__(256) void k_merge_chunks(const KeyT* __restrict__ k
   vals[at] = vin[e];
 }
 
-// Sorts n <= small_capacity<KeyT>() elements.  (tmp_keys, tmp_vals) hold n elements and
+// Sorts n <= small_capacity<KeyT>(key_bits) elements.  (tmp_keys, tmp_vals) hold n elements and
 // are used by more than one chunk; keys_out may be the keys that src reads.
 template <typename KeyT, class Src>
 inline int sort_small(hipStream_t s, const Src& src, uint32_t n, uint32_t key_bits, KeyT* keys_out,
@@ -1059,7 +1064,7 @@ inline int argsort(hipStream_t s, uint32_t n, KeyT* keys_inout, uint32_t* idx_ou
   if (!carve<KeyT>(a, n, key_bits, L)) return DMSH_ERR_WORKSPACE;
   uint32_t* err = device_error_word();
   if (!err) return DMSH_ERR_HIP;
-  if (n <= small_capacity<KeyT>())
+  if (n <= small_capacity<KeyT>(key_bits))
     return sort_small<KeyT>(s, KeysSrc<KeyT>{keys_inout}, n, key_bits, keys_inout, idx_out,
                             static_cast<KeyT*>(L.alt_keys), L.alt_vals);
   int rc = launch_fill(s, L.hist, L.zero_words, 0u);

@@ -10,7 +10,8 @@ import del_msh_dlpack.Array1D.torch as Array1D
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [1, 2, 64, 65, 1023, 1024, 1025, 4095, 4096, 4097, 8193, 16384, 20481, 40960, 40961, 65537,
+SIZES = [1, 2, 64, 65, 1023, 1024, 1025, 4095, 4096, 4097, 8193, 16384, 16385, 20481, 24576, 24577,
+         28672, 28673, 36864, 36865, 40960, 40961, 53248, 53249, 65537,
          98304, 98305]
 
 
