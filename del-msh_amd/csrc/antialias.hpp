@@ -18,12 +18,14 @@
 //     stores its value.
 //   backward: dL/dp of an edge's two vertices is accumulated over its walk and
 //     added with six float atomics.
-// A group of kEdgeLanes lanes walks an edge, one step each: the positions are
-// the serial walk's (each lane adds its way to its own), the pixel reads and
+// A group of L lanes walks an edge, one step each: the positions are the
+// serial walk's (each lane adds its way to its own), the pixel reads and
 // crossings of the steps run side by side.  With a thread an edge a step cost
 // a chain of up to eight reads and a pass took the longest edge's walk: 46 us
 // for the keys, 50 for the writes and 54 backward on 53 000-triangle meshes at
-// 512^2; with 16 lanes 5.6, 5.8 and 8.6 us.
+// 512^2; with 16 lanes 5.6, 5.8 and 8.6 us.  Many edges fill the GPU with
+// fewer lanes each, and then a lane past the end of a short walk is lost: see
+// edge_lanes.
 // A walk stops once it has left the image in its direction of travel (no
 // pixel after that point can be inside), and edges with a non-finite
 // projection are skipped.
@@ -81,8 +83,23 @@ __device__ __forceinline__ void dldw_intersection_edge2(const float c0[2], const
 // steps a pixel walk may take before it is abandoned (DMSH_DEVERR_WALK)
 constexpr uint32_t kWalkLimit = 1u << 26;
 
-constexpr uint32_t kEdgeLanes = 16;
-static_assert(kWalkLimit % kEdgeLanes == 0, "whole rounds");
+constexpr uint32_t kMaxEdgeLanes = 16;
+static_assert(kWalkLimit % kMaxEdgeLanes == 0, "whole rounds");
+
+// Lanes an edge of a pass over num_cedge edges.  The backward pass adds six
+// atomics an edge beside its walk, so it is full with fewer edges.  us with 16 /
+// 8 / 4 lanes (and a thread an edge), forward | backward:
+//     712 edges, 2048^2   20 / 27 / 36 (186)    |  6 / 8 / 11 (70)
+//   32,000 edges, 512^2   16 / 16 / 17 (51)     | 25 / 19 / 18 (30)
+//   32,000 edges, 2048^2  29 / 34 / 49 (204)    | 27 / 23 / 27 (85)
+//   82,000 edges, 512^2   24 / 17 / 15 (31)     | 53 / 45 / 39 (41)
+//   82,000 edges, 2048^2  30 / 27 / 30 (97)     | 52 / 45 / 42 (58)
+//  165,000 edges, 2048^2  54 / 50 / 60 (222)    | 75 / 62 / 61 (126)
+//  972,000 edges, 512^2  186 / 94 / 64 (101)    | 303 / 217 / 202 (235)
+inline uint32_t edge_lanes(uint32_t num_cedge, bool backward) {
+  const uint32_t n = backward ? num_cedge : num_cedge / 4u;
+  return n <= (1u << 14) ? 16u : (n <= (1u << 16) ? 8u : 4u);
+}
 
 struct Pair {
   uint32_t p0, p1;
@@ -130,11 +147,11 @@ __device__ __forceinline__ void cross_pixel(const float q0[2], const float q1[2]
   }
 }
 
-// Walks the edge q0 -> q1 with the kEdgeLanes lanes of a group, lane `sub` of
-// which takes the steps sub, sub + kEdgeLanes, ...; every lane of the group
+// Walks the edge q0 -> q1 with the L lanes of a group, lane `sub` of which
+// takes the steps sub, sub + L, ...; every lane of the group
 // calls with the same edge, and lanes of other groups may have left.  Returns
 // false when the walk hit the step cap.
-template <class Fn>
+template <uint32_t L, class Fn>
 __device__ __forceinline__ bool walk(const float q0[2], const float q1[2], uint32_t sub,
                                      uint32_t img_w, uint32_t img_h,
                                      const uint32_t* __restrict__ pix2tri, Fn fn) {
@@ -146,11 +163,11 @@ __device__ __forceinline__ bool walk(const float q0[2], const float q1[2], uint3
   const float step = fmax_sel(fabsf(dx), fabsf(dy));
   const float slope_x = dx / step, slope_y = dy / step;
   const float fw = (float)img_w, fh = (float)img_h;
-  const uint32_t group = (threadIdx.x & 63u) / kEdgeLanes * kEdgeLanes;
-  for (uint32_t k0 = 0; k0 < kWalkLimit; k0 += kEdgeLanes) {
+  const uint32_t group = (threadIdx.x & 63u) / L * L;
+  for (uint32_t k0 = 0; k0 < kWalkLimit; k0 += L) {
     float mx = x, my = y;  // this lane's step, by the serial walk's additions
 #pragma unroll
-    for (uint32_t i = 1; i <= kEdgeLanes; ++i) {
+    for (uint32_t i = 1; i <= L; ++i) {
       x = x + slope_x;
       y = y + slope_y;
       if (i == sub) {
@@ -166,7 +183,7 @@ __device__ __forceinline__ bool walk(const float q0[2], const float q1[2], uint3
                       (slope_x > 0.f && mx >= fw) || (slope_x < 0.f && mx < 0.f) ||
                       (slope_y > 0.f && my >= fh) || (slope_y < 0.f && my < 0.f);
     const uint32_t ends =
-        (uint32_t)(__ballot(last) >> group) & (uint32_t)((1ull << kEdgeLanes) - 1ull);
+        (uint32_t)(__ballot(last) >> group) & (uint32_t)((1ull << L) - 1ull);
     const bool mine = ends == 0u || sub <= (uint32_t)__builtin_ctz(ends);
     const float fx = floorf(mx), fy = floorf(my);
     if (mine && fx >= 0.f && fy >= 0.f && fx < fw && fy < fh)
@@ -211,19 +228,21 @@ static __global__ __launch_bounds__(256) void k_zero_u64(unsigned long long* __r
 
 // The writes of contour edge e, by the lanes of its group, as keys (edge, then
 // step and pair) into the pixels' maxima.
+template <uint32_t L>
 __device__ __forceinline__ void keys_of_edge(const EdgeArgs& a, uint32_t e, uint32_t sub,
                                              unsigned long long* __restrict__ keys) {
   const unsigned long long hi = (unsigned long long)(e + 1) << 32;
   float m[16], q0[2], q1[2];
   uint32_t i0, i1;
   if (!edge_setup(a, e, m, i0, i1, q0, q1)) return;
-  const bool done = walk(q0, q1, sub, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t seq) {
+  const bool done = walk<L>(q0, q1, sub, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t seq) {
     atomicMax(keys + (rc < 0.5f ? pr.p0 : pr.p1), hi | seq);
   });
   if (!done && sub == 0u) raise_error(a.err, DMSH_DEVERR_WALK);
 }
 
 // The values of its writes that hold their pixel's key.
+template <uint32_t L>
 __device__ __forceinline__ void values_of_edge(const EdgeArgs& a, uint32_t e, uint32_t sub,
                                                const unsigned long long* __restrict__ keys,
                                                const float* __restrict__ vin,
@@ -232,7 +251,7 @@ __device__ __forceinline__ void values_of_edge(const EdgeArgs& a, uint32_t e, ui
   float m[16], q0[2], q1[2];
   uint32_t i0, i1;
   if (!edge_setup(a, e, m, i0, i1, q0, q1)) return;
-  walk(q0, q1, sub, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t seq) {
+  walk<L>(q0, q1, sub, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t seq) {
     const uint32_t p = rc < 0.5f ? pr.p0 : pr.p1;
     if (keys[p] != (hi | seq)) return;
     const float r0 = rc < 0.5f ? 0.5f + rc : rc - 0.5f;
@@ -240,33 +259,36 @@ __device__ __forceinline__ void values_of_edge(const EdgeArgs& a, uint32_t e, ui
   });
 }
 
-// The contour edges of one launch: kEdgeLanes threads each, within the 2^32
-// threads that a launch may have.
+// The contour edges of one launch: up to kMaxEdgeLanes threads each, within the
+// 2^32 threads that a launch may have.
 struct EdgeSlice {
   uint32_t first, count;
 };
 constexpr uint32_t kEdgeSlice = 1u << 27;
-static_assert((uint64_t)kEdgeSlice * kEdgeLanes < (1ull << 32), "threads of a launch");
+static_assert((uint64_t)kEdgeSlice * kMaxEdgeLanes < (1ull << 32), "threads of a launch");
 
 // The edge of the thread's group, false past the slice's last.
+template <uint32_t L>
 __device__ __forceinline__ bool group_edge(const EdgeSlice& es, uint32_t& e) {
-  const uint32_t i = blockIdx.x * (64u / kEdgeLanes) + threadIdx.x / kEdgeLanes;
+  const uint32_t i = blockIdx.x * (64u / L) + threadIdx.x / L;
   e = es.first + i;
   return i < es.count;
 }
 
-static __global__ __launch_bounds__(64) void k_aa_keys(EdgeSlice es, EdgeArgs a,
+template <uint32_t L>
+__global__ __launch_bounds__(64) void k_aa_keys(EdgeSlice es, EdgeArgs a,
                                                        unsigned long long* __restrict__ keys) {
   uint32_t e;
-  if (group_edge(es, e)) keys_of_edge(a, e, threadIdx.x % kEdgeLanes, keys);
+  if (group_edge<L>(es, e)) keys_of_edge<L>(a, e, threadIdx.x % L, keys);
 }
 
-static __global__ __launch_bounds__(64) void k_aa_write(EdgeSlice es, EdgeArgs a,
+template <uint32_t L>
+__global__ __launch_bounds__(64) void k_aa_write(EdgeSlice es, EdgeArgs a,
                                                         const unsigned long long* __restrict__ keys,
                                                         const float* __restrict__ vin,
                                                         float* __restrict__ vout) {
   uint32_t e;
-  if (group_edge(es, e)) values_of_edge(a, e, threadIdx.x % kEdgeLanes, keys, vin, vout);
+  if (group_edge<L>(es, e)) values_of_edge<L>(a, e, threadIdx.x % L, keys, vin, vout);
 }
 
 __device__ __forceinline__ void proj_jacobian_xy(const float* m, const float* p, float J[2][3]) {
@@ -282,6 +304,7 @@ __device__ __forceinline__ void proj_jacobian_xy(const float* m, const float* p,
 }
 
 // dL/d(vertices) of contour edge e, by the lanes of its group.
+template <uint32_t L>
 __device__ __forceinline__ void bwd_of_edge(const EdgeArgs& a, uint32_t e, uint32_t sub,
                                             const float* __restrict__ val,
                                             const float* __restrict__ dldw,
@@ -293,7 +316,7 @@ __device__ __forceinline__ void bwd_of_edge(const EdgeArgs& a, uint32_t e, uint3
   proj_jacobian_xy(m, a.xyz + (size_t)i0 * 3, J0);
   proj_jacobian_xy(m, a.xyz + (size_t)i1 * 3, J1);
   float g0[3] = {0.f, 0.f, 0.f}, g1[3] = {0.f, 0.f, 0.f};
-  const bool done = walk(q0, q1, sub, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t) {
+  const bool done = walk<L>(q0, q1, sub, a.img_w, a.img_h, a.pix2tri, [&](const Pair& pr, float rc, uint32_t) {
     const float dv = val[pr.p0] - val[pr.p1];
     const float dldr0 = rc < 0.5f ? dldw[pr.p0] * dv : dldw[pr.p1] * dv;
     float dldq1[2], dldq0[2];
@@ -308,9 +331,9 @@ __device__ __forceinline__ void bwd_of_edge(const EdgeArgs& a, uint32_t e, uint3
 #pragma unroll
   for (int j = 0; j < 3; ++j) {
 #pragma unroll
-    for (uint32_t d = kEdgeLanes / 2u; d != 0u; d >>= 1) {
-      g0[j] += __shfl_xor(g0[j], (int)d, (int)kEdgeLanes);
-      g1[j] += __shfl_xor(g1[j], (int)d, (int)kEdgeLanes);
+    for (uint32_t d = L / 2u; d != 0u; d >>= 1) {
+      g0[j] += __shfl_xor(g0[j], (int)d, (int)L);
+      g1[j] += __shfl_xor(g1[j], (int)d, (int)L);
     }
     if (sub == 0u) {
       unsafeAtomicAdd(dldw_vtx2xyz + (size_t)i0 * 3 + j, g0[j]);
@@ -319,12 +342,13 @@ __device__ __forceinline__ void bwd_of_edge(const EdgeArgs& a, uint32_t e, uint3
   }
 }
 
-static __global__ __launch_bounds__(64) void k_aa_bwd(EdgeSlice es, EdgeArgs a,
+template <uint32_t L>
+__global__ __launch_bounds__(64) void k_aa_bwd(EdgeSlice es, EdgeArgs a,
                                                       const float* __restrict__ val,
                                                       const float* __restrict__ dldw,
                                                       float* __restrict__ dldw_vtx2xyz) {
   uint32_t e;
-  if (group_edge(es, e)) bwd_of_edge(a, e, threadIdx.x % kEdgeLanes, val, dldw, dldw_vtx2xyz);
+  if (group_edge<L>(es, e)) bwd_of_edge<L>(a, e, threadIdx.x % L, val, dldw, dldw_vtx2xyz);
 }
 
 // ---------------------------------------------------------------------------

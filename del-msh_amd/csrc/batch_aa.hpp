@@ -154,10 +154,10 @@ static __global__ __launch_bounds__(256) void k_batch_aa_init(
 
 // Calls fn(the mesh's args, its contour edge, lane of the group, its first
 // pixel, its first vertex) for the group's contour edge of the batch.
-template <class Fn>
+template <uint32_t L, class Fn>
 __device__ __forceinline__ void with_cedge(const aa::EdgeSlice& es, const Images& b, Fn fn) {
   uint32_t g;
-  if (!aa::group_edge(es, g) || *b.bad != 0u) return;
+  if (!aa::group_edge<L>(es, g) || *b.bad != 0u) return;
   const uint32_t m = bat::find_segment(b.mesh2cedge, b.M, g);
   const uint32_t p0 = b.mesh2pix[m], n = b.mesh2pix[m + 1] - p0, w = b.mesh2width[m];
   if (n == 0u) return;
@@ -166,30 +166,33 @@ __device__ __forceinline__ void with_cedge(const aa::EdgeSlice& es, const Images
                        b.mesh2vtx[m + 1] - v0,       b.w2p + (size_t)m * 16,
                        w,                            n / w,
                        b.pix2tri + p0,               b.err};
-  fn(a, g - c0, threadIdx.x % aa::kEdgeLanes, p0, v0);
+  fn(a, g - c0, threadIdx.x % L, p0, v0);
 }
 
-static __global__ __launch_bounds__(64) void k_batch_aa_keys(
+template <uint32_t L>
+__global__ __launch_bounds__(64) void k_batch_aa_keys(
     aa::EdgeSlice es, Images b, unsigned long long* __restrict__ keys) {
-  with_cedge(es, b, [&](const aa::EdgeArgs& a, uint32_t e, uint32_t sub, uint32_t p0, uint32_t) {
-    aa::keys_of_edge(a, e, sub, keys + p0);
+  with_cedge<L>(es, b, [&](const aa::EdgeArgs& a, uint32_t e, uint32_t sub, uint32_t p0, uint32_t) {
+    aa::keys_of_edge<L>(a, e, sub, keys + p0);
   });
 }
 
-static __global__ __launch_bounds__(64) void k_batch_aa_write(
+template <uint32_t L>
+__global__ __launch_bounds__(64) void k_batch_aa_write(
     aa::EdgeSlice es, Images b, const unsigned long long* __restrict__ keys,
     const float* __restrict__ vin, float* __restrict__ vout) {
-  with_cedge(es, b, [&](const aa::EdgeArgs& a, uint32_t e, uint32_t sub, uint32_t p0, uint32_t) {
-    aa::values_of_edge(a, e, sub, keys + p0, vin + p0, vout + p0);
+  with_cedge<L>(es, b, [&](const aa::EdgeArgs& a, uint32_t e, uint32_t sub, uint32_t p0, uint32_t) {
+    aa::values_of_edge<L>(a, e, sub, keys + p0, vin + p0, vout + p0);
   });
 }
 
-static __global__ __launch_bounds__(64) void k_batch_aa_bwd(aa::EdgeSlice es, Images b,
+template <uint32_t L>
+__global__ __launch_bounds__(64) void k_batch_aa_bwd(aa::EdgeSlice es, Images b,
                                                             const float* __restrict__ val,
                                                             const float* __restrict__ dldw,
                                                             float* __restrict__ dldw_vtx2xyz) {
-  with_cedge(es, b, [&](const aa::EdgeArgs& a, uint32_t e, uint32_t sub, uint32_t p0, uint32_t v0) {
-    aa::bwd_of_edge(a, e, sub, val + p0, dldw + p0, dldw_vtx2xyz + (size_t)v0 * 3);
+  with_cedge<L>(es, b, [&](const aa::EdgeArgs& a, uint32_t e, uint32_t sub, uint32_t p0, uint32_t v0) {
+    aa::bwd_of_edge<L>(a, e, sub, val + p0, dldw + p0, dldw_vtx2xyz + (size_t)v0 * 3);
   });
 }
 

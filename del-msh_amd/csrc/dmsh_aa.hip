@@ -1,5 +1,6 @@
 // dmsh_aa.hip -- C ABI: contour edges and the anti-aliased silhouette.
 #include <algorithm>
+#include <type_traits>
 
 #include "antialias.hpp"
 #include "batch_aa.hpp"
@@ -14,19 +15,28 @@ struct ContourLayout {
   uint32_t* block_count;
 };
 
-// Launches a kernel over num_cedge contour edges in blocks of 64 threads,
-// kEdgeLanes an edge.
+// Launches a kernel over num_cedge contour edges in blocks of 64 threads, `lanes`
+// an edge.
 template <typename... KArgs, typename... Args>
-int launch_edges(const char* label, void (*kernel)(aa::EdgeSlice, KArgs...), uint32_t num_cedge,
-                 hipStream_t s, const Args&... args) {
+int launch_edges(const char* label, void (*kernel)(aa::EdgeSlice, KArgs...), uint32_t lanes,
+                 uint32_t num_cedge, hipStream_t s, const Args&... args) {
   int st = DMSH_OK;
   for (aa::EdgeSlice es{0u, 0u}; st == DMSH_OK && es.first < num_cedge; es.first += es.count) {
     es.count = std::min(num_cedge - es.first, aa::kEdgeSlice);
-    launch(label, kernel, dim3(ceil_div(es.count, 64u / aa::kEdgeLanes)), dim3(64), 0, s, es,
-           args...);
+    launch(label, kernel, dim3(ceil_div(es.count, 64u / lanes)), dim3(64), 0, s, es, args...);
     st = launch_status();
   }
   return st;
+}
+
+// Calls fn(integral_constant of the lanes an edge).
+template <class Fn>
+int with_lanes(uint32_t num_cedge, bool backward, Fn fn) {
+  switch (aa::edge_lanes(num_cedge, backward)) {
+    case 16: return fn(std::integral_constant<uint32_t, 16>());
+    case 8: return fn(std::integral_constant<uint32_t, 8>());
+    default: return fn(std::integral_constant<uint32_t, 4>());
+  }
 }
 
 inline uint32_t contour_blocks(uint32_t num_edge) { return ceil_div(num_edge, 256); }
@@ -139,9 +149,13 @@ int dmsh_antialias_fwd(void* stream, uint32_t num_cedge, const uint32_t* cedge2v
   if (st != DMSH_OK) return st;
   const aa::EdgeArgs ea{cedge2vtx, vtx2xyz, num_vtx, transform_world2pix,
                         img_w, img_h, pix2tri, err};
-  st = launch_edges("k_aa_keys", aa::k_aa_keys, num_cedge, s, ea, keys);
-  if (st != DMSH_OK) return st;
-  return launch_edges("k_aa_write", aa::k_aa_write, num_cedge, s, ea, keys, pix2vin, pix2vout);
+  return with_lanes(num_cedge, false, [&](auto lanes) {
+    constexpr uint32_t L = decltype(lanes)::value;
+    const int rc = launch_edges("k_aa_keys", aa::k_aa_keys<L>, L, num_cedge, s, ea, keys);
+    if (rc != DMSH_OK) return rc;
+    return launch_edges("k_aa_write", aa::k_aa_write<L>, L, num_cedge, s, ea, keys, pix2vin,
+                        pix2vout);
+  });
 }
 
 int dmsh_antialias_bwd(void* stream, uint32_t num_cedge, const uint32_t* cedge2vtx,
@@ -158,8 +172,11 @@ int dmsh_antialias_bwd(void* stream, uint32_t num_cedge, const uint32_t* cedge2v
   if (!err) return DMSH_ERR_HIP;
   const aa::EdgeArgs ea{cedge2vtx, vtx2xyz, num_vtx, transform_world2pix,
                         img_w, img_h, pix2tri, err};
-  return launch_edges("k_aa_bwd", aa::k_aa_bwd, num_cedge, as_stream(stream), ea, pix2val,
-                      dldw_pix2val, dldw_vtx2xyz);
+  return with_lanes(num_cedge, true, [&](auto lanes) {
+    constexpr uint32_t L = decltype(lanes)::value;
+    return launch_edges("k_aa_bwd", aa::k_aa_bwd<L>, L, num_cedge, as_stream(stream), ea, pix2val,
+                        dldw_pix2val, dldw_vtx2xyz);
+  });
 }
 
 size_t dmsh_batch_contour_workspace_bytes(uint32_t num_mesh, uint32_t total_edge) {
@@ -243,11 +260,14 @@ int dmsh_batch_antialias_fwd(void* stream, uint32_t num_mesh, uint32_t total_vtx
          total_vtx, total_pix, L.keys, (uint64_t)total_pix);
   int st = launch_status();
   if (st != DMSH_OK) return st;
-  if ((st = launch_edges("k_batch_aa_keys", baa::k_batch_aa_keys, num_cedge, s, b, L.keys)) !=
-      DMSH_OK)
-    return st;
-  return launch_edges("k_batch_aa_write", baa::k_batch_aa_write, num_cedge, s, b, L.keys, pix2vin,
-                      pix2vout);
+  return with_lanes(num_cedge, false, [&](auto lanes) {
+    constexpr uint32_t N = decltype(lanes)::value;
+    const int rc =
+        launch_edges("k_batch_aa_keys", baa::k_batch_aa_keys<N>, N, num_cedge, s, b, L.keys);
+    if (rc != DMSH_OK) return rc;
+    return launch_edges("k_batch_aa_write", baa::k_batch_aa_write<N>, N, num_cedge, s, b, L.keys,
+                        pix2vin, pix2vout);
+  });
 }
 
 int dmsh_batch_antialias_bwd(void* stream, uint32_t num_mesh, uint32_t total_vtx,
@@ -275,8 +295,11 @@ int dmsh_batch_antialias_bwd(void* stream, uint32_t num_mesh, uint32_t total_vtx
          total_pix, L.keys, (uint64_t)0);
   int st = launch_status();
   if (st != DMSH_OK) return st;
-  return launch_edges("k_batch_aa_bwd", baa::k_batch_aa_bwd, num_cedge, s, b, pix2val,
-                      dldw_pix2val, dldw_vtx2xyz);
+  return with_lanes(num_cedge, true, [&](auto lanes) {
+    constexpr uint32_t N = decltype(lanes)::value;
+    return launch_edges("k_batch_aa_bwd", baa::k_batch_aa_bwd<N>, N, num_cedge, s, b, pix2val,
+                        dldw_pix2val, dldw_vtx2xyz);
+  });
 }
 
 }  // extern "C"

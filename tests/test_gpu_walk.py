@@ -29,11 +29,16 @@ def _edges(rng):
     return vtx, np.arange(len(ends), dtype=np.uint32).reshape(-1, 2)
 
 
+# edges that are skipped, after the others, so that sixteen, eight and four lanes
+# walk an edge
+@pytest.mark.parametrize("more", [0, (1 << 14) + 1, (1 << 16) + 1, (1 << 18) + 1])
 @pytest.mark.parametrize("seed", [0, 1])
 @pytest.mark.parametrize("cover", [0.5, 0.95])
-def test_walks_equal_the_serial_walk(gpu, oracle, seed, cover):
+def test_walks_equal_the_serial_walk(gpu, oracle, seed, cover, more):
     rng = np.random.default_rng(seed)
     vtx, edge = _edges(rng)
+    assert not np.isfinite(vtx[-1]).all()
+    edge = np.concatenate([edge, np.full((more, 2), len(vtx) - 1, np.uint32)])
     pix = np.where(rng.random((H, W)) < cover, 3, 0xFFFFFFFF).astype(np.uint32)
     val = rng.random((H, W), dtype=np.float32)
     dldw = rng.normal(size=(H, W)).astype(np.float32)
