@@ -855,8 +855,9 @@ enum class Tile { kNarrow, kWide, kLong };
 // with wide ones, 1.2 M 104 and 106, 2.2 M 138 and 151.  Past that u64 keys take
 // narrow tiles (4.0 M 192 us, 194 with wide, 207 with long; 16 M 590, 640 and
 // 750).  u32 keys take long ones while they are one round (3.1 M keys of 30 bits
-// 165 us, 177 with narrow, 184 with wide) and from two full rounds on (12 M 406,
-// 440, 472), in between narrow ones (5.2 M 253 long, 240 narrow, 259 wide).
+// 165 us, 177 with narrow, 184 with wide) and from two nearly full rounds on (8 M
+// 316, 333, 346; 12 M 406, 440, 472), in between narrow ones (5.2 M 253 long, 240
+// narrow, 259 wide).
 // A count on the device is mostly far below the capacity, whose tiles exit:
 // narrow.
 template <typename KeyT>
@@ -869,7 +870,7 @@ inline Tile tile_for(uint32_t n, int items, bool device_count) {
   if (opt == 2) return long_tiles ? Tile::kLong : Tile::kWide;
   if (wide <= cus)
     return 2u * num_tiles_items(n, items) > 3u * cus ? Tile::kWide : Tile::kNarrow;
-  return long_tiles && (wide <= 2u * cus || wide >= 4u * cus) ? Tile::kLong : Tile::kNarrow;
+  return long_tiles && (wide <= 2u * cus || 2u * wide >= 7u * cus) ? Tile::kLong : Tile::kNarrow;
 }
 
 template <typename KeyT, int ITEMS, bool SEG = false>
