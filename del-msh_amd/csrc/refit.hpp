@@ -1361,6 +1361,10 @@ inline int launch_refit_treelets(hipStream_t s, const TreeView& v, uint32_t* fla
 //   topology kernel does.  One failed check sets *bad: the treelet kernels
 //   then skip and the generic climb (gated on *bad) refits the tree instead.
 constexpr uint32_t kPlanHashBlocks = 1024;  // row-hash partials (see k_plan_hash)
+// A plan that is kept has at most kTopSlots top nodes, and their children
+// below the top are its treelets: one more than the nodes.
+constexpr uint32_t kPlanEntries = kTopSlots + 1;
+constexpr uint32_t kPlanSumBlocks = (kPlanEntries + 255) / 256;  // plan-hash partials
 
 struct StandaloneLayout {
   uint32_t* flags;     // num_leaf - 1 arrival counters
@@ -1370,7 +1374,7 @@ struct StandaloneLayout {
   uint32_t* counters;  // treelet count, top count, next treelet, bad, plan needed
   uint4* treelets;     // num_leaf
   uint4* top_list;     // kTopSlots: (node, left child, right child, top-child flags)
-  unsigned long long* hash;  // -, stamp of the kept plan, tag, -, row-hash partials
+  unsigned long long* hash;  // plan sum, row stamp, tag, -, row partials, plan partials
   uint32_t* top_kid;   // kTopClimbSlots (TopStage)
   float* top_box;      // 2 kTopClimbSlots boxes (TopStage)
 };
@@ -1384,20 +1388,23 @@ inline bool carve_standalone(Arena& a, uint32_t n, StandaloneLayout& L) {
   L.counters = a.take<uint32_t>(8);
   L.treelets = a.take<uint4>(n ? n : 1);
   L.top_list = a.take<uint4>(kTopSlots);
-  L.hash = a.take<unsigned long long>(4 + kPlanHashBlocks);
+  L.hash = a.take<unsigned long long>(4 + kPlanHashBlocks + kPlanSumBlocks);
   L.top_kid = a.take<uint32_t>(kTopClimbSlots);
   L.top_box = a.take<float>((size_t)kTopClimbSlots * 12);
   return a.ok();
 }
 
-// The plan -- leaf ranges, treelet and top lists -- depends on the rows
-// only, so a workspace that is used again for the same rows keeps it:
-// k_plan_hash sums a mixed hash of every (word index, word) of bvhnodes,
-// k_plan_gate compares the sum with the stamp kept beside the plan and sets
-// the gate of the two plan kernels when they differ (or when the workspace
-// has never held a plan, the tree failed the layout check, or its top list
-// overflowed).  A workspace fresh from an allocator holds no valid tag, so
-// its first call builds the plan.
+// The plan -- treelet and top lists, slots of the top nodes -- depends on the
+// rows only, so a workspace that is used again for the same rows keeps it:
+// k_plan_hash sums a mixed hash of every (word index, word) of bvhnodes and
+// one of the plan's own words, k_plan_gate compares the sums with those kept
+// beside the plan and sets the gate of the two plan kernels when either
+// differs (or when the workspace has never held a plan, the tree failed the
+// layout check, or its top list overflowed).  The plan itself is summed
+// because the stamp outlives it: the parts of a workspace lie where the
+// number of leaves puts them, so a call for a larger tree can write over the
+// lists of a smaller one and leave its stamp whole, and so can any other use
+// of the memory between two calls or before the first.
 constexpr unsigned long long kPlanTag = 0x646d73685f706c6eull;
 
 __device__ __forceinline__ unsigned long long mix64(unsigned long long z) {
@@ -1416,19 +1423,64 @@ __device__ __forceinline__ unsigned long long word_hash(unsigned long long w, ui
   return v ^ (v >> 29);
 }
 
-static __global__ __launch_bounds__(256) void k_plan_hash(const uint32_t* __restrict__ words, size_t num_words,
-                                                          unsigned long long* __restrict__ part) {
+// The terms of the plan's sum: an entry's four words, numbered by its slot;
+// for a top entry also the slot that node2slot gives its node.
+__device__ __forceinline__ unsigned long long entry_hash(unsigned long long w, const uint4& x) {
+  return word_hash(w, x.x) + word_hash(w + 1, x.y) + word_hash(w + 2, x.z) + word_hash(w + 3, x.w);
+}
+__device__ __forceinline__ unsigned long long treelet_hash(uint32_t slot, const uint4& t) {
+  return entry_hash(4ull * slot, t);
+}
+__device__ __forceinline__ unsigned long long top_hash(uint32_t slot, const uint4& t,
+                                                       uint32_t node_slot) {
+  const unsigned long long w = (1ull << 40) + 5ull * slot;
+  return entry_hash(w, t) + word_hash(w + 4, node_slot);
+}
+
+// Sum of h over the workgroup's 256 threads, in thread 0.
+__device__ __forceinline__ unsigned long long block_sum(unsigned long long h,
+                                                        unsigned long long* s_part) {
+  for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
+  if ((threadIdx.x & 63u) == 0) s_part[threadIdx.x >> 6] = h;
+  __syncthreads();
+  return s_part[0] + s_part[1] + s_part[2] + s_part[3];
+}
+
+// part[0 .. row_blocks): the row sums of the first row_blocks workgroups;
+// part[kPlanHashBlocks ..): the plan sums of the others, one treelet and one
+// top entry a thread.  Workgroups of their own, because the counts, the
+// entries and the gather through node2slot are three dependent loads: behind
+// the rows in the same threads a kept refit took 1.3 us more, beside them
+// 0.7 us (200 K triangles, 32.4 us without the plan's sum).  The lists may
+// hold anything (see above), so the counts are clamped to them and the nodes
+// checked before they are used as indexes.
+static __global__ __launch_bounds__(256) void k_plan_hash(
+    const uint32_t* __restrict__ words, size_t num_words, uint32_t row_blocks, uint32_t num_leaf,
+    const uint32_t* __restrict__ counters, const uint4* __restrict__ treelets,
+    const uint4* __restrict__ top_list, const uint32_t* __restrict__ node2slot,
+    unsigned long long* __restrict__ part) {
   __shared__ unsigned long long s_part[4];
   unsigned long long h = 0;
-  const size_t stride = (size_t)gridDim.x * 256;
+  if (blockIdx.x >= row_blocks) {
+    const uint32_t b = blockIdx.x - row_blocks, e = b * 256 + threadIdx.x;
+    const uint32_t nt = counters[0] < num_leaf ? counters[0] : num_leaf, tc = counters[1];
+    if (e < kPlanEntries && e < nt) h += treelet_hash(e, treelets[e]);
+    if (e < (uint32_t)kTopSlots && e < tc) {
+      const uint4 t = top_list[e];
+      h += top_hash(e, t, t.x < num_leaf - 1 ? node2slot[t.x] : DMSH_U32MAX);
+    }
+    h = block_sum(h, s_part);
+    if (threadIdx.x == 0) part[kPlanHashBlocks + b] = h;
+    return;
+  }
+  const size_t stride = (size_t)row_blocks * 256;
   if ((reinterpret_cast<uintptr_t>(words) & 15u) == 0) {
     const uint4* q = reinterpret_cast<const uint4*>(words);
     const size_t nq = num_words / 4;
     for (size_t i = (size_t)blockIdx.x * 256 + threadIdx.x; i < nq; i += stride) {
       const uint4 x = q[i];
       const unsigned long long w = 4 * (unsigned long long)i;
-      h += word_hash(w, x.x) + word_hash(w + 1, x.y) + word_hash(w + 2, x.z) +
-           word_hash(w + 3, x.w);
+      h += entry_hash(w, x);
     }
     for (size_t w = nq * 4 + (size_t)blockIdx.x * 256 + threadIdx.x; w < num_words; w += stride)
       h += word_hash(w, words[w]);
@@ -1436,29 +1488,29 @@ static __global__ __launch_bounds__(256) void k_plan_hash(const uint32_t* __rest
     for (size_t w = (size_t)blockIdx.x * 256 + threadIdx.x; w < num_words; w += stride)
       h += word_hash(w, words[w]);
   }
-  for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
-  if ((threadIdx.x & 63u) == 0) s_part[threadIdx.x >> 6] = h;
-  __syncthreads();
+  h = block_sum(h, s_part);
   // one partial per block (the gate adds them): thousands of blocks adding
   // into one word would queue one device-scope atomic behind the other
-  if (threadIdx.x == 0) part[blockIdx.x] = s_part[0] + s_part[1] + s_part[2] + s_part[3];
+  if (threadIdx.x == 0) part[blockIdx.x] = h;
 }
 
 static __global__ __launch_bounds__(256) void k_plan_gate(unsigned long long* __restrict__ hash,
                                                           uint32_t* __restrict__ counters,
-                                                          uint32_t num_leaf, uint32_t num_part,
-                                                          int cache) {
-  __shared__ unsigned long long s_part[4];
-  unsigned long long h = 0;
-  for (uint32_t b = threadIdx.x; b < num_part; b += 256) h += hash[4 + b];
-  for (int o = 32; o > 0; o >>= 1) h += __shfl_xor(h, o);
-  if ((threadIdx.x & 63u) == 0) s_part[threadIdx.x >> 6] = h;
-  __syncthreads();
+                                                          uint32_t num_leaf, uint32_t row_blocks,
+                                                          uint32_t sum_blocks, int cache) {
+  __shared__ unsigned long long s_part[4], s_sum[4];
+  unsigned long long h = 0, g = 0;
+  if (threadIdx.x < sum_blocks) g = hash[4 + kPlanHashBlocks + threadIdx.x];
+  for (uint32_t b = threadIdx.x; b < row_blocks; b += 256) h += hash[4 + b];
+  h = block_sum(h, s_part);
+  g = block_sum(g, s_sum);
   if (threadIdx.x != 0) return;
-  h = (s_part[0] + s_part[1] + s_part[2] + s_part[3]) ^ mix64(num_leaf);
-  const bool keep = cache && hash[2] == kPlanTag && hash[1] == h && counters[3] == 0u &&
-                    counters[1] <= (uint32_t)kTopSlots && counters[0] <= num_leaf;
+  h ^= mix64(num_leaf);
+  const bool keep = cache && hash[2] == kPlanTag && hash[1] == h && hash[0] == g &&
+                    counters[3] == 0u && counters[1] <= (uint32_t)kTopSlots &&
+                    counters[0] <= num_leaf && counters[0] <= kPlanEntries;
   counters[4] = keep ? 0u : 1u;
+  if (!keep) hash[0] = 0ull;  // k_list_treelets adds the new plan's terms
   counters[2] = 0u;  // the treelet kernel's ticket counter
   hash[1] = h;
   hash[2] = kPlanTag;
@@ -1557,15 +1609,17 @@ template <int T>
 __global__ __launch_bounds__(T) void k_list_treelets(
     uint32_t num_leaf, const uint32_t* __restrict__ bvhnodes, const uint32_t* __restrict__ first,
     const uint32_t* __restrict__ last, uint32_t* __restrict__ counters,
-    uint4* __restrict__ treelets, uint4* __restrict__ top_list, uint32_t* __restrict__ node2slot) {
+    uint4* __restrict__ treelets, uint4* __restrict__ top_list, uint32_t* __restrict__ node2slot,
+    unsigned long long* __restrict__ plan_sum) {
   __shared__ uint32_t s_cnt[2];  // treelets, tops of this round
-  __shared__ unsigned long long s_base;
+  __shared__ unsigned long long s_base, s_sum;
   if (counters[4] == 0u) return;  // the kept plan is valid
   const uint32_t nb = num_leaf - 1;
   const uint32_t K = kTreeletLeaves;
   for (uint32_t base = blockIdx.x * T; base < nb; base += gridDim.x * T) {
     const uint32_t i = base + threadIdx.x;
     uint32_t n_tl = 0, n_top = 0;
+    unsigned long long h = 0;  // this node's terms of the plan's sum
     uint4 tl[2];
     uint4 top = make_uint4(0u, 0u, 0u, 0u);
     if (i < nb) {
@@ -1584,6 +1638,7 @@ __global__ __launch_bounds__(T) void k_list_treelets(
       }
       if (!ok) {
         atomicOr(counters + 3, 1u);
+        h = 1ull;  // no sum of lists equals that of a tree that failed
       } else if (l - f + 1 > K) {
         n_top = 1;
         top = make_uint4(i, a, b, (la - fa + 1 > K ? 1u : 0u) | (lb - fb + 1 > K ? 2u : 0u));
@@ -1593,7 +1648,10 @@ __global__ __launch_bounds__(T) void k_list_treelets(
         tl[n_tl++] = make_uint4(0u, 0u, nb, DMSH_U32MAX);
       }
     }
-    if (threadIdx.x == 0) s_cnt[0] = s_cnt[1] = 0u;
+    if (threadIdx.x == 0) {
+      s_cnt[0] = s_cnt[1] = 0u;
+      s_sum = 0ull;
+    }
     __syncthreads();
     const uint32_t o_tl = n_tl ? atomicAdd(&s_cnt[0], n_tl) : 0u;
     const uint32_t o_top = n_top ? atomicAdd(&s_cnt[1], 1u) : 0u;
@@ -1609,17 +1667,21 @@ __global__ __launch_bounds__(T) void k_list_treelets(
       t.w = (t.w != DMSH_U32MAX && n_top && my_top < (uint32_t)kTopSlots) ? 2u * my_top + t.w
                                                                            : DMSH_U32MAX;
       if (b_tl + o_tl + e < num_leaf) treelets[b_tl + o_tl + e] = t;
+      h += treelet_hash(b_tl + o_tl + e, t);
     }
-    if (n_top && b_top + o_top < (uint32_t)kTopSlots) {
-      top_list[b_top + o_top] = top;
-      node2slot[i] = b_top + o_top;
+    if (n_top && my_top < (uint32_t)kTopSlots) {
+      top_list[my_top] = top;
+      node2slot[i] = my_top;
+      h += top_hash(my_top, top, my_top);
     }
-    __syncthreads();  // s_cnt and s_base are reset next round
+    if (h) atomicAdd(&s_sum, h);
+    __syncthreads();  // s_sum is complete; s_cnt and s_base are reset next round
+    if (threadIdx.x == 0 && s_sum) atomicAdd(plan_sum, s_sum);
   }
 }
 
-// ws: standalone_workspace_bytes(v.num_leaf).  Launches: row hash and plan
-// gate, ranges and list (gated: idle when the workspace keeps this tree's
+// ws: standalone_workspace_bytes(v.num_leaf).  Launches: row and plan hash
+// and gate, ranges and list (gated: idle when the workspace keeps this tree's
 // plan), treelets, top (more than kTreeletLeaves leaves), gated generic climb.
 template <int LK>
 inline int launch_refit_standalone(hipStream_t s, const TreeView& v, float eps, void* ws,
@@ -1639,17 +1701,18 @@ inline int launch_refit_standalone(hipStream_t s, const TreeView& v, float eps, 
   const int cache = (refit_option(kRefitPlanCache) == 1 && !leaves_in_aabb) ? 1 : 0;
   const size_t num_words = (size_t)(2 * (size_t)n - 1) * 3;
   const uint32_t hash_blocks = std::min<uint32_t>(ceil_div(num_words, 1024), kPlanHashBlocks);
-  launch("k_plan_hash", k_plan_hash, dim3(hash_blocks), dim3(256), 0, s, v.bvhnodes, num_words,
-         L.hash + 4);
+  const uint32_t sum_blocks = ceil_div(std::min<uint32_t>(n, kPlanEntries), 256);
+  launch("k_plan_hash", k_plan_hash, dim3(hash_blocks + sum_blocks), dim3(256), 0, s, v.bvhnodes,
+         num_words, hash_blocks, n, L.counters, L.treelets, L.top_list, L.node2slot, L.hash + 4);
   launch("k_plan_gate", k_plan_gate, dim3(1), dim3(256), 0, s, L.hash, L.counters, n, hash_blocks,
-         cache);
+         sum_blocks, cache);
   launch("k_leaf_ranges", k_leaf_ranges<LK>, dim3(ceil_div(n, 256 * kRangeWalks)), dim3(256), 0, s,
          v, eps, leaves_in_aabb ? 1 : 0, L.first, L.last, L.flags, L.counters, err);
   int rc = launch_status();
   if (rc != DMSH_OK) return rc;
   launch("k_list_treelets", k_list_treelets<kListThreads>,
          dim3(std::min<uint32_t>(ceil_div(n - 1, kListThreads), kListGrid)), dim3(kListThreads), 0,
-         s, n, v.bvhnodes, L.first, L.last, L.counters, L.treelets, L.top_list, L.node2slot);
+         s, n, v.bvhnodes, L.first, L.last, L.counters, L.treelets, L.top_list, L.node2slot, L.hash);
   if ((rc = launch_status()) != DMSH_OK) return rc;
   rc = launch_refit_treelets<LK>(s, v, L.flags, L.counters + 0, L.treelets, eps, err,
                                  L.counters + 1, L.top_list, L.node2slot, L.counters + 2,

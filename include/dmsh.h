@@ -136,9 +136,11 @@ int dmsh_bvhnodes_from_sorted_mortons_u64(void *stream, uint32_t n,
  * that layout by the per-leaf climb through arrival counters.  Both give
  * the same boxes.  The workspace (about 32 bytes per leaf) holds the
  * counters, the leaf ranges and the subtree lists -- the tree's plan -- with
- * a hash of the rows they were made from: a later call with the same
- * workspace and unchanged rows keeps the plan and skips its two kernels
- * (tuning key "refit.plan_cache" = 0 rebuilds it every call).  Calls that
+ * a hash of the rows they were made from and one of the lists themselves: a
+ * later call with the same workspace, unchanged rows and a plan that nothing
+ * wrote over (a call for another tree, another use of the memory) keeps the
+ * plan and skips its two kernels (tuning key "refit.plan_cache" = 0 rebuilds
+ * it every call).  What the workspace holds before a call is free.  Calls that
  * share a workspace must run in order (one stream).
  * ------------------------------------------------------------------- */
 size_t dmsh_refit_workspace_bytes(uint32_t num_leaf);
