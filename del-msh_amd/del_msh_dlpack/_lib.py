@@ -334,7 +334,12 @@ _KEPT = {}
 def kept_workspace(entry: str, nbytes: int, device: torch.device, stream: int) -> torch.Tensor:
     """A workspace kept for `entry` on (device, stream) and handed to its later
     calls on that stream (which run in order).  The standalone refits keep the
-    tree's plan in it, checked against a hash of the rows on every call."""
+    tree's plan in it, checked on every call.  A call that is captured into a
+    graph gets one of its own from the graph's pool: the graph holds its
+    address for as long as it lives, and a kept one goes back to the allocator
+    when a larger tree needs a larger one."""
+    if torch.cuda.is_current_stream_capturing():
+        return workspace(nbytes, device)
     key = (entry, torch.device(device).index, int(stream))
     ws = _KEPT.get(key)
     if ws is None or ws.numel() < nbytes:

@@ -112,3 +112,43 @@ def test_a_plan_that_was_written_over_is_made_again(gpu, oracle, part):
         words[a], words[b] = y, x
     assert not kept()
     assert kept() == (part != "failed")
+
+
+def test_a_captured_refit_outlives_the_kept_workspace(gpu, oracle):
+    """A graph holds its workspace's address: later refits of larger trees, which
+    replace the kept workspace, must not take it away from the graph, nor the
+    replays write into what the allocator made of it."""
+    rng = np.random.default_rng(5)
+    tri, vtx = primitives.torus_zup(0.7, 0.3, 40, 30)
+    bn = oracle.build_trimesh3(tri, vtx)[0]
+    t_tri, t_vtx, t_bn = G(tri, gpu), G(vtx, gpu), G(bn, gpu)
+    stream = torch.cuda.Stream(gpu)
+    with torch.cuda.stream(stream):
+        TriMesh3.make_bvhnode2aabb_from_bvhnodes(t_tri, t_vtx, t_bn)
+        torch.cuda.synchronize()
+        key = ("dmsh_bvhnode2aabb_trimesh3", gpu.index or 0, stream.cuda_stream)
+        kept = _lib._KEPT[key]
+        before = kept.clone()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph, stream=stream):
+            aabb = TriMesh3.make_bvhnode2aabb_from_bvhnodes(t_tri, t_vtx, t_bn)
+        assert _lib._KEPT[key] is kept
+        for step, n in enumerate((0, 60, 90, 120)):
+            if n:  # a larger tree: a larger kept workspace, and new tensors where the old one was
+                btri, bvtx = primitives.torus_zup(0.7, 0.3, n, n)
+                bbn = oracle.build_trimesh3(btri, bvtx)[0]
+                got = TriMesh3.make_bvhnode2aabb_from_bvhnodes(G(btri, gpu), G(bvtx, gpu),
+                                                               G(bbn, gpu))
+                assert same_bits(got, oracle.refit_trimesh3(bbn, btri, bvtx, 0.0)), n
+                kept = before = None
+            fill = [torch.full((1 << 18,), 7, dtype=torch.int32, device=gpu) for _ in range(8)]
+            moved = (vtx + rng.normal(size=vtx.shape) * 0.01).astype(np.float32)
+            t_vtx.copy_(G(moved, gpu))
+            aabb.fill_(float("nan"))
+            graph.replay()
+            torch.cuda.synchronize()
+            assert same_bits(aabb, oracle.refit_trimesh3(bn, tri, moved, 0.0)), step
+            assert all(bool((f == 7).all()) for f in fill), step
+            if kept is not None:
+                assert torch.equal(kept, before)  # the replay ran in a workspace of its own
+    assert _lib.device_errors() == 0
