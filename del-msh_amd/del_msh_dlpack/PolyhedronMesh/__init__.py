@@ -25,12 +25,13 @@ def bvhnode2aabb_from_bvhnodes(elem2idx_offset, idx2vtx, vtx2xyz, bvhnodes, bvhn
     num_elem = elem2idx_offset.shape[0] - 1
     L = _lib.lib()
     stream = stream_ptr or _lib.stream_of(dev)
-    ws = _lib.kept_workspace("dmsh_bvhnode2aabb_polyhedron",
-                             L.dmsh_polyhedron_refit_workspace_bytes(num_elem), dev, stream)
-    _lib.check(L.dmsh_bvhnode2aabb_polyhedron(
-        stream, bvhnodes.shape[0], _lib.ptr(bvhnodes), num_elem, _lib.ptr(elem2idx_offset),
-        idx2vtx.shape[0], _lib.ptr(idx2vtx), vtx2xyz.shape[0], _lib.ptr(vtx2xyz),
-        _lib.ptr(bvhnode2aabb), _lib.ptr(ws), ws.numel()), "dmsh_bvhnode2aabb_polyhedron")
+    _lib.check(_lib.call_with_kept_workspace(
+        "dmsh_bvhnode2aabb_polyhedron", L.dmsh_polyhedron_refit_workspace_bytes(num_elem), dev,
+        stream,
+        lambda ws: L.dmsh_bvhnode2aabb_polyhedron(
+            stream, bvhnodes.shape[0], _lib.ptr(bvhnodes), num_elem, _lib.ptr(elem2idx_offset),
+            idx2vtx.shape[0], _lib.ptr(idx2vtx), vtx2xyz.shape[0], _lib.ptr(vtx2xyz),
+            _lib.ptr(bvhnode2aabb), _lib.ptr(ws), ws.numel())), "dmsh_bvhnode2aabb_polyhedron")
 
 
 def search_elem_contain_points(bvhnodes, bvhnode2aabb, elem2idx_offset, idx2vtx, vtx2xyz, wtx2xyz,

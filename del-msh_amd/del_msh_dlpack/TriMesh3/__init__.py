@@ -14,12 +14,13 @@ def make_bvhnode2aabb_from_bvhnodes(tri2vtx, vtx2xyz0, vtx2xyz1, bvhnodes, bvhno
     num_tri = tri2vtx.shape[0]
     num_node = bvhnodes.shape[0]
     stream = stream_ptr or _lib.stream_of(dev)
-    ws = _lib.kept_workspace("dmsh_bvhnode2aabb_trimesh3",
-                             _lib.lib().dmsh_refit_workspace_bytes(num_tri), dev, stream)
+    L = _lib.lib()
     _lib.check(
-        _lib.lib().dmsh_bvhnode2aabb_trimesh3(
-            stream, _lib.ptr(bvhnode2aabb), num_node, _lib.ptr(bvhnodes), num_tri,
-            _lib.ptr(tri2vtx), vtx2xyz0.shape[0], _lib.ptr(vtx2xyz0), 0.0, _lib.ptr(ws),
-            ws.numel()),
+        _lib.call_with_kept_workspace(
+            "dmsh_bvhnode2aabb_trimesh3", L.dmsh_refit_workspace_bytes(num_tri), dev, stream,
+            lambda ws: L.dmsh_bvhnode2aabb_trimesh3(
+                stream, _lib.ptr(bvhnode2aabb), num_node, _lib.ptr(bvhnodes), num_tri,
+                _lib.ptr(tri2vtx), vtx2xyz0.shape[0], _lib.ptr(vtx2xyz0), 0.0, _lib.ptr(ws),
+                ws.numel())),
         "dmsh_bvhnode2aabb_trimesh3",
     )

@@ -10,6 +10,7 @@ from __future__ import annotations
 import ctypes
 import os
 import pathlib
+import threading
 
 import torch
 
@@ -331,18 +332,30 @@ def workspace(nbytes: int, device: torch.device) -> torch.Tensor:
 _KEPT = {}
 
 
-def kept_workspace(entry: str, nbytes: int, device: torch.device, stream: int) -> torch.Tensor:
-    """A workspace kept for `entry` on (device, stream) and handed to its later
-    calls on that stream (which run in order).  The standalone refits keep the
+class _Kept:
+    """The workspace kept for one entry point on one stream, and its lock."""
+
+    __slots__ = ("lock", "ws")
+
+    def __init__(self):
+        self.lock = threading.Lock()
+        self.ws = None
+
+
+def call_with_kept_workspace(entry: str, nbytes: int, device: torch.device, stream: int, call):
+    """call(ws), with a workspace kept for `entry` on (device, stream) and
+    handed to its later calls on that stream (which run in order: a call
+    queues its launches under a lock, so that those of another thread on the
+    same stream do not come between them).  The standalone refits keep the
     tree's plan in it, checked on every call.  A call that is captured into a
     graph gets one of its own from the graph's pool: the graph holds its
     address for as long as it lives, and a kept one goes back to the allocator
     when a larger tree needs a larger one."""
     if torch.cuda.is_current_stream_capturing():
-        return workspace(nbytes, device)
+        return call(workspace(nbytes, device))
     key = (entry, torch.device(device).index, int(stream))
-    ws = _KEPT.get(key)
-    if ws is None or ws.numel() < nbytes:
-        ws = workspace(nbytes, device)
-        _KEPT[key] = ws
-    return ws
+    kept = _KEPT.get(key) or _KEPT.setdefault(key, _Kept())
+    with kept.lock:
+        if kept.ws is None or kept.ws.numel() < nbytes:
+            kept.ws = workspace(nbytes, device)
+        return call(kept.ws)

@@ -1,6 +1,8 @@
 """GPU: the plan that a standalone refit keeps in its workspace is used only while
 it is whole, whatever the memory was used for since it was made."""
 
+import threading
+
 import numpy as np
 import pytest
 import torch
@@ -127,12 +129,12 @@ def test_a_captured_refit_outlives_the_kept_workspace(gpu, oracle):
         TriMesh3.make_bvhnode2aabb_from_bvhnodes(t_tri, t_vtx, t_bn)
         torch.cuda.synchronize()
         key = ("dmsh_bvhnode2aabb_trimesh3", gpu.index or 0, stream.cuda_stream)
-        kept = _lib._KEPT[key]
+        kept = _lib._KEPT[key].ws
         before = kept.clone()
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph, stream=stream):
             aabb = TriMesh3.make_bvhnode2aabb_from_bvhnodes(t_tri, t_vtx, t_bn)
-        assert _lib._KEPT[key] is kept
+        assert _lib._KEPT[key].ws is kept
         for step, n in enumerate((0, 60, 90, 120)):
             if n:  # a larger tree: a larger kept workspace, and new tensors where the old one was
                 btri, bvtx = primitives.torus_zup(0.7, 0.3, n, n)
@@ -151,4 +153,33 @@ def test_a_captured_refit_outlives_the_kept_workspace(gpu, oracle):
             assert all(bool((f == 7).all()) for f in fill), step
             if kept is not None:
                 assert torch.equal(kept, before)  # the replay ran in a workspace of its own
+    assert _lib.device_errors() == 0
+
+
+def test_threads_share_a_stream(gpu, oracle):
+    """Refits of two trees by two threads on one stream share its workspace: the
+    launches of one call must not come between those of the other."""
+    errors = []
+
+    def work(n):
+        try:
+            tri, vtx = primitives.torus_zup(0.7, 0.3, n, n)
+            bn = oracle.build_trimesh3(tri, vtx)[0]
+            want = G(oracle.refit_trimesh3(bn, tri, vtx, 0.0), gpu)
+            t_tri, t_vtx, t_bn = G(tri, gpu), G(vtx, gpu), G(bn, gpu)
+            wrong = torch.zeros((), dtype=torch.int64, device=gpu)
+            for _ in range(300):
+                wrong += (TriMesh3.make_bvhnode2aabb_from_bvhnodes(t_tri, t_vtx, t_bn)
+                          != want).any()
+            if int(wrong):
+                errors.append((n, int(wrong)))
+        except Exception as e:  # pylint: disable=broad-except
+            errors.append((n, e))
+
+    threads = [threading.Thread(target=work, args=(n,)) for n in (40, 90)]
+    for th in threads:
+        th.start()
+    for th in threads:
+        th.join()
+    assert not errors
     assert _lib.device_errors() == 0

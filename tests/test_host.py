@@ -2,6 +2,7 @@
 timing registry."""
 
 import math
+import threading
 
 import numpy as np
 import torch
@@ -188,3 +189,31 @@ def test_cast_workspaces_hold_the_waves_that_a_launch_can_start():
             assert min(tiles * wave, most) <= f(w, h) <= most + slack, (w, h)
         assert f(8, 8) <= 16 * wave + slack
         assert all(f(n, n) <= f(n + 1, n + 1) for n in range(1, 1000, 7))
+
+
+def test_calls_on_a_kept_workspace_take_turns(monkeypatch):
+    """While one thread's call queues its launches, another's on the same stream
+    waits, and one on another stream runs."""
+    monkeypatch.setattr(torch.cuda, "is_current_stream_capturing", lambda: False)
+    monkeypatch.setattr(_lib, "_KEPT", {})
+    cpu = torch.device("cpu")
+    inside, go, order = threading.Event(), threading.Event(), []
+
+    def first(ws):
+        inside.set()
+        go.wait(10)
+        order.append("first")
+
+    a = threading.Thread(target=_lib.call_with_kept_workspace, args=("e", 64, cpu, 1, first))
+    b = threading.Thread(target=_lib.call_with_kept_workspace,
+                         args=("e", 128, cpu, 1, lambda ws: order.append("second")))
+    a.start()
+    assert inside.wait(10)
+    b.start()
+    _lib.call_with_kept_workspace("e", 64, cpu, 2, lambda ws: order.append("other stream"))
+    b.join(0.2)
+    assert order == ["other stream"]
+    go.set()
+    a.join(10)
+    b.join(10)
+    assert order == ["other stream", "first", "second"]
