@@ -40,7 +40,7 @@ def test_trees_of_several_sizes_share_a_workspace(gpu, oracle):
     # the parts of a workspace lie where the size puts them: 5000 leaves write
     # over the lists of 2 leaves and not over their stamp, 70 000 over those of
     # 5000, and so on down and up again
-    clouds = {n: cloud(oracle, n) for n in (2, 3, 1025, 5000, 70_000, 300_000)}
+    clouds = {n: cloud(oracle, n) for n in (2, 3, 1025, 5000, 64_000, 70_000, 300_000)}
     want = {n: oracle.refit_points(bn, pts) for n, (pts, bn) in clouds.items()}
     ws = torch.full((_lib.lib().dmsh_refit_workspace_bytes(300_000),), 0xA5, dtype=torch.uint8,
                     device=gpu)
